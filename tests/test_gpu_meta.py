@@ -154,6 +154,30 @@ def test_route_latest_wins_packed_batch(dev):
         assert list(got[cu[s]:cu[s + 1]]) == exp, s
 
 
+@pytest.mark.parametrize("lens,rate", [
+    ([1023, 1, 1024, 1025], 0.002),
+    ([9217, 40, 20000, 3], 0.0),                # the look-back takes more than one trip and finds nothing
+    ([300, 25000, 7], 1 / 9000),                # ... and finds a token some trips back
+    ([1] * 2500 + [1500], 0.3),                 # more sequences than the staged table holds
+    ([0, 5, 0, 0, 2100, 0], 0.001),             # empty sequences
+])
+def test_route_latest_wins_across_chunks(dev, lens, rate):
+    """Sequences longer than a workgroup's chunk of 1024 tokens, and around its edges; an unsorted control list
+    with a repeated token (the first slot fires)."""
+    rng = np.random.default_rng(sum(lens))
+    atok = [500, 90007, 41, 500, 90001]
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    toks = rng.integers(1000, 40000, size=int(cu[-1]))
+    ctl = rng.random(toks.size) < rate
+    toks[ctl] = rng.choice(atok, size=int(ctl.sum()))
+    start = rng.integers(0, 6, size=len(lens))
+    got = switched.route_latest_wins(torch.tensor(toks, device=dev), atok, 1, torch.tensor(cu, device=dev),
+                                     torch.tensor(start, device=dev)).cpu().numpy()
+    for s in range(len(lens)):
+        if lens[s]:
+            assert list(got[cu[s]:cu[s + 1]]) == omap.latest_wins_ids(list(toks[cu[s]:cu[s + 1]]), atok, False, start[s]), s
+
+
 def test_bitmask_hand_derived(dev, kats):
     k = kats["bitmask"]
     ids = torch.tensor(k["adapter_indices"], device=dev)
