@@ -346,7 +346,7 @@ def test_gemm_shapes(M, N, K, pad):
 @pytest.mark.parametrize("T,nseq,NA,modules,block_m,seed", [
     (1, 1, 1, 1, 32, 0), (700, 40, 6, 4, 32, 1), (5000, 1, 64, 128, 32, 2), (333, 7, 10, 3, 24, 3),
     (1024, 1024, 255, 2, 1, 4), (4144, 304, 24, 128, 64, 5),
-    (20000, 3, 12, 40, 32, 6), (3000, 2500, 255, 17, 8, 7)])
+    (20000, 3, 12, 40, 32, 6), (3000, 2500, 255, 17, 8, 7), (513, 1, 255, 33, 512, 8)])
 def test_token_kernels(T, nseq, NA, modules, block_m, seed):
     rng = np.random.default_rng(seed)
     ids = rng.integers(-2, NA + 3, size=T).astype(np.int64)     # includes out-of-range ids

@@ -178,6 +178,21 @@ def test_route_latest_wins_across_chunks(dev, lens, rate):
             assert list(got[cu[s]:cu[s + 1]]) == omap.latest_wins_ids(list(toks[cu[s]:cu[s + 1]]), atok, False, start[s]), s
 
 
+@pytest.mark.parametrize("M", [1, 511, 512, 513, 1300])
+@pytest.mark.parametrize("block_m,NA,modules", [(8, 40, 33), (32, 64, 161), (128, 256, 3), (512, 7, 1)])
+def test_bitmask_and_remap_table_form(dev, M, block_m, NA, modules):
+    rng = np.random.default_rng(M + block_m)
+    ids = rng.integers(-2, NA + 3, size=M)
+    remap = rng.integers(0, 65, size=(modules, NA + 1))
+    remap[:, 0] = 0
+    out = torch.full((modules, M), -1, dtype=torch.int64, device=dev)
+    for dt in (torch.int64, torch.int32):
+        got = kernels.compute_per_module_bitmasks(torch.tensor(ids, device=dev, dtype=dt),
+                                                  torch.tensor(remap, device=dev).T.contiguous(), block_m, remapped_out=out)
+        assert np.array_equal(got.cpu().numpy(), omap.compute_bitmasks(np.clip(ids, 0, NA), remap.T, block_m))
+        assert np.array_equal(out.cpu().numpy(), remap[:, np.clip(ids, 0, NA)])
+
+
 def test_bitmask_hand_derived(dev, kats):
     k = kats["bitmask"]
     ids = torch.tensor(k["adapter_indices"], device=dev)
