@@ -157,6 +157,28 @@ GS_HD bool gemm_tile(int bid, int tiles_m, int tiles_n, int group, int& tm, int&
   tn = rr / gm;
   return true;
 }
+// As gemm_tile, where the last tile row is thin (at most half its rows exist)
+// and its tiles cost half as much: they come after the others in every XCD's
+// range, shared out evenly, so that the XCDs end together.
+GS_HD int64_t gemm_thin_grid(int tiles_m, int tiles_n, int thin) {
+  const int64_t full = static_cast<int64_t>(tiles_m - thin) * tiles_n, t = thin ? tiles_n : 0;
+  return 8 * ((full + 7) / 8 + (t + 7) / 8);
+}
+GS_HD bool gemm_tile_thin(int bid, int tiles_m, int tiles_n, int thin, int group, int& tm, int& tn, bool& half) {
+  const int full = (tiles_m - thin) * tiles_n;
+  const int per = (full + 7) >> 3;
+  half = (bid >> 3) >= per;
+  if (!half) return gemm_tile(bid, tiles_m - thin, tiles_n, group, tm, tn);
+  tm = tiles_m - 1;
+  tn = (bid & 7) * ((tiles_n + 7) >> 3) + (bid >> 3) - per;
+  return thin && tn < tiles_n;
+}
+// The tile column staged as row r (0 .. 127) of column half h: the 32 rows of
+// wave column r / 32 hold its columns h * 32 .. + 31, so ordered that matrix
+// row i of 16-row block j is column 8 * (i / 4) + 4 j + i % 4.
+GS_HD int gemm_b_row(int r, int h) {
+  return (r >> 5) * 64 + h * 32 + ((r & 15) >> 2) * 8 + ((r >> 4) & 1) * 4 + (r & 3);
+}
 // An operand row a thread moves: rows past the matrix re-read its last.
 GS_HD int gemm_row(int r, int rows) { return imin(r, rows - 1); }
 // The global 16-byte piece a lane moves into LDS position l % 8 of row r.

@@ -5,18 +5,16 @@
 // src/granite_switch/kernels/switch_lora_kernel.py:134-163).
 //
 // Both operands are K-contiguous rows, the layout MFMA reads directly.  A
-// workgroup of 8 waves owns a 256 x 256 tile of C; wave (wm, wn) of the 2 x 4
-// wave grid owns 128 x 64 of it as 4 x 2 blocks of v_mfma_f32_32x32x16_bf16,
-// accumulated in fp32.  K is walked in tiles of 64 through two LDS stages
-// (one barrier per k-tile).  The 256 x 256 tile gives 128 FLOP per byte moved
-// from the L2 into the CU.  Tiles are numbered in groups of 8 tile rows
-// (consecutive workgroups share B columns and A rows in the L2), and each XCD
-// takes a contiguous range of that order, so the tiles running together on
-// one XCD share its L2.  Partial tiles clamp their loads to the last row and
-// mask their stores.
+// workgroup of 8 waves owns a 256 x 256 tile of C, accumulated in fp32, which
+// gives 128 FLOP per byte moved from the L2 into the CU.  Tiles are numbered
+// in groups of 8 tile rows (consecutive workgroups share B columns and A rows
+// in the L2), and each XCD takes a contiguous range of that order, so the
+// tiles running together on one XCD share its L2.  Partial tiles clamp their
+// loads to the last row and mask their stores.
 //
-// Two kernels: for K % 64 == 0 the k-tiles go from global memory straight
-// into LDS (gemm_bf16_tn_dma_kernel); otherwise they are loaded into
+// Two kernels: for K % 64 == 0 (and K >= 128) the k-tiles go from global memory
+// straight into LDS and the two waves of a SIMD alternate between reading and
+// multiplying (gemm_bf16_tn_pingpong_kernel); otherwise they are loaded into
 // registers, zero-filled past K, and written to padded LDS rows
 // (gemm_bf16_tn_kernel).
 #include <stdarg.h>
@@ -50,9 +48,11 @@ struct GemmParams {
   int64_t ldc;
   int M, N, K;
   int tiles_m, tiles_n;
+  int thin;               // the last tile row has at most 128 rows (the ping-pong form runs it at half the work)
 };
 
-// WM x WN waves; wave (wm, wn) owns rows wm*(256/WM) and columns wn*(256/WN)
+// WM x WN waves over k-tiles of 64 in two LDS stages (one barrier per k-tile);
+// wave (wm, wn) owns rows wm*(256/WM) and columns wn*(256/WN)
 // of the tile as MI x NJ blocks of 32 x 32.
 template <bool KTAIL, int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_tn_kernel(GemmParams p) {
@@ -176,126 +176,295 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_tn_kernel(GemmParams p
 }
 
 // ---------------------------------------------------------------------------
-// Direct-to-LDS variant (K % 64 == 0): the same 256 x 256 tile, wave grid and
-// two-stage LDS ring, but the k-tiles travel from global memory straight into
-// LDS with global_load_lds_dwordx4 -- no staging registers and no LDS writes
-// by the waves.  A wave-wide transfer moves 1 KB: 8 rows x 128 bytes, so
-// every request is one whole cache line (transfers of half lines doubled the
-// L2 request count).  Each wave moves 32 rows of each operand per k-tile.  A
-// transfer fills LDS contiguously, so bank spreading comes from an XOR
-// swizzle instead of padding: the 16-byte piece p of row r sits at position
-// p ^ addr::lds_swz(r), which puts the operand reads of 16 consecutive rows at
-// one k (the lanes a 128-bit LDS read serves together) in distinct banks.
-// The next k-tile's transfers are issued before the current tile's MFMAs;
-// the waits are explicit (the transfers are written as assembly, so the
-// compiler does not wait for them before every LDS read).
+// The form for K % 64 == 0, K >= 128: the k-tiles travel from global memory
+// straight into LDS, and the two waves of a SIMD take turns on its matrix core.
+//
+// Tile: 256 x 256, wave (wm, wn) of 2 x 4 owns rows half*128 + wm*64 + 0..63
+// (half = 0, 1) and columns wn*64 + 0..63, as four quadrants of 64 x 32 (row
+// half, column half).  Per k-tile of 64 a wave runs four phases, one quadrant
+// each: 16 v_mfma_f32_16x16x32_bf16, 256 matrix-core clocks.  A phase is a
+// memory part (LDS reads of the operands that the quadrant newly needs, the
+// transfers of one half-operand of k-tile kt+2) and a matrix part, with a
+// barrier after each; waves 4-7 run one part behind waves 0-3, so on every
+// SIMD one wave multiplies while the other reads.
+//
+// LDS: two stages of [A half 0, A half 1, B half 0, B half 1], 128 rows of 128
+// bytes each.  Schedule of k-tile kt (reads | transfers issued):
+//   P1  A0(kt)    | B0(kt+2)      quadrant (0, 0)
+//   P2  B1(kt)    | A0(kt+2)      quadrant (0, 1)
+//   P3  A1(kt)    | B1(kt+2)      quadrant (1, 0)
+//   P4  B0(kt+1)  | A1(kt+2)      quadrant (1, 1)
+// A half is overwritten one phase after its last read, by both wave groups'
+// barriers (a memory part waits for its own reads before its barrier).  A
+// wave has two transfers per phase in flight and waits, at the end of each
+// memory part, until those older than six phases have landed: exactly the half
+// that the next phase reads.  So a transfer has ~3000 clocks to arrive.
+//
+// A last tile row of at most 128 rows runs the two phases of row half 0 only
+// (HALF), at half the time; those tiles come last in every XCD's range.
+//
+// A transfer moves 1 KB: 8 LDS rows x 128 bytes, every request one whole cache
+// line.  It fills LDS contiguously, so bank spreading comes from an XOR
+// swizzle: the 16-byte piece p of row r sits at position p ^ addr::lds_swz(r),
+// which puts the operand reads of 16 consecutive rows at one k in distinct
+// banks.  B rows are staged in the order (addr::gemm_b_row) that gives a lane
+// 8 consecutive columns of its C row, stored as 16 bytes.
+//
+// Measured: 4144 x 27136 x 4096 894 -> 676 us (1363 TFLOP/s), 8192 x 26368 x
+// 4096 1443 TFLOP/s, against the form it replaces (one barrier per k-tile, all
+// waves reading, then all multiplying; 1 transfer stage in flight).
 // ---------------------------------------------------------------------------
-constexpr int kDBK = 64;                        // k per tile
-constexpr int kDRow = kDBK * 2;                 // bytes of one operand row per tile (one cache line)
-constexpr int kDOp = kGBM * kDRow;              // one operand of one stage
+constexpr int kPBK = 64;                        // k per tile
+constexpr int kPRow = kPBK * 2;                 // bytes of one operand row per tile (one cache line)
+constexpr int kPHalf = 128 * kPRow;             // one half-operand of one stage
+constexpr int kPStage = 4 * kPHalf;             // A0, A1, B0, B1
+constexpr int64_t kPMaxLd = int64_t(1) << 22;   // a tile's rows stay within 32-bit byte offsets
 
-template <int WM, int WN>
-__global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_tn_dma_kernel(GemmParams p) {
-  constexpr int NW = WM * WN;
-  constexpr int RPW = kGBM / NW;                // rows of each operand one wave moves per k-tile
-  constexpr int TPO = RPW / 8;                  // its 1 KB transfers per operand
-  static_assert(RPW % 8 == 0 && kGBM == kGBN, "waves move whole 8-row transfers");
-  constexpr int MI = kGBM / WM / 32;
-  constexpr int NJ = kGBN / WN / 32;
-  __shared__ __align__(16) char sA0[kDOp], sB0[kDOp], sA1[kDOp], sB1[kDOp];
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
-  int tm, tn;
-  if (!addr::gemm_tile(static_cast<int>(blockIdx.x), p.tiles_m, p.tiles_n, kGGroup, tm, tn)) return;
+__device__ __forceinline__ f32x4 mfma16_bf16(u32x4 a, u32x4 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c,
+                                                 0, 0, 0);
+}
 
+// Transfer of 16 bytes per lane from base + off (a lane's byte offset) to LDS
+// at dst + 16 * lane; counts in vmcnt (see dma16).
+__device__ __forceinline__ void dma16_at(const char* base, uint32_t off, uint32_t dst) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(dst)
+               : "memory", "m0");
+}
+
+// s_waitcnt for "vmcnt <= n and lgkmcnt == 0"
+constexpr int wait_vm_lds(int n) { return (n & 15) | (7 << 4) | ((n >> 4) << 14); }
+
+template <bool HALF>
+__device__ __forceinline__ void gemm_tile_pingpong(const GemmParams& p, char* smem, int tm, int tn) {
+  constexpr int NA = HALF ? 1 : 2;              // row halves
   const int tid = threadIdx.x;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l = tid & 63;
-  // transfer i of this wave: LDS row RPW*wave + 8*i + l/8, position l % 8,
-  // which holds global piece (l % 8) ^ lds_swz(row) of that row
-  const char* da[TPO];
-  const char* db[TPO];
+  const int wm = wave >> 2;
+  const int wn = wave & 3;
+  const int nk = p.K / kPBK;
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr_t)(smem)));
+
+  // transfers j = 0, 1 of this wave and half-operand: LDS rows 8 * (2 * wave + j) on
+  uint32_t offa[NA][2], offb[2][2];
 #pragma unroll
-  for (int i = 0; i < TPO; ++i) {
-    const int r = RPW * wave + 8 * i + (l >> 3);
-    const int piece = addr::gemm_piece(l, r);
-    da[i] = p.a + static_cast<int64_t>(addr::gemm_row(tm * kGBM + r, p.M)) * p.lda * 2 + piece * 16;
-    db[i] = p.b + static_cast<int64_t>(addr::gemm_row(tn * kGBN + r, p.N)) * p.ldb * 2 + piece * 16;
+  for (int j = 0; j < 2; ++j) {
+    const int r = 8 * (2 * wave + j) + (l >> 3);
+    const uint32_t piece = addr::gemm_piece(l, r) * 16;
+#pragma unroll
+    for (int h = 0; h < NA; ++h)
+      offa[h][j] = static_cast<uint32_t>((addr::gemm_row(tm * kGBM + h * 128 + r, p.M) - tm * kGBM) * p.lda * 2) + piece;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      offb[h][j] = static_cast<uint32_t>((addr::gemm_row(tn * kGBN + addr::gemm_b_row(r, h), p.N) - tn * kGBN) * p.ldb * 2) + piece;
   }
-  auto issue = [&](int kt, char* sa, char* sb) {
-    const int64_t off = static_cast<int64_t>(kt) * kDRow;
-#pragma unroll
-    for (int i = 0; i < TPO; ++i) {
-      dma16(da[i] + off, sa + (RPW * wave + 8 * i) * kDRow);
-      dma16(db[i] + off, sb + (RPW * wave + 8 * i) * kDRow);
-    }
+  const char* const basea = p.a + static_cast<int64_t>(tm) * kGBM * p.lda * 2;
+  const char* const baseb = p.b + static_cast<int64_t>(tn) * kGBN * p.ldb * 2;
+  const uint32_t dst0 = lds0 + wave * 2048;
+  auto issue_a = [&](int h, int kt) {
+    const char* g = basea + static_cast<int64_t>(min(kt, nk - 1)) * kPRow;
+    const uint32_t d = dst0 + (kt & 1) * kPStage + h * kPHalf;
+    dma16_at(g, offa[HALF ? 0 : h][0], d);
+    dma16_at(g, offa[HALF ? 0 : h][1], d + 1024);
+  };
+  auto issue_b = [&](int h, int kt) {
+    const char* g = baseb + static_cast<int64_t>(min(kt, nk - 1)) * kPRow;
+    const uint32_t d = dst0 + (kt & 1) * kPStage + (2 + h) * kPHalf;
+    dma16_at(g, offb[h][0], d);
+    dma16_at(g, offb[h][1], d + 1024);
   };
 
-  const int wm = wave / WN;
-  const int wn = wave % WN;
-  const int i32 = l & 31;
-  const int h = l >> 5;
-  const int sw = addr::lds_swz(i32);            // swizzle of this lane's rows (blocks start at multiples of 32)
-  f32x16 acc[MI][NJ];
+  f32x4 acc[NA][2][4][2];                       // [row half][column half][16-row block][16-column block]
 #pragma unroll
-  for (int i = 0; i < MI; ++i)
+  for (int h = 0; h < NA; ++h)
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) acc[i][j] = f32x16{};
-  auto compute = [&](const char* sa, const char* sb) {
-    const char* pa = sa + (wm * MI * 32 + i32) * kDRow;
-    const char* pb = sb + (wn * NJ * 32 + i32) * kDRow;
+    for (int c = 0; c < 2; ++c)
 #pragma unroll
-    for (int kk = 0; kk < kDBK / 16; ++kk) {
-      const int pos = ((kk * 2 + h) ^ sw) * 16;
-      u32x4 af[MI], bf[NJ];
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int i = 0; i < MI; ++i) af[i] = *reinterpret_cast<const u32x4*>(pa + i * 32 * kDRow + pos);
+        for (int j = 0; j < 2; ++j) acc[h][c][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  // operand reads: lane l reads row l % 16 of a block, k 8 * (l / 16) .. + 7 of each 32
+  const int pos = ((l >> 4) ^ addr::lds_swz(l & 15)) * 16;
+  const char* const ra = smem + (wm * 64 + (l & 15)) * kPRow;
+  const char* const rb = smem + 2 * kPHalf + (wn * 32 + (l & 15)) * kPRow;
+  u32x4 fa[4][2], fb[2][2][2];                  // [16-row block][k step], [column half][16-column block][k step]
+  auto read_a = [&](int h, int st) {
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) bf[j] = *reinterpret_cast<const u32x4*>(pb + j * 32 * kDRow + pos);
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) acc[i][j] = mfma32_bf16(af[i], bf[j], acc[i][j]);
+    for (int i = 0; i < 4; ++i) {
+      fa[i][0] = ld16(ra + st * kPStage + h * kPHalf + i * 16 * kPRow + pos);
+      fa[i][1] = ld16(ra + st * kPStage + h * kPHalf + i * 16 * kPRow + (pos ^ 64));
     }
   };
-  // wait until this wave's transfers landed, then the barrier makes every
-  // wave's part visible (and every wave is done with the other stage)
-  auto sync = [&]() {
-    __builtin_amdgcn_s_waitcnt(wait_vm(0));
+  auto read_b = [&](int h, int st) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      fb[h][j][0] = ld16(rb + st * kPStage + h * kPHalf + j * 16 * kPRow + pos);
+      fb[h][j][1] = ld16(rb + st * kPStage + h * kPHalf + j * 16 * kPRow + (pos ^ 64));
+    }
+  };
+  auto bar = [&]() {
     mem_fence_compiler();
     __builtin_amdgcn_s_barrier();
     mem_fence_compiler();
   };
-  const int nk = p.K / kDBK;
-  // one k-tile: transfers of tile kt+1 into the stage every wave finished
-  // with before the last barrier, the MFMAs of tile kt, then the wait
-  auto step = [&](int kt, const char* ca, const char* cb, char* na, char* nb) {
-    if (kt + 1 < nk) issue(kt + 1, na, nb);
-    compute(ca, cb);
-    sync();
+  // the end of a memory part: own reads done, transfers older than the last n landed
+#define GS_GEMM_MEM_END(n)                          \
+  do {                                              \
+    mem_fence_compiler();                           \
+    __builtin_amdgcn_s_waitcnt(wait_vm_lds(n));     \
+    bar();                                          \
+    __builtin_amdgcn_sched_barrier(0);              \
+  } while (0)
+  auto mma = [&](int h, int c) {
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[HALF ? 0 : h][c][i][j] = mfma16_bf16(fb[c][j][k], fa[i][k], acc[HALF ? 0 : h][c][i][j]);
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+    bar();
   };
-  issue(0, sA0, sB0);
-  sync();
-  for (int kt = 0; kt < nk; kt += 2) {
-    step(kt, sA0, sB0, sA1, sB1);
-    if (kt + 1 < nk) step(kt + 1, sA1, sB1, sA0, sB0);
-  }
 
-  const int row0 = tm * kGBM + wm * MI * 32;
-  const int col0 = tn * kGBN + wn * NJ * 32 + i32;
+  if constexpr (!HALF) {
 #pragma unroll
-  for (int i = 0; i < MI; ++i) {
+    for (int kt = 0; kt < 2; ++kt) {
+      issue_b(0, kt);
+      issue_a(0, kt);
+      issue_b(1, kt);
+      issue_a(1, kt);
+    }
+    GS_GEMM_MEM_END(12);                        // B0(0) and A0(0) landed
+    read_b(0, 0);
+    GS_GEMM_MEM_END(12);                        // every wave holds B0(0)
+    if (wm == 1) bar();                         // waves 4-7 start one part behind
+    int st = 0;
+    for (int kt = 0; kt < nk - 2; ++kt, st ^= 1) {
+      read_a(0, st);
+      issue_b(0, kt + 2);
+      GS_GEMM_MEM_END(12);
+      mma(0, 0);
+      read_b(1, st);
+      issue_a(0, kt + 2);
+      GS_GEMM_MEM_END(12);
+      mma(0, 1);
+      read_a(1, st);
+      issue_b(1, kt + 2);
+      GS_GEMM_MEM_END(12);
+      mma(1, 0);
+      // B0(kt+1) replaces the operand that quadrant (1, 0) was the last to use
+      read_b(0, st ^ 1);
+      issue_a(1, kt + 2);
+      GS_GEMM_MEM_END(12);
+      mma(1, 1);
+    }
+    // the last two k-tiles: nothing left to issue, the waits count down
+    read_a(0, st);
+    GS_GEMM_MEM_END(10);
+    mma(0, 0);
+    read_b(1, st);
+    GS_GEMM_MEM_END(8);
+    mma(0, 1);
+    read_a(1, st);
+    GS_GEMM_MEM_END(6);
+    mma(1, 0);
+    read_b(0, st ^ 1);
+    GS_GEMM_MEM_END(4);
+    mma(1, 1);
+    st ^= 1;
+    read_a(0, st);
+    GS_GEMM_MEM_END(2);
+    mma(0, 0);
+    read_b(1, st);
+    GS_GEMM_MEM_END(0);
+    mma(0, 1);
+    read_a(1, st);
+    GS_GEMM_MEM_END(0);
+    mma(1, 0);
+    mma(1, 1);
+    if (wm == 0) bar();
+  } else {
+    // two phases per k-tile: P1 reads A0(kt), issues B1(kt+1) and B0(kt+2);
+    // P2 reads B1(kt) and B0(kt+1), issues A0(kt+2).  Past the last k-tile
+    // the last one is moved again (into a stage nothing reads any more).
+    issue_b(0, 0);
+    issue_a(0, 0);
+    issue_b(1, 0);
+    issue_b(0, 1);
+    issue_a(0, 1);
+    GS_GEMM_MEM_END(6);                         // B0(0) and A0(0) landed
+    read_b(0, 0);
+    GS_GEMM_MEM_END(6);
+    if (wm == 1) bar();
+    int st = 0;
+    for (int kt = 0; kt < nk; ++kt, st ^= 1) {
+      read_a(0, st);
+      issue_b(1, kt + 1);
+      issue_b(0, kt + 2);
+      GS_GEMM_MEM_END(6);
+      mma(0, 0);
+      read_b(1, st);
+      read_b(0, st ^ 1);
+      issue_a(0, kt + 2);
+      GS_GEMM_MEM_END(6);
+      mma(0, 1);
+    }
+    if (wm == 0) bar();
+    __builtin_amdgcn_s_waitcnt(wait_vm(0));     // no transfer may land after the workgroup's LDS is given back
+  }
+#undef GS_GEMM_MEM_END
+
+  // lane l holds row l % 16 of each 16-row block and columns 8 * (l / 16) .. + 7
+  // of each column half
+  const bool wide = p.ldc % 8 == 0 && (reinterpret_cast<uintptr_t>(p.c) & 15) == 0;
+  const int row0 = tm * kGBM + wm * 64 + (l & 15);
+  const int col0 = tn * kGBN + wn * 64 + (l >> 4) * 8;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const int col = col0 + j * 32;
-      if (col >= p.N) continue;
+  for (int h = 0; h < NA; ++h)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int row = row0 + i * 32 + mfma32_row(v, l);
-        if (row < p.M) p.c[static_cast<int64_t>(row) * p.ldc + col] = f32_to_bf16_bits(acc[i][j][v]);
+    for (int i = 0; i < 4; ++i) {
+      const int row = row0 + h * 128 + i * 16;
+      if (row >= p.M) continue;
+      uint16_t* crow = p.c + static_cast<int64_t>(row) * p.ldc;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int col = col0 + c * 32;
+        const f32x4 lo = acc[h][c][i][0], hi = acc[h][c][i][1];
+        const u32x4 v = {pack_bf16x2(lo[0], lo[1]), pack_bf16x2(lo[2], lo[3]), pack_bf16x2(hi[0], hi[1]),
+                         pack_bf16x2(hi[2], hi[3])};
+        if (wide && col + 8 <= p.N) {
+          st16(crow + col, v);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (col + e < p.N) crow[col + e] = static_cast<uint16_t>(v[e >> 1] >> (16 * (e & 1)));
+        }
       }
     }
-  }
 }
+
+__global__ __launch_bounds__(512) void gemm_bf16_tn_pingpong_kernel(GemmParams p) {
+  __shared__ __align__(16) char smem[2 * kPStage];
+  int tm, tn;
+  bool half;
+  if (!addr::gemm_tile_thin(static_cast<int>(blockIdx.x), p.tiles_m, p.tiles_n, p.thin, kGGroup, tm, tn, half)) return;
+  if (half) gemm_tile_pingpong<true>(p, smem, tm, tn);
+  else gemm_tile_pingpong<false>(p, smem, tm, tn);
+}
+
+// Whole 64-k tiles, at least the two that its stages hold, and rows within
+// 32-bit offsets of a tile's first.
+inline bool pingpong_form(int64_t K, int64_t lda, int64_t ldb) {
+  return K % kPBK == 0 && K >= 2 * kPBK && lda <= kPMaxLd && ldb <= kPMaxLd;
+}
+inline int gemm_thin(int64_t M) { return M % kGBM >= 1 && M % kGBM <= kGBM / 2 ? 1 : 0; }
 
 template <bool KTAIL>
 void launch_gemm(unsigned grid, const GemmParams& p, hipStream_t st) {
@@ -351,27 +520,26 @@ struct GemmModel {
         break;
       }
   }
-  // The stage layout a writer mapping produces: slot (row, position) must be
-  // written exactly once and hold the global piece position ^ lds_swz(row),
-  // which is where the operand reads look for it.
-  struct StageLayout {
-    std::vector<int> piece = std::vector<int>(kGBM * 8, -1);
+  // The layout of one half-operand a writer mapping produces: slot (row,
+  // position) must be written exactly once and hold the global piece position
+  // ^ lds_swz(row), which is where the operand reads look for it.
+  struct HalfLayout {
+    std::vector<int> piece = std::vector<int>(128 * 8, -1);
   };
-  void put(StageLayout& st, int row, int pos, int gpiece) {
+  void put(HalfLayout& st, int row, int pos, int gpiece) {
     ++checked;
-    if (row < 0 || row >= kGBM || pos < 0 || pos >= 8) return fail("stage slot (%d, %d) outside the stage", row, pos);
+    if (row < 0 || row >= 128 || pos < 0 || pos >= 8) return fail("stage slot (%d, %d) outside the half", row, pos);
     int& slot = st.piece[row * 8 + pos];
     if (slot >= 0) return fail("stage slot (%d, %d) written twice", row, pos);
     slot = gpiece;
   }
-  void check_layout(const StageLayout& st, const char* who) {
-    for (int r = 0; r < kGBM; ++r)
+  void check_layout(const HalfLayout& st) {
+    for (int r = 0; r < 128; ++r)
       for (int q = 0; q < 8; ++q) {
         ++checked;
         const int g = st.piece[r * 8 + q];
         if (g != (q ^ addr::lds_swz(r)))
-          return fail("%s: stage slot (%d, %d) holds piece %d, the operand reads expect %d", who, r, q, g,
-                      q ^ addr::lds_swz(r));
+          return fail("stage slot (%d, %d) holds piece %d, the operand reads expect %d", r, q, g, q ^ addr::lds_swz(r));
       }
   }
   void stores(int tm, int tn, int WM, int WN) {
@@ -391,44 +559,93 @@ struct GemmModel {
           }
       }
   }
-  // gemm_bf16_tn_dma_kernel<WM, WN> (K % 64 == 0)
-  void dma(int WM, int WN) {
-    const int NW = WM * WN, RPW = kGBM / NW, TPO = RPW / 8, MI = kGBM / WM / 32, NJ = kGBN / WN / 32;
-    const int nk = static_cast<int>(K / kDBK);
-    StageLayout st;
-    for (int wave = 0; wave < NW; ++wave)
+  // gemm_bf16_tn_pingpong_kernel: every workgroup's transfers, operand reads
+  // and stores, each tile and each element of C once, and each operand read
+  // landing on the rows and columns its result is stored at
+  void pingpong() {
+    const int nk = static_cast<int>(K / kPBK), thin = gemm_thin(M);
+    HalfLayout st;
+    for (int wave = 0; wave < 8; ++wave)
       for (int l = 0; l < 64; ++l)
-        for (int i = 0; i < TPO; ++i) {
+        for (int j = 0; j < 2; ++j) {
           // a transfer fills 8 rows x 128 bytes of LDS in lane order
-          const int64_t lds = (RPW * wave + 8 * i) * kDRow + l * 16;
-          put(st, static_cast<int>(lds / kDRow), static_cast<int>((lds % kDRow) / 16),
-              addr::gemm_piece(l, RPW * wave + 8 * i + (l >> 3)));
+          const int64_t lds = (8 * (2 * wave + j)) * kPRow + l * 16;
+          put(st, static_cast<int>(lds / kPRow), static_cast<int>((lds % kPRow) / 16),
+              addr::gemm_piece(l, 8 * (2 * wave + j) + (l >> 3)));
         }
-    check_layout(st, "dma");
-    tiles([&](int tm, int tn) {
-      for (int wave = 0; wave < NW; ++wave) {
-        for (int l = 0; l < 64; ++l)
-          for (int i = 0; i < TPO; ++i) {
-            const int r = RPW * wave + 8 * i + (l >> 3);
+    check_layout(st);
+    for (int wave = 0; wave < 8; ++wave)        // operand reads
+      for (int l = 0; l < 64; ++l) {
+        const int wm = wave >> 2, wn = wave & 3, pos = ((l >> 4) ^ addr::lds_swz(l & 15)) * 16;
+        for (int stage = 0; stage < 2; ++stage)
+          for (int h = 0; h < 2; ++h)
+            for (int k = 0; k < 2; ++k) {
+              for (int i = 0; i < 4; ++i) {
+                const int64_t in_half = (wm * 64 + (l & 15) + i * 16) * kPRow + (pos ^ (64 * k));
+                in("A operand (LDS)", in_half, 16, kPHalf);
+                in("A operand (LDS)", stage * kPStage + h * kPHalf + in_half, 16, 2 * kPStage);
+              }
+              for (int j = 0; j < 2; ++j) {
+                const int r = wn * 32 + (l & 15) + j * 16;
+                const int64_t in_half = r * kPRow + (pos ^ (64 * k));
+                in("B operand (LDS)", in_half, 16, kPHalf);
+                in("B operand (LDS)", stage * kPStage + (2 + h) * kPHalf + in_half, 16, 2 * kPStage);
+                // matrix row l % 16 of block j is column 8 * (row / 4) + 4 j + row % 4 of the wave's column half
+                if (addr::gemm_b_row(r, h) != wn * 64 + h * 32 + 8 * ((l & 15) >> 2) + 4 * j + (l & 3))
+                  fail("B row %d of half %d is staged as tile column %d", r, h, addr::gemm_b_row(r, h));
+              }
+            }
+      }
+    const int64_t total = int64_t(tiles_m) * tiles_n, grid = addr::gemm_thin_grid(tiles_m, tiles_n, thin);
+    std::vector<char> seen(total, 0);
+    for (int64_t b = 0; b < grid; ++b) {
+      int tm, tn;
+      bool half;
+      if (!addr::gemm_tile_thin(static_cast<int>(b), tiles_m, tiles_n, thin, kGGroup, tm, tn, half)) continue;
+      if (!in("tile row", tm, 1, tiles_m) || !in("tile column", tn, 1, tiles_n)) continue;
+      if (seen[int64_t(tm) * tiles_n + tn]++) fail("tile (%d, %d) taken twice", tm, tn);
+      if (half && M - int64_t(tm) * kGBM > kGBM / 2) fail("tile row %d has rows past the first half", tm);
+      std::vector<char> cseen(kGBM * kGBN, 0);
+      for (int wave = 0; wave < 8; ++wave)
+        for (int l = 0; l < 64; ++l) {
+          for (int j = 0; j < 2; ++j) {
+            const int r = 8 * (2 * wave + j) + (l >> 3);
             const int piece = addr::gemm_piece(l, r);
-            const int64_t ra = addr::gemm_row(tm * kGBM + r, static_cast<int>(M));
-            const int64_t rb = addr::gemm_row(tn * kGBN + r, static_cast<int>(N));
-            in("stage row (LDS)", (RPW * wave + 8 * i) * kDRow + l * 16, 16, kDOp);
-            for (int kt = 0; kt < nk; ++kt) {
-              in("A", ra * lda + int64_t(kt) * kDBK + piece * 8, 8, a_elems());
-              in("B", rb * ldb + int64_t(kt) * kDBK + piece * 8, 8, b_elems());
+            for (int h = 0; h < 2; ++h) {
+              const int64_t ra = addr::gemm_row(tm * kGBM + h * 128 + r, static_cast<int>(M));
+              const int64_t rb = addr::gemm_row(tn * kGBN + addr::gemm_b_row(r, h), static_cast<int>(N));
+              in("A offset in 32 bits", (ra - int64_t(tm) * kGBM) * lda * 2 + piece * 16, 16, int64_t(1) << 32);
+              in("B offset in 32 bits", (rb - int64_t(tn) * kGBN) * ldb * 2 + piece * 16, 16, int64_t(1) << 32);
+              for (int kt = 0; kt < nk; ++kt) {
+                if (h == 0 || !half) in("A", ra * lda + int64_t(kt) * kPBK + piece * 8, 8, a_elems());
+                in("B", rb * ldb + int64_t(kt) * kPBK + piece * 8, 8, b_elems());
+              }
             }
           }
-        const int wm = wave / WN, wn = wave % WN;
-        for (int l = 0; l < 64; ++l)
-          for (int kk = 0; kk < kDBK / 16; ++kk) {
-            const int pos = ((kk * 2 + (l >> 5)) ^ addr::lds_swz(l & 31)) * 16;
-            for (int i = 0; i < MI; ++i) in("A operand (LDS)", (wm * MI * 32 + (l & 31) + i * 32) * kDRow + pos, 16, kDOp);
-            for (int j = 0; j < NJ; ++j) in("B operand (LDS)", (wn * NJ * 32 + (l & 31) + j * 32) * kDRow + pos, 16, kDOp);
+          const int wm = wave >> 2, wn = wave & 3;
+          for (int h = 0; h < (half ? 1 : 2); ++h)
+            for (int i = 0; i < 4; ++i)
+              for (int c = 0; c < 2; ++c)
+                for (int e = 0; e < 8; ++e) {
+                  const int row = wm * 64 + (l & 15) + h * 128 + i * 16, col = wn * 64 + (l >> 4) * 8 + c * 32 + e;
+                  if (tm * kGBM + row >= M || tn * kGBN + col >= N) continue;
+                  in("C", int64_t(tm * kGBM + row) * ldc + tn * kGBN + col, 1, (M - 1) * ldc + N);
+                  if (cseen[row * kGBN + col]++) fail("C element (%d, %d) of a tile stored twice", row, col);
+                }
+        }
+      for (int r = 0; r < kGBM; ++r)
+        for (int c = 0; c < kGBN; ++c)
+          if (tm * kGBM + r < M && tn * kGBN + c < N && !cseen[r * kGBN + c]) {
+            fail("C element (%d, %d) of tile (%d, %d) is never stored", r, c, tm, tn);
+            r = kGBM;
+            break;
           }
+    }
+    for (int64_t t = 0; t < total; ++t)
+      if (!seen[t]) {
+        fail("tile %lld of %lld is never taken", (long long)t, (long long)total);
+        break;
       }
-      stores(tm, tn, WM, WN);
-    });
   }
   // gemm_bf16_tn_kernel<KTAIL, WM, WN>
   void reg(bool KTAIL, int WM, int WN) {
@@ -505,12 +722,11 @@ int gs_gemm_bf16_tn(const void* a, int64_t lda, const void* b, int64_t ldb, void
   GS_CHECK_ARG(total <= (int64_t(1) << 30), "%s: too many tiles", who);
   const unsigned grid = static_cast<unsigned>(8 * ((total + 7) / 8));
   hipStream_t st = static_cast<hipStream_t>(stream);
-#ifndef GS_GEMM_NO_DMA
-  if (K % kDBK == 0) {
-    hipLaunchKernelGGL((gemm_bf16_tn_dma_kernel<2, 4>), dim3(grid), dim3(512), 0, st, p);
-  } else
-#endif
-  if (K % kGBK == 0) launch_gemm<false>(grid, p, st);
+  if (pingpong_form(K, lda, ldb)) {
+    p.thin = gemm_thin(M);
+    const unsigned n = static_cast<unsigned>(addr::gemm_thin_grid(p.tiles_m, p.tiles_n, p.thin));
+    hipLaunchKernelGGL(gemm_bf16_tn_pingpong_kernel, dim3(n), dim3(512), 0, st, p);
+  } else if (K % kGBK == 0) launch_gemm<false>(grid, p, st);
   else launch_gemm<true>(grid, p, st);
   GS_CHECK_LAUNCH(who);
   return GS_OK;
@@ -529,12 +745,8 @@ int64_t gs_check_gemm_addresses(int64_t M, int64_t N, int64_t K, int64_t lda, in
   m.ldc = ldc;
   m.tiles_m = static_cast<int>((M + kGBM - 1) / kGBM);
   m.tiles_n = static_cast<int>((N + kGBN - 1) / kGBN);
-  if (K % kDBK == 0) {
-    m.dma(2, 4);
-    m.reg(false, 2, 4);      // the register-staged form of the same shape
-  } else {
-    m.reg(true, 2, 4);
-  }
+  if (pingpong_form(K, lda, ldb)) m.pingpong();
+  m.reg(K % kGBK != 0, 2, 4);      // the register-staged form takes any shape
   if (checked) *checked = m.checked;
   if (msg && msg_len > 0) snprintf(msg, static_cast<size_t>(msg_len), "%s", m.msg);
   return m.bad;

@@ -331,6 +331,8 @@ def test_builder_random_batches(T, NA, seed):
     (4144, 4864, 1024, 8),         # step down-projection shape at a shorter K, padded strides
     (257, 257, 512, 64),
     (1100, 3000, 8, 0),
+    (128, 264, 192, 0),            # a thin tile row alone
+    (2049, 775, 128, 8),           # tile rows of 8, then one of one row
 ])
 def test_gemm_shapes(M, N, K, pad):
     msg = ctypes.create_string_buffer(512)

@@ -45,6 +45,18 @@ def test_gemm_matches_fp32_reference(dev, M, N, K, seed):
     _check(got, x, w)
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (256, 256, 128),            # the two k-tiles that the direct-to-LDS form's stages hold, nothing left to issue
+    (128, 264, 192),            # a thin last tile row alone; an odd number of k-tiles
+    (385, 520, 256),            # a thin tile row of one row more than half a tile is not thin: 256 + 129
+    (384, 1032, 320),           # full tiles, then thin ones, over two tile columns and a partial one
+    (2049, 775, 128),           # one row in the thin row; columns that end inside an 8-column store
+    (300, 301, 256),            # rows of C that are not 16-byte aligned
+])
+def test_gemm_pingpong_tile_edges(dev, M, N, K):
+    test_gemm_matches_fp32_reference(dev, M, N, K, M + N)
+
+
 def test_gemm_strided_rows_and_output(dev):
     """x and out with row strides (a view into a wider buffer), as the layer's x_ext slices are."""
     g = torch.Generator(device=dev).manual_seed(11)
