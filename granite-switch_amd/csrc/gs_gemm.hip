@@ -20,6 +20,8 @@
 #include <stdarg.h>
 
 #include <algorithm>
+#include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "gs_addr.h"
@@ -48,6 +50,7 @@ struct GemmParams {
   int64_t ldc;
   int M, N, K;
   int tiles_m, tiles_n;
+  int tile_rows;          // 256, or 128: every tile is one row half (ping-pong form)
   int thin;               // the last tile row has at most 128 rows (the ping-pong form runs it at half the work)
 };
 
@@ -201,7 +204,13 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_tn_kernel(GemmParams p
 // that the next phase reads.  So a transfer has ~3000 clocks to arrive.
 //
 // A last tile row of at most 128 rows runs the two phases of row half 0 only
-// (HALF), at half the time; those tiles come last in every XCD's range.
+// (HALF), at two thirds of the time; those tiles come last in every XCD's
+// range.  Calls whose 256-row tiles would leave most CUs idle cut every tile
+// to that form (pick_gemm).
+//
+// Bound by LDS (64 KB of transfers in at 64 bytes per clock, 192 KB of operand
+// reads at 128: 2560 clocks per k-tile against 2048 of MFMAs; 1.1 us measured)
+// and, with every CU busy, by the clock that the power limit leaves.
 //
 // A transfer moves 1 KB: 8 LDS rows x 128 bytes, every request one whole cache
 // line.  It fills LDS contiguously, so bank spreading comes from an XOR
@@ -238,7 +247,7 @@ __device__ __forceinline__ void dma16_at(const char* base, uint32_t off, uint32_
 constexpr int wait_vm_lds(int n) { return (n & 15) | (7 << 4) | ((n >> 4) << 14); }
 
 template <bool HALF>
-__device__ __forceinline__ void gemm_tile_pingpong(const GemmParams& p, char* smem, int tm, int tn) {
+__device__ __forceinline__ void gemm_tile_pingpong(const GemmParams& p, char* smem, int first_row, int tn) {
   constexpr int NA = HALF ? 1 : 2;              // row halves
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -256,12 +265,12 @@ __device__ __forceinline__ void gemm_tile_pingpong(const GemmParams& p, char* sm
     const uint32_t piece = addr::gemm_piece(l, r) * 16;
 #pragma unroll
     for (int h = 0; h < NA; ++h)
-      offa[h][j] = static_cast<uint32_t>((addr::gemm_row(tm * kGBM + h * 128 + r, p.M) - tm * kGBM) * p.lda * 2) + piece;
+      offa[h][j] = static_cast<uint32_t>((addr::gemm_row(first_row + h * 128 + r, p.M) - first_row) * p.lda * 2) + piece;
 #pragma unroll
     for (int h = 0; h < 2; ++h)
       offb[h][j] = static_cast<uint32_t>((addr::gemm_row(tn * kGBN + addr::gemm_b_row(r, h), p.N) - tn * kGBN) * p.ldb * 2) + piece;
   }
-  const char* const basea = p.a + static_cast<int64_t>(tm) * kGBM * p.lda * 2;
+  const char* const basea = p.a + static_cast<int64_t>(first_row) * p.lda * 2;
   const char* const baseb = p.b + static_cast<int64_t>(tn) * kGBN * p.ldb * 2;
   const uint32_t dst0 = lds0 + wave * 2048;
   auto issue_a = [&](int h, int kt) {
@@ -424,7 +433,7 @@ __device__ __forceinline__ void gemm_tile_pingpong(const GemmParams& p, char* sm
   // lane l holds row l % 16 of each 16-row block and columns 8 * (l / 16) .. + 7
   // of each column half
   const bool wide = p.ldc % 8 == 0 && (reinterpret_cast<uintptr_t>(p.c) & 15) == 0;
-  const int row0 = tm * kGBM + wm * 64 + (l & 15);
+  const int row0 = first_row + wm * 64 + (l & 15);
   const int col0 = tn * kGBN + wn * 64 + (l >> 4) * 8;
 #pragma unroll
   for (int h = 0; h < NA; ++h)
@@ -455,16 +464,271 @@ __global__ __launch_bounds__(512) void gemm_bf16_tn_pingpong_kernel(GemmParams p
   int tm, tn;
   bool half;
   if (!addr::gemm_tile_thin(static_cast<int>(blockIdx.x), p.tiles_m, p.tiles_n, p.thin, kGGroup, tm, tn, half)) return;
-  if (half) gemm_tile_pingpong<true>(p, smem, tm, tn);
-  else gemm_tile_pingpong<false>(p, smem, tm, tn);
+  half |= p.tile_rows == kGBM / 2;
+  if (half) gemm_tile_pingpong<true>(p, smem, tm * p.tile_rows, tn);
+  else gemm_tile_pingpong<false>(p, smem, tm * p.tile_rows, tn);
 }
 
+// ---------------------------------------------------------------------------
+// Streaming form (K % 64 == 0), for calls whose 256 x 256 tiles would leave
+// most CUs idle: tiles of 16*MB x 16*NB, and the W waves of a workgroup split
+// K, each computing the whole tile over its own chunks of 64 k (chunk c
+// belongs to wave c % W).  Every byte that a tile needs is then used by one
+// wave only, so each wave stages its chunks for itself, with no barrier in
+// the loop.
+//
+// A chunk is MB + NB slots of 2 KB (16 rows x 128 bytes, whole cache lines; a
+// load straight into MFMA registers takes 16 rows x 16 bytes per 16 lanes and
+// ran at a quarter of the rate): the B blocks, then the A blocks.  A wave's
+// LDS ring holds RS slots.  Slots are read LA ahead of their MFMAs (one wave
+// per SIMD has nothing else to hide an LDS trip behind), and a slot is
+// refilled as soon as its reads have returned.  Waits count transfers (vmcnt);
+// the last TC chunks, where refills run out, count down with them.  The W
+// partial tiles are summed through LDS at the end, in wave order.
+//
+// Tiles are numbered down the rows first, in one contiguous range per XCD: the
+// row tiles that share weights run together on one XCD, which reads them from
+// HBM once.
+//
+// Bound by LDS (each byte written once and read once) and, for few rows, by
+// HBM: 256 x 7296 x 4096 76 -> 28.9 us and 256 x 4480 x 12800 245 -> 78 against
+// the 256 x 256 tiles; 16 x 7296 x 4096 47 -> 13.2 us (4.6 TB/s of weights),
+// 7 x 4480 x 4096 47 -> 8.9 us (4.1 TB/s).  Deeper rings and longer lookaheads
+// measured the same.
+// ---------------------------------------------------------------------------
+// s_waitcnt for "lgkmcnt <= n"
+constexpr int wait_lds(int n) { return 15 | (7 << 4) | (n << 8) | (3 << 14); }
+
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+// f(integral_constant 0) .. f(integral_constant N - 1): steps whose waits are immediates
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+template <int MB, int NB, int W, int RS, int LA>
+struct StreamShape {
+  static constexpr int NS = MB + NB;            // slots per chunk
+  static constexpr int TC = (RS + NS - 1) / NS; // chunks at the end whose refills run out
+  static constexpr int kSlot = 16 * kPRow;
+  static constexpr int kRing = RS * kSlot;      // bytes per wave
+  static constexpr int NP = NB >= 2 ? NB / 2 : 1;   // column units of a row block: 2 (or 1) 16-column blocks
+  static constexpr int UB = NB >= 2 ? 2 : 1;        // blocks per unit
+  static constexpr int U = MB * NP;
+  static constexpr int kSum = W * U * UB * 1024;    // the partial tiles
+  static constexpr int kLds = W * kRing > kSum ? W * kRing : kSum;
+  static_assert(NB == 1 || NB % 2 == 0, "column blocks pair up");
+  static_assert(RS >= NS && LA >= 1 && LA < NS && kLds <= 160 * 1024, "the ring holds a chunk, LDS holds the rings");
+};
+
+template <int MB, int NB, int W, int RS, int LA>
+__global__ __launch_bounds__(64 * W) void gemm_bf16_tn_stream_kernel(GemmParams p) {
+  using S = StreamShape<MB, NB, W, RS, LA>;
+  constexpr int NS = S::NS, NP = S::NP, UB = S::UB, U = S::U, TC = S::TC;
+  __shared__ __align__(16) char smem[S::kLds];
+  int tm, tn;
+  if (!addr::gemm_tile(static_cast<int>(blockIdx.x), p.tiles_m, p.tiles_n, p.tiles_m, tm, tn)) return;
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l = tid & 63;
+  const int i16 = l & 15;
+  const int q = l >> 4;
+
+  // slot s of a chunk: 16-column block s of B (s < NB), else 16-row block s - NB of A
+  uint32_t off[NS][2];
+#pragma unroll
+  for (int s = 0; s < NS; ++s)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int r = 8 * t + (l >> 3);
+      const uint32_t piece = addr::gemm_piece(l, r) * 16;
+      off[s][t] = piece + static_cast<uint32_t>(
+          s < NB ? (addr::gemm_row(tn * 16 * NB + addr::gemm_s_brow(r, s, NB), p.N) - tn * 16 * NB) * p.ldb * 2
+                 : (addr::gemm_row(tm * 16 * MB + 16 * (s - NB) + r, p.M) - tm * 16 * MB) * p.lda * 2);
+    }
+  const char* const basea = p.a + static_cast<int64_t>(tm) * 16 * MB * p.lda * 2;
+  const char* const baseb = p.b + static_cast<int64_t>(tn) * 16 * NB * p.ldb * 2;
+  const uint32_t ring0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr_t)(smem))) + wave * S::kRing;
+  const int mine = addr::gemm_s_chunks(p.K / kPBK, wave, W);   // this wave's chunks
+  // slot s of chunk i into the ring at byte `at`
+  auto issue = [&](int i, int s, uint32_t at) {
+    const char* g = (s < NB ? baseb : basea) + static_cast<int64_t>(wave + W * i) * kPRow;
+    dma16_at(g, off[s][0], ring0 + at);
+    dma16_at(g, off[s][1], ring0 + at + 1024);
+  };
+  const char* const rd = smem + wave * S::kRing + i16 * kPRow;
+  const int pos = (q ^ addr::lds_swz(i16)) * 16;
+
+  f32x4 acc[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  u32x4 fb[NB][2], fa[LA + 1][2];
+  auto mma = [&](int i, const u32x4 (&a)[2]) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) acc[i][j] = mfma16_bf16(fb[j][k], a[k], acc[i][j]);
+  };
+  // One chunk, whose slot 0 is at ring byte p0.  Step s reads slot s (once all
+  // but the `kYoung` slots issued after it have landed) and completes slot
+  // s - LA: its reads are back, its place is refilled, its MFMAs are issued.
+  // kTail: -1 while every refill exists, else the chunk's place in the last TC.
+  auto chunk = [&](int i, uint32_t p0, auto tail_tag) {
+    constexpr int kTail = decltype(tail_tag)::value;
+    auto at = [&](int s) {
+      const uint32_t x = p0 + s * S::kSlot;
+      return x >= S::kRing ? x - S::kRing : x;
+    };
+    static_for<NS + LA>([&](auto step) {
+      constexpr int s = decltype(step)::value;
+      if constexpr (s < NS) {
+        constexpr int kDone = s > LA ? s - LA : 0;             // slots of this chunk refilled so far
+        constexpr int kIssued = kTail < 0 ? RS + kDone
+                                          : (RS + kTail * NS + kDone < TC * NS ? RS + kTail * NS + kDone : TC * NS) - kTail * NS;
+        constexpr int kYoung = 2 * (kIssued - 1 - s);
+        mem_fence_compiler();
+        __builtin_amdgcn_s_waitcnt(wait_vm(kYoung < 63 ? kYoung : 63));
+        mem_fence_compiler();
+        const char* r = rd + at(s);
+        if constexpr (s < NB) {
+          fb[s][0] = ld16(r + pos);
+          fb[s][1] = ld16(r + (pos ^ 64));
+        } else {
+          fa[s % (LA + 1)][0] = ld16(r + pos);
+          fa[s % (LA + 1)][1] = ld16(r + (pos ^ 64));
+        }
+      }
+      if constexpr (s >= LA) {
+        constexpr int d = s - LA;                              // the slot completed
+        mem_fence_compiler();
+        __builtin_amdgcn_s_waitcnt(wait_lds(2 * (s < NS ? LA : NS - 1 - d)));
+        mem_fence_compiler();
+        if constexpr (kTail < 0 || kTail * NS + d + RS < TC * NS) issue(i + (d + RS) / NS, (d + RS) % NS, at(d));
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (d >= NB) mma(d - NB, fa[d % (LA + 1)]);
+      }
+    });
+  };
+  uint32_t p0 = 0;
+  auto next = [&]() { p0 = p0 + NS * S::kSlot >= S::kRing ? p0 + NS * S::kSlot - S::kRing : p0 + NS * S::kSlot; };
+  static_for<RS>([&](auto g) {
+    constexpr int s = decltype(g)::value;
+    issue(s / NS, s % NS, s * S::kSlot);
+  });
+  int i = 0;
+  for (; i < mine - TC; ++i) {
+    chunk(i, p0, std::integral_constant<int, -1>{});
+    next();
+  }
+  static_for<TC>([&](auto t) {
+    chunk(i + decltype(t)::value, p0, t);
+    next();
+  });
+  lds_barrier();                                // every wave is done with its ring
+
+  // sum the waves' partial tiles: unit u (row block u / NP, column unit u % NP)
+  // is summed and stored by wave u % W
+  f32x4* part = reinterpret_cast<f32x4*>(smem);
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) part[((wave * U + i * NP + j / UB) * UB + j % UB) * 64 + l] = acc[i][j];
+  lds_barrier();
+  const bool wide = p.ldc % 8 == 0 && (reinterpret_cast<uintptr_t>(p.c) & 15) == 0;
+  for (int u = wave; u < U; u += W) {
+    f32x4 v[UB];
+#pragma unroll
+    for (int e = 0; e < UB; ++e) v[e] = part[(u * UB + e) * 64 + l];
+#pragma unroll
+    for (int w = 1; w < W; ++w)
+#pragma unroll
+      for (int e = 0; e < UB; ++e) v[e] += part[((w * U + u) * UB + e) * 64 + l];
+    const int row = tm * 16 * MB + (u / NP) * 16 + i16;
+    const int col = tn * 16 * NB + (u % NP) * 32 + q * 4 * UB;
+    if (row >= p.M) continue;
+    uint16_t* crow = p.c + static_cast<int64_t>(row) * p.ldc;
+    uint32_t o[2 * UB];
+#pragma unroll
+    for (int e = 0; e < UB; ++e) {
+      o[2 * e] = pack_bf16x2(v[e][0], v[e][1]);
+      o[2 * e + 1] = pack_bf16x2(v[e][2], v[e][3]);
+    }
+    if (UB == 2 && wide && col + 8 <= p.N) {
+      st16(crow + col, u32x4{o[0], o[1], o[2 * UB - 2], o[2 * UB - 1]});
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4 * UB; ++e)
+        if (col + e < p.N) crow[col + e] = static_cast<uint16_t>(o[e >> 1] >> (16 * (e & 1)));
+    }
+  }
+}
+
+// ---- which form a call takes ---------------------------------------------------
 // Whole 64-k tiles, at least the two that its stages hold, and rows within
 // 32-bit offsets of a tile's first.
 inline bool pingpong_form(int64_t K, int64_t lda, int64_t ldb) {
   return K % kPBK == 0 && K >= 2 * kPBK && lda <= kPMaxLd && ldb <= kPMaxLd;
 }
 inline int gemm_thin(int64_t M) { return M % kGBM >= 1 && M % kGBM <= kGBM / 2 ? 1 : 0; }
+
+struct StreamForm {
+  int MB, NB, W, RS, LA;
+  void (*kernel)(GemmParams);
+};
+template <int MB, int NB, int W, int RS, int LA>
+constexpr StreamForm stream_form() {
+  return {MB, NB, W, RS, LA, gemm_bf16_tn_stream_kernel<MB, NB, W, RS, LA>};
+}
+const StreamForm kStreamForms[] = {
+    stream_form<1, 2, 4, 10, 2>(), stream_form<2, 2, 4, 10, 2>(), stream_form<4, 2, 4, 10, 2>(),
+    stream_form<4, 4, 4, 10, 3>(), stream_form<8, 4, 4, 16, 3>(),
+};
+
+// The form with the fewest clocks per 64 k on the busiest of 256 CUs: tiles
+// per CU times a tile's measured clocks, which follow its LDS time (transfers
+// in at 64 bytes per clock plus operand reads at 128).  A streaming form takes
+// 60 per 2 KB slot (48 of LDS), the 256 x 256 tile 2400, its 128-row form
+// 1700.  The HBM time of the operands is the same for all of them.  Every wave
+// of a streaming form needs TC chunks.
+// Measured, M x 7296 x 4096, us, every form (16*MB x 16*NB) that was close:
+//   M     16 x 32  32 x 32  64 x 32  64 x 64  128 x 64  128 x 256  256 x 256
+//   16      13.2                                                     47
+//   32      17.1     14.7                                            48
+//   64               21.0     18.2     22.9                49        50
+//   128                       26.2     21.4      28.4                55
+//   256                                34.8      28.9                76
+//   512                                59.2      50.8                75
+//   777                                83.3      83.2      55        75
+struct GemmPick {
+  const StreamForm* stream;   // nullptr: the ping-pong form
+  int tile_rows;
+};
+inline GemmPick pick_gemm(int64_t M, int64_t N, int64_t K) {
+  constexpr int64_t kCus = 256;
+  auto tiles = [&](int64_t tm, int64_t tn) { return ((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
+  auto rounds = [&](int64_t n) { return (n + kCus - 1) / kCus; };
+  GemmPick best{nullptr, kGBM};
+  int64_t cost = 2400 * rounds(tiles(kGBM, kGBN));
+  const int64_t half = 1700 * rounds(tiles(kGBM / 2, kGBN));
+  if (half < cost) {
+    cost = half;
+    best.tile_rows = kGBM / 2;
+  }
+  for (const StreamForm& f : kStreamForms) {
+    const int64_t tc = (f.RS + f.MB + f.NB - 1) / (f.MB + f.NB);
+    const int64_t c = 60 * (f.MB + f.NB) * rounds(tiles(16 * f.MB, 16 * f.NB));
+    if (K / kPBK / f.W >= tc && c < cost) {
+      cost = c;
+      best.stream = &f;
+    }
+  }
+  return best;
+}
 
 template <bool KTAIL>
 void launch_gemm(unsigned grid, const GemmParams& p, hipStream_t st) {
@@ -562,8 +826,9 @@ struct GemmModel {
   // gemm_bf16_tn_pingpong_kernel: every workgroup's transfers, operand reads
   // and stores, each tile and each element of C once, and each operand read
   // landing on the rows and columns its result is stored at
-  void pingpong() {
-    const int nk = static_cast<int>(K / kPBK), thin = gemm_thin(M);
+  void pingpong(int tile_rows) {
+    const int nk = static_cast<int>(K / kPBK), thin = tile_rows == kGBM ? gemm_thin(M) : 0;
+    tiles_m = static_cast<int>((M + tile_rows - 1) / tile_rows);
     HalfLayout st;
     for (int wave = 0; wave < 8; ++wave)
       for (int l = 0; l < 64; ++l)
@@ -604,7 +869,9 @@ struct GemmModel {
       if (!addr::gemm_tile_thin(static_cast<int>(b), tiles_m, tiles_n, thin, kGGroup, tm, tn, half)) continue;
       if (!in("tile row", tm, 1, tiles_m) || !in("tile column", tn, 1, tiles_n)) continue;
       if (seen[int64_t(tm) * tiles_n + tn]++) fail("tile (%d, %d) taken twice", tm, tn);
-      if (half && M - int64_t(tm) * kGBM > kGBM / 2) fail("tile row %d has rows past the first half", tm);
+      half |= tile_rows == kGBM / 2;
+      const int first = tm * tile_rows;
+      if (half && std::min<int64_t>(M - first, tile_rows) > kGBM / 2) fail("tile row %d has rows past the first half", tm);
       std::vector<char> cseen(kGBM * kGBN, 0);
       for (int wave = 0; wave < 8; ++wave)
         for (int l = 0; l < 64; ++l) {
@@ -612,9 +879,9 @@ struct GemmModel {
             const int r = 8 * (2 * wave + j) + (l >> 3);
             const int piece = addr::gemm_piece(l, r);
             for (int h = 0; h < 2; ++h) {
-              const int64_t ra = addr::gemm_row(tm * kGBM + h * 128 + r, static_cast<int>(M));
+              const int64_t ra = addr::gemm_row(first + h * 128 + r, static_cast<int>(M));
               const int64_t rb = addr::gemm_row(tn * kGBN + addr::gemm_b_row(r, h), static_cast<int>(N));
-              in("A offset in 32 bits", (ra - int64_t(tm) * kGBM) * lda * 2 + piece * 16, 16, int64_t(1) << 32);
+              if (h == 0 || !half) in("A offset in 32 bits", (ra - first) * lda * 2 + piece * 16, 16, int64_t(1) << 32);
               in("B offset in 32 bits", (rb - int64_t(tn) * kGBN) * ldb * 2 + piece * 16, 16, int64_t(1) << 32);
               for (int kt = 0; kt < nk; ++kt) {
                 if (h == 0 || !half) in("A", ra * lda + int64_t(kt) * kPBK + piece * 8, 8, a_elems());
@@ -628,14 +895,14 @@ struct GemmModel {
               for (int c = 0; c < 2; ++c)
                 for (int e = 0; e < 8; ++e) {
                   const int row = wm * 64 + (l & 15) + h * 128 + i * 16, col = wn * 64 + (l >> 4) * 8 + c * 32 + e;
-                  if (tm * kGBM + row >= M || tn * kGBN + col >= N) continue;
-                  in("C", int64_t(tm * kGBM + row) * ldc + tn * kGBN + col, 1, (M - 1) * ldc + N);
+                  if (first + row >= M || tn * kGBN + col >= N) continue;
+                  in("C", int64_t(first + row) * ldc + tn * kGBN + col, 1, (M - 1) * ldc + N);
                   if (cseen[row * kGBN + col]++) fail("C element (%d, %d) of a tile stored twice", row, col);
                 }
         }
-      for (int r = 0; r < kGBM; ++r)
+      for (int r = 0; r < tile_rows; ++r)
         for (int c = 0; c < kGBN; ++c)
-          if (tm * kGBM + r < M && tn * kGBN + c < N && !cseen[r * kGBN + c]) {
+          if (first + r < M && tn * kGBN + c < N && !cseen[r * kGBN + c]) {
             fail("C element (%d, %d) of tile (%d, %d) is never stored", r, c, tm, tn);
             r = kGBM;
             break;
@@ -646,6 +913,92 @@ struct GemmModel {
         fail("tile %lld of %lld is never taken", (long long)t, (long long)total);
         break;
       }
+  }
+  // gemm_bf16_tn_stream_kernel: the ring's schedule of every wave (each slot
+  // has landed when it is read, and is refilled only after its reads are
+  // back), then every workgroup's transfers and stores
+  void stream(const StreamForm& f) {
+    const int NS = f.MB + f.NB, TC = (f.RS + NS - 1) / NS, nk = static_cast<int>(K / kPBK);
+    tiles_m = static_cast<int>((M + 16 * f.MB - 1) / (16 * f.MB));
+    tiles_n = static_cast<int>((N + 16 * f.NB - 1) / (16 * f.NB));
+    int chunks_seen = 0;
+    for (int w = 0; w < f.W; ++w) {
+      const int mine = addr::gemm_s_chunks(nk, w, f.W);
+      chunks_seen += mine;
+      if (mine < TC) return fail("wave %d has %d chunks, its last %d are counted down", w, mine, TC);
+      std::vector<int64_t> held(f.RS);                       // the stream slot in each ring place
+      int64_t issued = f.RS;
+      for (int g = 0; g < f.RS; ++g) held[g] = g;
+      for (int i = 0; i < mine; ++i) {
+        const int tail = i < mine - TC ? -1 : i - (mine - TC);
+        for (int s = 0; s < NS + f.LA; ++s) {
+          const int64_t g = int64_t(i) * NS + s;
+          if (s < NS) {
+            const int done = s > f.LA ? s - f.LA : 0;
+            const int iss = tail < 0 ? f.RS + done : std::min(f.RS + tail * NS + done, TC * NS) - tail * NS;
+            const int young = std::min(2 * (iss - 1 - s), 63);
+            ++checked;
+            if (2 * (issued - 1 - g) < young) fail("slot %lld is read before it has landed", (long long)g);
+            if (held[g % f.RS] != g) fail("slot %lld is not in its ring place", (long long)g);
+          }
+          const int d = s - f.LA;
+          if (d >= 0 && (tail < 0 || tail * NS + d + f.RS < TC * NS)) {
+            const int64_t gd = int64_t(i) * NS + d, nx = gd + f.RS;
+            in("chunk", i + (d + f.RS) / NS, 1, mine);
+            if (nx != int64_t(i + (d + f.RS) / NS) * NS + (d + f.RS) % NS || nx != issued)
+              fail("slot %lld is refilled out of order", (long long)gd);
+            held[gd % f.RS] = nx;
+            ++issued;
+          }
+        }
+      }
+      if (issued != int64_t(mine) * NS) fail("wave %d moved %lld slots of %lld", w, (long long)issued, (long long)mine * NS);
+    }
+    if (chunks_seen != nk) fail("the waves take %d chunks of %d", chunks_seen, nk);
+    for (int l = 0; l < 64; ++l) {                           // LDS: a slot's transfers and operand reads
+      const int i16 = l & 15, q = l >> 4, pos = (q ^ addr::lds_swz(i16)) * 16;
+      for (int k = 0; k < 2; ++k) {
+        in("operand (LDS)", i16 * kPRow + (pos ^ (64 * k)), 16, 16 * kPRow);
+        if ((((pos ^ (64 * k)) / 16) ^ addr::lds_swz(i16)) != q + 4 * k) fail("operand reads another piece");
+      }
+      for (int t = 0; t < 2; ++t) {
+        const int r = 8 * t + (l >> 3);
+        if ((addr::gemm_piece(l, r) ^ addr::lds_swz(r)) != (l & 7)) fail("transfer lands at another piece");
+      }
+    }
+    std::vector<char> cseen(static_cast<size_t>(M) * N, 0);
+    const int64_t total = int64_t(tiles_m) * tiles_n;
+    for (int64_t b = 0; b < 8 * ((total + 7) / 8); ++b) {
+      int tm, tn;
+      if (!addr::gemm_tile(static_cast<int>(b), tiles_m, tiles_n, tiles_m, tm, tn)) continue;
+      const int row0 = tm * 16 * f.MB, col0 = tn * 16 * f.NB;
+      for (int l = 0; l < 64; ++l) {
+        for (int s = 0; s < NS; ++s)
+          for (int t = 0; t < 2; ++t) {
+            const int r = 8 * t + (l >> 3), piece = addr::gemm_piece(l, r);
+            const bool isb = s < f.NB;
+            const int64_t row = isb ? addr::gemm_row(col0 + addr::gemm_s_brow(r, s, f.NB), static_cast<int>(N))
+                                    : addr::gemm_row(row0 + 16 * (s - f.NB) + r, static_cast<int>(M));
+            const int64_t ld = isb ? ldb : lda;
+            in("offset in 32 bits", (row - (isb ? col0 : row0)) * ld * 2 + piece * 16, 16, int64_t(1) << 32);
+            for (int kt = 0; kt < nk; ++kt)
+              in(isb ? "B" : "A", row * ld + int64_t(kt) * kPBK + piece * 8, 8, isb ? b_elems() : a_elems());
+          }
+        const int NP = f.NB / 2;
+        for (int u = 0; u < f.MB * NP; ++u)
+          for (int e = 0; e < 8; ++e) {
+            const int row = row0 + (u / NP) * 16 + (l & 15), col = col0 + (u % NP) * 32 + (l >> 4) * 8 + e;
+            // element e of the lane: matrix row 4 (l / 16) + e % 4 of block 2 (u % NP) + e / 4
+            if (addr::gemm_s_brow(4 * (l >> 4) + (e & 3), 2 * (u % NP) + (e >> 2), f.NB) != col - col0)
+              fail("column %d is stored from another B row", col);
+            if (row >= M || col >= N) continue;
+            in("C", int64_t(row) * ldc + col, 1, (M - 1) * ldc + N);
+            if (cseen[int64_t(row) * N + col]++) fail("C element (%d, %d) stored twice", row, col);
+          }
+      }
+    }
+    for (char c : cseen)
+      if (!c) return fail("an element of C is never stored");
   }
   // gemm_bf16_tn_kernel<KTAIL, WM, WN>
   void reg(bool KTAIL, int WM, int WN) {
@@ -723,7 +1076,18 @@ int gs_gemm_bf16_tn(const void* a, int64_t lda, const void* b, int64_t ldb, void
   const unsigned grid = static_cast<unsigned>(8 * ((total + 7) / 8));
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (pingpong_form(K, lda, ldb)) {
-    p.thin = gemm_thin(M);
+    const GemmPick pick = pick_gemm(M, N, K);
+    if (pick.stream != nullptr) {
+      p.tiles_m = static_cast<int>((M + 16 * pick.stream->MB - 1) / (16 * pick.stream->MB));
+      p.tiles_n = static_cast<int>((N + 16 * pick.stream->NB - 1) / (16 * pick.stream->NB));
+      const int64_t n = 8 * ((static_cast<int64_t>(p.tiles_m) * p.tiles_n + 7) / 8);
+      hipLaunchKernelGGL(pick.stream->kernel, dim3(static_cast<unsigned>(n)), dim3(64 * pick.stream->W), 0, st, p);
+      GS_CHECK_LAUNCH(who);
+      return GS_OK;
+    }
+    p.tile_rows = pick.tile_rows;
+    p.tiles_m = static_cast<int>((M + p.tile_rows - 1) / p.tile_rows);
+    p.thin = p.tile_rows == kGBM ? gemm_thin(M) : 0;
     const unsigned n = static_cast<unsigned>(addr::gemm_thin_grid(p.tiles_m, p.tiles_n, p.thin));
     hipLaunchKernelGGL(gemm_bf16_tn_pingpong_kernel, dim3(n), dim3(512), 0, st, p);
   } else if (K % kGBK == 0) launch_gemm<false>(grid, p, st);
@@ -745,7 +1109,14 @@ int64_t gs_check_gemm_addresses(int64_t M, int64_t N, int64_t K, int64_t lda, in
   m.ldc = ldc;
   m.tiles_m = static_cast<int>((M + kGBM - 1) / kGBM);
   m.tiles_n = static_cast<int>((N + kGBN - 1) / kGBN);
-  if (pingpong_form(K, lda, ldb)) m.pingpong();
+  if (pingpong_form(K, lda, ldb)) {
+    m.pingpong(kGBM);
+    m.pingpong(kGBM / 2);
+    for (const StreamForm& f : kStreamForms)
+      if (K / kPBK / f.W >= (f.RS + f.MB + f.NB - 1) / (f.MB + f.NB)) m.stream(f);
+    m.tiles_m = static_cast<int>((M + kGBM - 1) / kGBM);
+    m.tiles_n = static_cast<int>((N + kGBN - 1) / kGBN);
+  }
   m.reg(K % kGBK != 0, 2, 4);      // the register-staged form takes any shape
   if (checked) *checked = m.checked;
   if (msg && msg_len > 0) snprintf(msg, static_cast<size_t>(msg_len), "%s", m.msg);

@@ -57,10 +57,24 @@ def test_gemm_pingpong_tile_edges(dev, M, N, K):
     test_gemm_matches_fp32_reference(dev, M, N, K, M + N)
 
 
-def test_gemm_strided_rows_and_output(dev):
+@pytest.mark.parametrize("M,N,K", [
+    # streaming forms, K from the fewest chunks a wave may have to uneven shares of them; ragged rows and columns
+    (1, 33, 1088), (7, 4480, 4096), (16, 45, 1024),                   # 16 x 32 tiles
+    (32, 7296, 1088), (27, 9001, 768),                                # 32 x 32
+    (64, 7296, 1024), (49, 8003, 576),                                # 64 x 32
+    (128, 7296, 576), (113, 16000, 512), (70, 14989, 1344),           # 64 x 64
+    (256, 7296, 512), (255, 7290, 1152), (300, 6149, 832),            # 128 x 64
+    # 128-row tiles of the ping-pong form (too few 256-row ones to fill the CUs)
+    (777, 7296, 256), (1100, 6001, 192), (129, 300, 128),
+])
+def test_gemm_forms_for_few_tiles(dev, M, N, K):
+    test_gemm_matches_fp32_reference(dev, M, N, K, M + N + K)
+
+
+@pytest.mark.parametrize("M,N,K", [(333, 520, 1024), (200, 9000, 640), (900, 7000, 320)])
+def test_gemm_strided_rows_and_output(dev, M, N, K):
     """x and out with row strides (a view into a wider buffer), as the layer's x_ext slices are."""
     g = torch.Generator(device=dev).manual_seed(11)
-    M, N, K = 333, 520, 1024
     xb = torch.randn(M, K + 64, generator=g, device=dev).to(torch.bfloat16)
     x = xb[:, 32:32 + K]
     w = (torch.randn(N, K, generator=g, device=dev) / K ** 0.5).to(torch.bfloat16)
