@@ -68,6 +68,21 @@ GS_HD int64_t reg_a_elem(bool ok, int j, int64_t astep_elems, int64_t kp, int64_
 GS_HD int64_t reg_x_elem(bool ok, int64_t kp, int64_t k_lo) { return ok ? kp : k_lo; }
 
 // ---- expand (expand_kernel, expand_sparse_kernel) --------------------------
+// Part i of `parts` near-equal contiguous ranges of n items: [lo, lo + count).
+GS_HD void even_range(int n, int parts, int i, int& lo, int& count) {
+  const int q = n / parts, r = n - q * parts;
+  lo = i * q + imin(i, r);
+  count = q + (i < r ? 1 : 0);
+}
+// The sub-tiles of workgroup b of an expand launch of `grid` (a multiple of 8)
+// workgroups, as positions tile * n_sub + sub of `total` tiles: XCD b % 8
+// takes an eighth of them, its workgroups near-equal shares of that.
+GS_HD void expand_span(int b, int grid, int total, int n_sub, int& lo, int& count) {
+  int xlo, xn;
+  even_range(total * n_sub, 8, b & 7, xlo, xn);
+  even_range(xn, grid >> 3, b >> 3, lo, count);
+  lo += xlo;
+}
 // First output column of the lane's 16-byte y piece in sub-tile sub of NT
 // columns (the last piece of a partial sub-tile re-reads the row's last one).
 GS_HD int64_t y_col(int sub, int nt, int cx, int out_total, int epl) {

@@ -395,22 +395,20 @@ __device__ __forceinline__ TileRef find_tile(const int32_t* __restrict__ seg, co
   return ref;
 }
 
-// The tile of work item `lin` of a 1-D launch over (tile, sub) pairs (see
-// work_item), in one pass over the adapter table when it fits one wave
-// (<= 64 adapters): the tile count and the tile's lookup share the same
-// loads.  nsub_of(total tiles) gives the number of subs per tile (every wave
-// computes the same value); the tile count is returned in `total_out` (a
-// workgroup that loops over items finds its later tiles with tile_at).
-// Returns g = 0 when the item has no tile.
-template <int TM, bool BAL = false, typename NsubOf>
-__device__ __forceinline__ TileRef locate_tile_by(const int32_t* __restrict__ seg, const int32_t* __restrict__ ranks,
-                                                  const int64_t* __restrict__ offs, int num_adapters, RankWindow rw,
-                                                  int lin, bool flat, NsubOf nsub_of, int& sub, int& total_out) {
+// The tile of a workgroup's (first) item, in one pass over the adapter table
+// when it fits one wave (<= 64 adapters): the tile count and the tile's lookup
+// share the same loads.  item_of(total tiles) names the item (every wave
+// computes the same value; tile -1: none); the tile count is returned in
+// `total_out`.  Returns g = 0 when the item has no tile.
+template <int TM, bool BAL = false, typename ItemOf>
+__device__ __forceinline__ TileRef locate_item(const int32_t* __restrict__ seg, const int32_t* __restrict__ ranks,
+                                               const int64_t* __restrict__ offs, int num_adapters, RankWindow rw,
+                                               ItemOf item_of, int& sub, int& total_out) {
   TileRef ref{0, 0, 0, 0, 0};
   if (num_adapters > 64) {
     const int total = count_tiles<TM>(seg, ranks, num_adapters, rw);
     total_out = total;
-    const XcdItem it = work_item(lin, total, nsub_of(total), flat);
+    const XcdItem it = item_of(total);
     sub = it.sub;
     return it.tile < 0 ? ref : find_tile<TM, BAL>(seg, ranks, offs, num_adapters, rw, it.tile);
   }
@@ -433,7 +431,7 @@ __device__ __forceinline__ TileRef locate_tile_by(const int32_t* __restrict__ se
   }
   const int total = __shfl(incl, 63, 64);
   total_out = total;
-  const XcdItem it = work_item(lin, total, nsub_of(total), flat);
+  const XcdItem it = item_of(total);
   sub = it.sub;
   if (it.tile < 0) return ref;
   const int excl = incl - ntiles;
@@ -448,6 +446,17 @@ __device__ __forceinline__ TileRef locate_tile_by(const int32_t* __restrict__ se
   ref.rank = __shfl(rk, src, 64);
   ref.off = __shfl(of, src, 64);
   return ref;
+}
+
+// The tile of work item `lin` of a 1-D launch over (tile, sub) pairs (see
+// work_item).  nsub_of(total tiles) gives the number of subs per tile; a
+// workgroup that loops over items finds its later tiles with tile_at.
+template <int TM, bool BAL = false, typename NsubOf>
+__device__ __forceinline__ TileRef locate_tile_by(const int32_t* __restrict__ seg, const int32_t* __restrict__ ranks,
+                                                  const int64_t* __restrict__ offs, int num_adapters, RankWindow rw,
+                                                  int lin, bool flat, NsubOf nsub_of, int& sub, int& total_out) {
+  return locate_item<TM, BAL>(seg, ranks, offs, num_adapters, rw,
+                              [&](int total) { return work_item(lin, total, nsub_of(total), flat); }, sub, total_out);
 }
 
 // As locate_tile_by with a fixed number of subs per tile.

@@ -488,14 +488,20 @@ __global__ __launch_bounds__(kThreads) void reduce_parts_kernel(const float* __r
 }
 
 // ----------------------------------------------------------------------------
-// Expand.  1-D grid over (tile, group of column sub-tiles) items, tiles
-// spread over the XCDs in contiguous ranges (xcd_item).  A workgroup owns one
-// tile (32 slots of one adapter) and walks its group's consecutive column
-// sub-tiles of NT columns.  The number of groups per tile is chosen on the
-// device from the batch's tile count so that the items about fill the GPU
-// once (wt workgroups): each workgroup's start -- the tile lookup and the
-// staging of its shrink values -- is paid once per group, and a group long
-// enough to hide it beats a second round of workgroups.  The tile's shrink values for every slice (z rows, or the sum of
+// Expand.  The batch's (tile, column sub-tile of NT columns) pairs, tile by
+// tile (a tile is up to 32 slots of one adapter), are cut into one contiguous
+// span per workgroup of a launch that fills the GPU once (addr::expand_span):
+// an eighth of them to each XCD, so an adapter's tiles mostly share an L2, and
+// equal shares to its workgroups.  A span mostly lies inside one tile, whose
+// start -- the tile lookup and the staging of its shrink values -- is then
+// paid once per workgroup; one that crosses into the next tile pays it again.
+// Whole column groups per tile in place of spans left workgroup slots without
+// work and XCDs with fewer tiles than others: 4096 rows x 4096 of 48 adapters
+// 17.5 -> 16.1 us, 256 x 6144 of 12 (13 tiles) 7.0 -> 6.3, and 22.2 -> 18.6
+// in the pair expand.  From there it is bound by the y stream: 4500 rows x
+// 25600 take 97 us, 4.76 TB/s read + written, the rate of a bare
+// read-modify-write of the same rows (4.7 TB/s).
+// The tile's shrink values for every slice (z rows, or the sum of
 // the split-K partials rounded to the element type exactly like a
 // materialised z) are staged in LDS once.  Per sub-tile each wave computes NBW
 // 32x32 delta blocks with MFMA over the adapter's rank (all KSTEP k-groups of
@@ -522,7 +528,6 @@ struct ExpandParams {
   const int32_t* ranks;
   int NA;
   int max_rank;
-  int wt;                 // workgroups that fill the GPU once
   const int32_t* seg;
   const int32_t* perm;
   RankWindow rw;          // adapters of this launch's rank class
@@ -592,16 +597,6 @@ __device__ __forceinline__ void z_stage(const ExpandParams& p, const TileRef& tr
       *reinterpret_cast<f32x4*>(dst) = f32x4{v[0], v[1], v[2], v[3]};
     }
   }
-}
-
-// Column groups per tile: as many as keep 8*ceil(tiles/8) * groups within wt
-// (the launch holds max(wt, 8*ceil(max_tiles/8)) workgroups), 1..n_sub.
-__host__ __device__ inline int expand_groups(int tiles, int n_sub, int wt) {
-  const int t8 = 8 * ((tiles + 7) / 8);
-  int g = t8 > 0 ? wt / t8 : n_sub;
-  if (g > n_sub) g = n_sub;
-  if (g < 1) g = 1;
-  return g;
 }
 
 // An adapter's slots are cut into 32-slot tiles of near-equal size (the
@@ -821,37 +816,57 @@ __device__ __forceinline__ void expand_item(const ExpandParams& p, const TileRef
   compute(sub0 + nsub - 1, bc, yc);
 }
 
-// LOOP = false: one item per workgroup (the grid covers the items).  LOOP =
-// true (a rank class expected to hold few tiles, laid out flat with one
-// sub-tile per item, grid capped at one round): a workgroup takes items
-// blockIdx.x, + gridDim.x, ... while they lie in the batch's item range.  A
-// separate instantiation, so the one-item form keeps its registers.
+// A workgroup's span of a launch of `grid` workgroups (addr::expand_span).
+// before_last() runs before the span's last sub-tile's products.
+template <bool BF16, int NBW, int PRE, typename Hook = NoHook>
+__device__ __forceinline__ void expand_walk(const ExpandParams& p, float (&dtile)[kTM][4 * NBW * 32 + kOutPad],
+                                            char* zs, Hook before_last = Hook{}) {
+  constexpr int NT = 4 * NBW * 32;
+  const int n_sub = (p.out_total + NT - 1) / NT;
+  int lo = 0, left = 0, sub = 0, total = 0;
+  TileRef tr = locate_item<kTM, kExpandBalanced>(p.seg, p.ranks, p.b_off, p.NA, p.rw,
+                                                 [&](int tot) {
+                                                   addr::expand_span(static_cast<int>(blockIdx.x),
+                                                                     static_cast<int>(gridDim.x), tot, n_sub, lo, left);
+                                                   return left > 0 ? XcdItem{lo / n_sub, lo % n_sub} : XcdItem{-1, 0};
+                                                 }, sub, total);
+  if (left <= 0) return;
+  int tile = lo / n_sub;
+  for (;;) {
+    const int n = min(left, n_sub - sub);
+    left -= n;
+    expand_item<BF16, NBW, PRE, false>(p, tr, sub, n, p.nparts, dtile, zs, [&]() {
+      if (left == 0) before_last();
+    });
+    if (left == 0) return;
+    // the item's last barrier is past every read of zs and dtile
+    tr = find_tile<kTM, kExpandBalanced>(p.seg, p.ranks, p.b_off, p.NA, p.rw, ++tile);
+    sub = 0;
+  }
+}
+
+// LOOP = false: the workgroups' spans.  LOOP = true (a rank class expected to
+// hold few tiles, laid out flat with one sub-tile per item, grid capped at one
+// round): a workgroup takes items blockIdx.x, + gridDim.x, ... while they lie
+// in the batch's item range.
 // The narrow bf16 forms up to rank 64 hold 4 workgroups per CU (<= 128
 // registers per lane; the rank-64 multiswitch projection measured faster at
 // 4 than at 3).
 template <bool BF16, int NBW, int PRE, bool LOOP>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BF16 && NBW == 1 && PRE <= 4 && !LOOP ? 4 : 1)))
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(!BF16 || LOOP || PRE > 4 ? 1 : (NBW == 1 ? 4 : 3))))
 void expand_kernel(ExpandParams p) {
   constexpr int NT = 4 * NBW * 32;
   __shared__ float dtile[kTM][NT + kOutPad];
   extern __shared__ __align__(16) char zs[];   // [32][S*max_rank + 8] element type
-  const int n_sub = (p.out_total + NT - 1) / NT;
-  const bool flat = LOOP;                      // the looping form is the flat one
-  int lin = static_cast<int>(blockIdx.x);
-  int sub = 0, groups = 1, total = 0;
-  TileRef tr = locate_tile_by<kTM, kExpandBalanced>(p.seg, p.ranks, p.b_off, p.NA, p.rw, lin, flat,
-                                                    [&](int tot) {
-                                                      groups = flat ? n_sub : expand_groups(tot, n_sub, p.wt);
-                                                      return groups;
-                                                    }, sub, total);
   if constexpr (!LOOP) {
-    if (tr.g == 0) return;
-    // group sub of `groups` covers sub-tiles [sub*n_sub/groups, (sub+1)*n_sub/groups)
-    const int sub0 = (sub * n_sub) / groups;
-    const int nsub = ((sub + 1) * n_sub) / groups - sub0;
-    if (nsub > 0) expand_item<BF16, NBW, PRE, false>(p, tr, sub0, nsub, p.nparts, dtile, zs);
+    expand_walk<BF16, NBW, PRE>(p, dtile, zs);
     return;
   }
+  const int n_sub = (p.out_total + NT - 1) / NT;
+  int lin = static_cast<int>(blockIdx.x);
+  int sub = 0, total = 0;
+  TileRef tr = locate_tile_by<kTM, kExpandBalanced>(p.seg, p.ranks, p.b_off, p.NA, p.rw, lin, true,
+                                                    [&](int) { return n_sub; }, sub, total);
   // the shrink's k-split when it chose it on the device: the same function of
   // the same 64-slot tile count
   int nparts = p.nparts;
@@ -859,17 +874,13 @@ void expand_kernel(ExpandParams p) {
     const int ks = dyn_ksplit(count_tiles<kTMS>(p.seg, p.ranks, p.NA, p.rw), p.ks_chunks, p.ks_target, p.nparts);
     nparts = ks > 1 ? ks : 0;
   }
-  const int items = work_items(total, groups, flat);
+  const int items = work_items(total, n_sub, true);
   for (;;) {
-    if (tr.g != 0) {
-      const int sub0 = (sub * n_sub) / groups;
-      const int nsub = ((sub + 1) * n_sub) / groups - sub0;
-      if (nsub > 0) expand_item<BF16, NBW, PRE, true>(p, tr, sub0, nsub, nparts, dtile, zs);
-    }
+    if (tr.g != 0) expand_item<BF16, NBW, PRE, true>(p, tr, sub, 1, nparts, dtile, zs);
     lin += static_cast<int>(gridDim.x);
     if (lin >= items) break;
     lds_barrier();                         // every wave is done with zs and dtile before the next item
-    tr = tile_at<kTM, kExpandBalanced>(p.seg, p.ranks, p.b_off, p.NA, p.rw, lin, flat, total, groups, sub);
+    tr = tile_at<kTM, kExpandBalanced>(p.seg, p.ranks, p.b_off, p.NA, p.rw, lin, true, total, n_sub, sub);
   }
 }
 
@@ -1166,29 +1177,14 @@ __global__ __launch_bounds__(kThreads) void expand_pair_kernel(ExpandParams p0, 
   auto& dtile = *reinterpret_cast<float(*)[kTM][NT + kOutPad]>(buf);
   auto& red = *reinterpret_cast<float(*)[2][kTM][32 * kPairQB + kOutPad]>(buf);
   int ticket = 0;
-  bool early = false;                      // uniform: the small item ran and claimed
-  {
-    const int n_sub = (p0.out_total + NT - 1) / NT;
-    int sub = 0, groups = 1, total = 0;
-    const TileRef tr = locate_tile_by<kTM, kExpandBalanced>(p0.seg, p0.ranks, p0.b_off, p0.NA, p0.rw,
-                                                            static_cast<int>(blockIdx.x), false,
-                                                            [&](int tot) {
-                                                              groups = expand_groups(tot, n_sub, p0.wt);
-                                                              return groups;
-                                                            }, sub, total);
-    // the first claim goes out before the small item's last sub-tile, so
-    // its round trip passes while that sub-tile is computed; its result is
-    // written to LDS only afterwards (no wait for it before)
-    if (tr.g != 0) {
-      const int sub0 = (sub * n_sub) / groups;
-      const int nsub = ((sub + 1) * n_sub) / groups - sub0;
-      if (nsub > 0)
-        expand_item<true, NBW, PRE, false>(p0, tr, sub0, nsub, p0.nparts, dtile, zs, [&]() {
-          if (threadIdx.x == 0) ticket = claim_next(claim);
-          early = true;
-        });
-    }
-  }
+  bool early = false;                      // uniform: the small items ran and claimed
+  // the first claim goes out before the small class's last sub-tile, so its
+  // round trip passes while that sub-tile is computed; its result is written
+  // to LDS only afterwards (no wait for it before)
+  expand_walk<true, NBW, PRE>(p0, dtile, zs, [&]() {
+    if (threadIdx.x == 0) ticket = claim_next(claim);
+    early = true;
+  });
   const int n_sub1 = p1.out_total / (32 * kPairQB);
   const int total1 = count_tiles<kTM>(p1.seg, p1.ranks, p1.NA, p1.rw);
   const int items1 = work_items(total1, n_sub1, true);
@@ -1506,15 +1502,10 @@ int prepare_expand(ExpandParams& p, const char* who, int32_t dtype, void* y, int
   return GS_OK;
 }
 
-// Workgroups of a column-split expand launch: the items never exceed wt (or
-// one per tile slot when the tiles alone exceed it) nor one per (tile slot,
-// sub-tile); a flat launch is one round of workgroups that loop over its
-// (tile, sub-tile) items.
-int64_t expand_grid(int64_t wt, int max_tiles, int64_t n_sub, bool flat) {
-  const int64_t t8 = 8 * ((static_cast<int64_t>(max_tiles) + 7) / 8);
-  const int64_t items = flat ? std::min<int64_t>(wt, static_cast<int64_t>(max_tiles) * n_sub)
-                             : std::min<int64_t>(std::max(wt, t8), t8 * n_sub);
-  return (items + 7) / 8 * 8;
+// Workgroups of a column-split expand launch: one round (wt), at most one per
+// (tile slot, sub-tile); a multiple of 8 (addr::expand_span).
+int64_t expand_grid(int64_t wt, int max_tiles, int64_t n_sub) {
+  return (std::min<int64_t>(wt, static_cast<int64_t>(max_tiles) * n_sub) + 7) / 8 * 8;
 }
 
 // Workgroups of a rank-split (sparse) expand launch: one round, at most one
@@ -1539,19 +1530,19 @@ void launch_expand_t(int max_tiles, size_t lds, ExpandParams p, hipStream_t st) 
     o = (static_cast<uint64_t>(lds) << 16) | static_cast<uint64_t>(std::min(n, 0xffff));
     occ.store(o, std::memory_order_relaxed);
   }
-  p.wt = static_cast<int>(o & 0xffff) * device_cus();
   constexpr int NT = 4 * NBW * 32;
-  const int grid = static_cast<int>(expand_grid(p.wt, max_tiles, (p.out_total + NT - 1) / NT, p.flat != 0));
+  const int grid = static_cast<int>(expand_grid(static_cast<int64_t>(o & 0xffff) * device_cus(), max_tiles,
+                                                (p.out_total + NT - 1) / NT));
   hipLaunchKernelGGL(kern, dim3(grid), dim3(kThreads), lds, st, p);
 }
 
-template <bool BF16, int NBW>
-void launch_expand_pre(int max_tiles, size_t lds, const ExpandParams& p, hipStream_t st) {
-  constexpr int KSTEP = BF16 ? 16 : 8;
-  const int need = (p.max_rank + KSTEP - 1) / KSTEP;
-  if (need <= 2) launch_expand_t<BF16, NBW, 2>(max_tiles, lds, p, st);
-  else if (need <= 4) launch_expand_t<BF16, NBW, 4>(max_tiles, lds, p, st);
-  else launch_expand_t<BF16, NBW, 8>(max_tiles, lds, p, st);
+// NBW = 2 is chosen for at most 2 k-groups of lora_B only (expand_form).
+template <bool BF16>
+void launch_expand_form(int NBW, int PRE, int max_tiles, size_t lds, const ExpandParams& p, hipStream_t st) {
+  if (NBW == 2) launch_expand_t<BF16, 2, 2>(max_tiles, lds, p, st);
+  else if (PRE == 2) launch_expand_t<BF16, 1, 2>(max_tiles, lds, p, st);
+  else if (PRE == 4) launch_expand_t<BF16, 1, 4>(max_tiles, lds, p, st);
+  else launch_expand_t<BF16, 1, 8>(max_tiles, lds, p, st);
 }
 
 // The rank-split expand takes a sparse bf16 class whose sub-tiles of 128
@@ -1625,13 +1616,8 @@ void launch_expand(bool bf16, int64_t T, int adapters, ExpandParams p, hipStream
   }
   const int max_tiles = max_tiles_for(T, adapters);
   const size_t lds = expand_lds_bytes(bf16, p.si.S, p.max_rank);
-  if (bf16) {
-    if (f.NBW == 2) launch_expand_pre<true, 2>(max_tiles, lds, p, st);
-    else launch_expand_pre<true, 1>(max_tiles, lds, p, st);
-  } else {
-    if (f.NBW == 2) launch_expand_pre<false, 2>(max_tiles, lds, p, st);
-    else launch_expand_pre<false, 1>(max_tiles, lds, p, st);
-  }
+  if (bf16) launch_expand_form<true>(f.NBW, f.PRE, max_tiles, lds, p, st);
+  else launch_expand_form<false>(f.NBW, f.PRE, max_tiles, lds, p, st);
 }
 
 
@@ -1711,12 +1697,11 @@ int pair_expand_occupancy(const void* kern, size_t lds) {
   return n;
 }
 
-// The pair expand's grid: the small class's one-item grid at the pair
-// kernel's occupancy (sets e0.wt, which its items' column groups follow).
-int64_t pair_expand_grid(const PairForm& f, int64_t T, int adapters0, size_t lds, ExpandParams& e0) {
-  e0.wt = pair_expand_occupancy(expand_pair_fn_of(f), lds) * device_cus();
+// The pair expand's grid: the small class's, at the pair kernel's occupancy.
+int64_t pair_expand_grid(const PairForm& f, int64_t T, int adapters0, size_t lds, const ExpandParams& e0) {
+  const int64_t wt = static_cast<int64_t>(pair_expand_occupancy(expand_pair_fn_of(f), lds)) * device_cus();
   const int NT = 4 * f.f0.NBW * 32;
-  return expand_grid(e0.wt, max_tiles_for(T, adapters0), (e0.out_total + NT - 1) / NT, false);
+  return expand_grid(wt, max_tiles_for(T, adapters0), (e0.out_total + NT - 1) / NT);
 }
 
 void launch_shrink_pair(const PairForm& f, int64_t grid, const ShrinkParams& p0, const ShrinkParams& p1, int* claim,
@@ -2078,15 +2063,8 @@ struct AddrModel {
     const int KSTEP = bf16 ? 16 : 8, KHALF = KSTEP / 2;
     const int LPR = NT / EPL, RPI = kThreads / LPR, PASSES = kTM / RPI;
     const int64_t zs_ld = static_cast<int64_t>(si.S) * e.max_rank + 8, lds = kTM * zs_ld * ES;
-    const int groups = flat ? n_sub : expand_groups(total, n_sub, static_cast<int>(wt));
-    for_items("expand_kernel", expand_grid(wt, max_tiles, n_sub, flat), flat, work_items(total, groups, flat),
-              [&](int lin) {
-      const XcdItem it = work_item(lin, total, groups, flat);
-      if (it.tile < 0) return;
-      const TileRef& tr = tl[it.tile];
+    auto item = [&](const TileRef& tr, int sub0, int nsub) {
       const int r = tr.rank;
-      const int sub0 = (it.sub * n_sub) / groups, nsub = ((it.sub + 1) * n_sub) / groups - sub0;
-      if (nsub <= 0) return;
       const int nchunk = (r + f.PRE * KSTEP - 1) / (f.PRE * KSTEP);
       for (int sb = sub0; sb < sub0 + nsub; ++sb) {
         for (int wave = 0; wave < 4; ++wave)
@@ -2119,7 +2097,32 @@ struct AddrModel {
       s_hi = s_lo;
       while (s_hi + 1 < si.S && c_last >= si.bounds[s_hi + 1]) ++s_hi;
       stage(tr, s_lo, s_hi, s_lo * r, zs_ld, lds, nparts);
-    });
+    };
+    const int64_t grid = expand_grid(wt, max_tiles, n_sub);
+    if (flat) {
+      for_items("expand_kernel", grid, true, work_items(total, n_sub, true), [&](int lin) {
+        const XcdItem it = work_item(lin, total, n_sub, true);
+        item(tl[it.tile], it.sub, 1);
+      });
+      return;
+    }
+    // the workgroups' spans: each (tile, sub-tile) exactly once, in order per XCD
+    std::vector<char> seen(static_cast<size_t>(total) * n_sub, 0);
+    for (int64_t b = 0; b < grid; ++b) {
+      int lo = 0, left = 0;
+      addr::expand_span(static_cast<int>(b), static_cast<int>(grid), total, n_sub, lo, left);
+      while (left > 0) {
+        const int tile = lo / n_sub, sub = lo % n_sub, n = std::min(left, n_sub - sub);
+        if (!in("expand span", lo, n, static_cast<int64_t>(total) * n_sub)) break;
+        for (int k = 0; k < n; ++k)
+          if (seen[lo + k]++) fail("expand_kernel: (tile %d, sub-tile %d) is taken twice", tile, sub + k);
+        item(tl[tile], sub, n);
+        lo += n;
+        left -= n;
+      }
+    }
+    for (size_t k = 0; k < seen.size(); ++k)
+      if (!seen[k]) fail("expand_kernel: (tile %d, sub-tile %d) is not taken", static_cast<int>(k / n_sub), static_cast<int>(k % n_sub));
   }
 };
 }  // namespace

@@ -271,6 +271,22 @@ def test_one_adapter_past_2e18_slots(dev):
     _check_module(md, y, ids, np.arange(T), torch.bfloat16, hf_too=False)
 
 
+@pytest.mark.parametrize("T,NA,rank,slices", [
+    (40000, 3, 8, (128,)),              # more tiles than workgroups, one sub-tile each: a span is several tiles
+    (12000, 40, 32, (256, 128, 128)),   # spans that cross tiles, adapters and slices
+    (9000, 100, 64, (384,)),            # more than 64 adapters (the two-pass tile lookup), the 128-column form
+    (33, 2, 16, (4096,)),               # fewer sub-tiles than workgroups: some have no span
+])
+def test_expand_spans(dev, T, NA, rank, slices):
+    H, rng = 64, np.random.default_rng(T)
+    spec = workloads.ModuleSpec("spans", H, slices, [rank] * NA, rank)
+    md = workloads.make_module(spec, T, NA, torch.bfloat16, dev, seed=T)
+    r = workloads.Routing(req_ids=rng.integers(0, NA + 1, size=T), positions=np.arange(T),
+                          cu_seqlens=np.array([0, T], dtype=np.int32), act_offsets=None)
+    y, _, _ = _run_module(dev, md, r, NA)
+    _check_module(md, y, r.req_ids, slice(0, T), torch.bfloat16, hf_too=False)
+
+
 @pytest.mark.parametrize("ranks,slices,H", [([8, 24, 40, 64], (96,), 1000), ([16, 512], (32, 64), 264),
                                             ([128, 8], (4096, 1024, 1024), 4096)])
 def test_odd_shapes(dev, ranks, slices, H):
