@@ -141,8 +141,14 @@ def call(name: str, *args) -> int:
     return rc
 
 
+# the stream's handle without a Stream object around it (a launch asks once)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_ptr(device: torch.device | None = None) -> int:
     """hipStream_t of torch's current stream on ``device``."""
+    if device is not None and device.index is not None and _raw_stream is not None:
+        return _raw_stream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 

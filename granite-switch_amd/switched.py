@@ -68,20 +68,22 @@ class Segments:
     work: torch.Tensor | None = None
 
 
-def _as_i64(t, device):
+def _as_int(t, device, dtype):
     if t is None:
         return None
     if not isinstance(t, torch.Tensor):
         t = torch.as_tensor(t)
-    return t.to(device=device, dtype=torch.int64).contiguous()
+    elif t.dtype == dtype and t.device == device and t.is_contiguous():
+        return t
+    return t.to(device=device, dtype=dtype).contiguous()
+
+
+def _as_i64(t, device):
+    return _as_int(t, device, torch.int64)
 
 
 def _as_i32(t, device):
-    if t is None:
-        return None
-    if not isinstance(t, torch.Tensor):
-        t = torch.as_tensor(t)
-    return t.to(device=device, dtype=torch.int32).contiguous()
+    return _as_int(t, device, torch.int32)
 
 
 def build_segments(adapter_ids: torch.Tensor, num_adapters: int, positions=None, cu_seqlens=None,
@@ -100,7 +102,7 @@ def build_segments(adapter_ids: torch.Tensor, num_adapters: int, positions=None,
     """
     _require_cuda(adapter_ids)
     dev = adapter_ids.device
-    ids = _as_i64(adapter_ids.reshape(-1), dev)
+    ids = _as_i64(adapter_ids if adapter_ids.dim() == 1 else adapter_ids.reshape(-1), dev)
     T = ids.shape[0]
     pos = _as_i64(positions, dev)
     cu = _as_i32(cu_seqlens, dev)
@@ -239,10 +241,21 @@ class PackedAdapters:
 
     def rank_split(self) -> tuple:
         """(adapters of rank <= 64, adapters of larger rank) as restricted packs
-        (either may be None).  The one-launch decode kernel takes the first;
-        the segment kernels plan and launch each class for its own ranks."""
-        cut = _lib.GS_RANK_CLASS_SPLIT
-        return self.restricted(1, cut), self.restricted(cut + 1, _lib.GS_MAX_RANK)
+        (either may be None; the pack itself when one class holds every
+        adapter).  The one-launch decode kernel takes the first; the segment
+        kernels plan and launch each class for its own ranks."""
+        return self._host_tables().rank_split(self)
+
+    def __getstate__(self) -> dict:
+        """The fields: copies and pickles make their own host tables."""
+        return {k: v for k, v in self.__dict__.items() if k != "_host"}
+
+    def _host_tables(self) -> "_HostTables":
+        """The host tables of the pack's present fields."""
+        h = self.__dict__.get("_host")
+        if h is None or not h.matches(self):
+            h = self.__dict__["_host"] = _HostTables(self)
+        return h
 
     @staticmethod
     def from_slices(lora_A_slices, lora_B_slices, adapter_ranks=None, applicable=None) -> "PackedAdapters":
@@ -329,6 +342,55 @@ class PackedAdapters:
         )
 
 
+class _HostTables:
+    """What every call on a pack needs of its host-side fields, in the form the C
+    calls take: built at the first call and kept with the pack, since building
+    them cost a decode call more host time than its kernel runs (a 7-token
+    projection: 31 us a call for 7.7 us of kernel, 12.8 us with them).  ``matches``
+    compares the fields by value (the lists may be changed in place)."""
+
+    __slots__ = ("fields", "ranks_list", "a_list", "b_list", "bounds_list", "bounds", "ranks", "a_off", "b_off",
+                 "plan_key", "small_ws", "one_class", "_split")
+
+    def __init__(self, p: PackedAdapters):
+        self.fields = self._fields(p)
+        self.ranks_list = None if p.ranks_host is None else list(p.ranks_host)
+        self.a_list = None if p.a_off_host is None else list(p.a_off_host)
+        self.b_list = None if p.b_off_host is None else list(p.b_off_host)
+        self.bounds_list = p.slice_bounds
+        self.bounds = _i32_array(self.bounds_list)
+        self.ranks = _i32_array(self.ranks_list) if self.ranks_list else None    # None: one class up to max_rank
+        self.a_off = None if self.a_list is None else _i64_array(self.a_list)
+        self.b_off = None if self.b_list is None else _i64_array(self.b_list)
+        self.plan_key = (self.fields, tuple(self.ranks_list or ()), self.a_list is None, self.b_list is None)
+        self.small_ws = {}        # one-launch workspace bytes by token count (at most 1024 of them are eligible)
+        # the largest rank when it is max_rank and all ranks are on its side of the cut (or 0)
+        live = [r for r in self.ranks_list or () if r]
+        one = bool(live) and max(live) == p.max_rank <= _lib.GS_MAX_RANK and \
+            (min(live) > _lib.GS_RANK_CLASS_SPLIT) == (max(live) > _lib.GS_RANK_CLASS_SPLIT)
+        self.one_class = max(live) if one else None
+        self._split = None
+
+    @staticmethod
+    def _fields(p: PackedAdapters) -> tuple:
+        return (p.a_pack.dtype, p.hidden, p.num_adapters, p.max_rank, tuple(p.output_slices), p.a_pack.device)
+
+    def matches(self, p: PackedAdapters) -> bool:
+        return (self.ranks_list == p.ranks_host and self.a_list == p.a_off_host and self.b_list == p.b_off_host
+                and self.fields == self._fields(p))
+
+    def rank_split(self, p: PackedAdapters) -> tuple:
+        """``PackedAdapters.rank_split``; the views share p's device tensors, and
+        are made again when those are replaced."""
+        cut = _lib.GS_RANK_CLASS_SPLIT
+        if self.one_class is not None:
+            return (p, None) if self.one_class <= cut else (None, p)
+        held = (p.a_pack, p.b_pack, p.a_off, p.b_off, p.ranks)
+        if self._split is None or any(u is not v for u, v in zip(self._split[0], held)):
+            self._split = (held, p.restricted(1, cut), p.restricted(cut + 1, _lib.GS_MAX_RANK))
+        return self._split[1:]
+
+
 # ---------------------------------------------------------------------------
 # Workspace (split-K partial sums), cached per device
 # ---------------------------------------------------------------------------
@@ -365,11 +427,20 @@ def shrink_workspace(num_tokens: int, hidden: int, num_slices: int, num_adapters
     one stream apart); calls on different streams that may overlap in time
     must not share it.
     """
-    need = int(_lib.load().gs_shrink_workspace_bytes(num_tokens, hidden, num_slices, num_adapters, max_rank,
-                                                     None if ranks_host is None else _i32_array(ranks_host)))
+    return _shrink_workspace(num_tokens, hidden, num_slices, num_adapters, max_rank, device,
+                             _i32_array(ranks_host) if ranks_host else None)
+
+
+def _shrink_workspace(num_tokens, hidden, num_slices, num_adapters, max_rank, device, ranks) -> torch.Tensor:
+    need = int(_lib.load().gs_shrink_workspace_bytes(num_tokens, hidden, num_slices, num_adapters, max_rank, ranks))
     if need < 0:
         raise _lib.GraniteSwitchError("gs_shrink_workspace_bytes", _lib.GS_ERR_INVALID, _lib.last_error())
     return _workspace(device, need)
+
+
+def _pack_workspace(packed: "PackedAdapters", h: "_HostTables", num_tokens: int, device) -> torch.Tensor:
+    return _shrink_workspace(num_tokens, packed.hidden, packed.num_slices, packed.num_adapters, packed.max_rank, device,
+                             h.ranks)
 
 
 def shrink_ksplits(packed: "PackedAdapters", num_tokens: int) -> list:
@@ -465,6 +536,17 @@ def _small_plan(packed: "PackedAdapters", num_tokens: int, num_seqs: int | None,
     if len(_small_plans) >= _SMALL_PLAN_CAP:     # batch sizes vary per step: keep the cache bounded
         _small_plans.clear()
     _small_plans[key] = plan
+    return plan
+
+
+def _cached_small_plan(packed: "PackedAdapters", num_tokens: int, num_seqs: int | None,
+                       largest_group: int | None) -> tuple[bool, int]:
+    """``_small_plan`` of a pack, looked up by the key its host tables keep."""
+    key = (packed._host_tables().plan_key, num_tokens, num_seqs, largest_group)
+    plan = _small_plans.get(key)
+    if plan is None:
+        plan = _small_plan(packed, num_tokens, num_seqs, largest_group)
+        _small_plans[key] = plan                  # bounded: _small_plan clears a full cache
     return plan
 
 
@@ -717,10 +799,11 @@ def shrink(x: torch.Tensor, segments: Segments, packed: PackedAdapters, z: torch
         z = torch.empty(max(T, 1), zw, dtype=x2.dtype, device=x2.device)
     elif z.dtype != x2.dtype or z.stride(-1) != 1 or z.dim() != 2 or z.shape[0] < T or z.shape[1] < zw:
         raise ValueError("z must be a [T, >= S*max_rank] buffer of x's dtype with unit column stride")
-    ws = shrink_workspace(T, H, packed.num_slices, packed.num_adapters, packed.max_rank, x2.device, packed.ranks_host)
+    h = packed._host_tables()
+    ws = _pack_workspace(packed, h, T, x2.device)
     _lib.call("gs_shrink", _dtype_code(x2), x2.data_ptr(), x2.stride(0), T, H, packed.a_pack.data_ptr(),
               packed.a_off.data_ptr(), packed.ranks.data_ptr(), packed.num_slices, packed.num_adapters,
-              packed.max_rank, _i32_array(packed.ranks_host), segments.seg_offsets.data_ptr(),
+              packed.max_rank, h.ranks, segments.seg_offsets.data_ptr(),
               segments.perm.data_ptr(), _lib.ptr(z), zw if z is None else z.stride(0), ws.data_ptr(), ws.numel(),
               _lib.stream_ptr(x2.device))
     return z
@@ -741,20 +824,20 @@ def expand_add_(y: torch.Tensor, z: torch.Tensor, segments: Segments, packed: Pa
     zw = packed.num_slices * packed.max_rank
     if z.dim() != 2 or z.stride(-1) != 1 or z.shape[0] < T or z.shape[1] < zw:
         raise ValueError("z must be a [T, >= S*max_rank] buffer with unit column stride")
-    bounds = _i32_array(packed.slice_bounds)
-    _lib.call("gs_expand_add", _dtype_code(y2), y2.data_ptr(), y2.stride(0), T, O, bounds, packed.num_slices,
+    h = packed._host_tables()
+    _lib.call("gs_expand_add", _dtype_code(y2), y2.data_ptr(), y2.stride(0), T, O, h.bounds, packed.num_slices,
               z.data_ptr(), z.stride(0), 0, None, packed.b_pack.data_ptr(), packed.b_off.data_ptr(),
-              packed.ranks.data_ptr(), packed.num_adapters, packed.max_rank, _i32_array(packed.ranks_host),
+              packed.ranks.data_ptr(), packed.num_adapters, packed.max_rank, h.ranks,
               segments.seg_offsets.data_ptr(), segments.perm.data_ptr(), _lib.stream_ptr(y2.device))
     return y
 
 
 def _xy2(x: torch.Tensor, y: torch.Tensor, packed: PackedAdapters):
     _require_cuda(x, y)
-    x2 = x.reshape(-1, x.shape[-1])
+    x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
     if x2.stride(-1) != 1:
         x2 = x2.contiguous()
-    y2 = y.view(-1, y.shape[-1])
+    y2 = y if y.dim() == 2 else y.view(-1, y.shape[-1])
     if y2.stride(-1) != 1:
         raise ValueError("y must have unit column stride")
     if x2.dtype != packed.dtype or y2.dtype != packed.dtype:
@@ -765,21 +848,23 @@ def _xy2(x: torch.Tensor, y: torch.Tensor, packed: PackedAdapters):
 
 
 def _call_small(x2, y2, packed, eff_ids=None, req=None, pos=None, cu=None, off=None, num_seqs=1, row_split=1):
-    T = x2.shape[0]
-    ws = small_workspace(x2.device, small_workspace_bytes(packed, T))
-    sync = small_sync_buffer(x2.device)
+    T, dev, h = x2.shape[0], x2.device, packed._host_tables()
+    need = h.small_ws.get(T)
+    if need is None:
+        need = h.small_ws[T] = small_workspace_bytes(packed, T)
+    ws = small_workspace(dev, need)
+    sync = small_sync_buffer(dev)
     # issue every adapter's weight loads before the routing is known when most
     # adapters are likely to have tokens
     speculate = int(T >= 2 * packed.num_adapters)
-    i64 = lambda v: (ctypes.c_int64 * len(v))(*[int(u) for u in v])
     _lib.call("gs_switched_lora_small", _dtype_code(x2), _lib.ptr(req), _lib.ptr(pos), _lib.ptr(cu), _lib.ptr(off),
               int(num_seqs), _lib.ptr(eff_ids), x2.data_ptr(), x2.stride(0), y2.data_ptr(), y2.stride(0), T,
-              packed.hidden, packed.out_total, _i32_array(packed.slice_bounds), packed.num_slices,
-              packed.a_pack.data_ptr(), i64(packed.a_off_host), packed.b_pack.data_ptr(), i64(packed.b_off_host),
-              _i32_array(packed.ranks_host), packed.num_adapters, packed.max_rank, ws.data_ptr(), ws.numel(),
-              sync.data_ptr(), sync.numel() * 4, int(row_split), speculate, _lib.stream_ptr(x2.device))
+              packed.hidden, h.bounds_list[-1], h.bounds, packed.num_slices,
+              packed.a_pack.data_ptr(), h.a_off, packed.b_pack.data_ptr(), h.b_off,
+              h.ranks, packed.num_adapters, packed.max_rank, ws.data_ptr(), ws.numel(),
+              sync.data_ptr(), sync.numel() * 4, int(row_split), speculate, _lib.stream_ptr(dev))
     if _CHECK_EACH_CALL and not torch.cuda.is_current_stream_capturing():
-        check(x2.device)
+        check(dev)
 
 
 def pair_launches(packed: PackedAdapters, num_tokens: int) -> bool:
@@ -803,12 +888,21 @@ def path_plan(packed: PackedAdapters, num_tokens: int, num_seqs: int | None = No
     they run its two classes in the pair launches (decode QKV with one
     rank-512 adapter among twelve rank-32 ones: 33.6 us against 39.5 us for
     "split")."""
-    small_v, large_v = packed.rank_split()
-    if small_v is None or not num_tokens or not small_preferred(small_v, num_tokens, num_seqs, largest_group):
-        return "segments"
+    return _path_plan(packed, packed.rank_split(), num_tokens, num_seqs, largest_group)[0]
+
+
+def _path_plan(packed: PackedAdapters, views: tuple, num_tokens: int, num_seqs: int | None,
+               largest_group: int | None) -> tuple[str, int]:
+    """(``path_plan``, the row split of the one-launch kernel) with the pack's ``rank_split`` at hand."""
+    small_v, large_v = views
+    if small_v is None or not num_tokens:
+        return "segments", 1
+    prefer, row_split = _cached_small_plan(small_v, num_tokens, num_seqs, largest_group)
+    if not prefer:
+        return "segments", 1
     if large_v is None:
-        return "small"
-    return "segments" if pair_launches(packed, num_tokens) else "split"
+        return "small", row_split
+    return ("segments" if pair_launches(packed, num_tokens) else "split"), row_split
 
 
 def switched_lora_routed_(y: torch.Tensor, x: torch.Tensor, adapter_ids: torch.Tensor, packed: PackedAdapters,
@@ -831,7 +925,7 @@ def switched_lora_routed_(y: torch.Tensor, x: torch.Tensor, adapter_ids: torch.T
         raise ValueError(f"unknown path {path!r}")
     x2, y2 = _xy2(x, y, packed)
     dev = x2.device
-    ids = _as_i64(adapter_ids.reshape(-1), dev)
+    ids = _as_i64(adapter_ids if adapter_ids.dim() == 1 else adapter_ids.reshape(-1), dev)
     T = ids.shape[0]
     if T != x2.shape[0]:
         raise ValueError("adapter_ids must have one entry per token")
@@ -844,16 +938,20 @@ def switched_lora_routed_(y: torch.Tensor, x: torch.Tensor, adapter_ids: torch.T
     if off is not None and off.numel() != num_seqs:
         raise ValueError("act_offsets must have one entry per sequence")
     nseq_hint = num_seqs if cu is not None else None
-    small_v, large_v = packed.rank_split()
+    small_v, large_v = views = packed.rank_split() if path != "segments" else (None, None)
     if path == "small" and small_v is None:
         raise ValueError("the one-launch kernel takes adapters of rank <= 64; this module has none")
-    if path == "small" or (path == "auto" and path_plan(packed, T, nseq_hint, largest_group) != "segments"):
+    plan, row_split = "segments", 1
+    if path == "small":
         if not small_eligible(small_v, T, num_seqs):
             raise ValueError("this module / batch is outside the small-batch kernel's limits")
+        plan, row_split = "small", small_row_split(small_v, T, nseq_hint, largest_group)
+    elif path == "auto":
+        plan, row_split = _path_plan(packed, views, T, nseq_hint, largest_group)   # eligible, when not "segments"
+    if plan != "segments":
         def small():
             _call_small(x2, y2, small_v, req=ids, pos=pos, cu=cu if off is not None else None, off=off,
-                        num_seqs=num_seqs if off is not None else 1,
-                        row_split=small_row_split(small_v, T, nseq_hint, largest_group))
+                        num_seqs=num_seqs if off is not None else 1, row_split=row_split)
 
         if large_v is None:
             small()
@@ -893,13 +991,14 @@ def switched_lora_(y: torch.Tensor, x: torch.Tensor, segments: Segments, packed:
         raise ValueError("x / y shapes do not match the segments")
     _check_segments(segments, packed)
     if path != "segments" and T:
-        small_v, large_v = packed.rank_split()
+        small_v, large_v = views = packed.rank_split()
         if path == "small" and small_v is None:
             raise ValueError("the one-launch kernel takes adapters of rank <= 64; this module has none")
-        if path == "small" or path_plan(packed, T, None, largest_group) != "segments":
+        plan, row_split = (("small", small_row_split(small_v, T, None, largest_group)) if path == "small"
+                           else _path_plan(packed, views, T, None, largest_group))
+        if plan != "segments":
             def small():
-                _call_small(x2, y2, small_v, eff_ids=segments.eff_ids,
-                            row_split=small_row_split(small_v, T, None, largest_group))
+                _call_small(x2, y2, small_v, eff_ids=segments.eff_ids, row_split=row_split)
 
             if large_v is None:
                 small()
@@ -908,14 +1007,15 @@ def switched_lora_(y: torch.Tensor, x: torch.Tensor, segments: Segments, packed:
             return y
     zw = packed.num_slices * packed.max_rank
     if z is None:
-        z = torch.empty(max(T, 1), packed.num_slices * packed.max_rank, dtype=x2.dtype, device=x2.device)
+        z = torch.empty(max(T, 1), zw, dtype=x2.dtype, device=x2.device)
     elif z.stride(-1) != 1 or z.shape[-1] < zw or (T and z.stride(0) != zw):
         raise ValueError("z must be a contiguous [T, S*max_rank] buffer")
-    ws = shrink_workspace(T, H, packed.num_slices, packed.num_adapters, packed.max_rank, x2.device, packed.ranks_host)
+    h = packed._host_tables()
+    ws = _pack_workspace(packed, h, T, x2.device)
     _lib.call("gs_switched_lora", _dtype_code(x2), x2.data_ptr(), x2.stride(0), y2.data_ptr(), y2.stride(0), T, H,
-              packed.out_total, _i32_array(packed.slice_bounds), packed.num_slices, packed.a_pack.data_ptr(),
+              h.bounds_list[-1], h.bounds, packed.num_slices, packed.a_pack.data_ptr(),
               packed.a_off.data_ptr(), packed.b_pack.data_ptr(), packed.b_off.data_ptr(), packed.ranks.data_ptr(),
-              packed.num_adapters, packed.max_rank, _i32_array(packed.ranks_host), segments.seg_offsets.data_ptr(),
+              packed.num_adapters, packed.max_rank, h.ranks, segments.seg_offsets.data_ptr(),
               segments.perm.data_ptr(), z.data_ptr(), ws.data_ptr(), ws.numel(), _lib.stream_ptr(x2.device))
     return y
 
@@ -946,10 +1046,11 @@ def switched_lora_noalloc_(y: torch.Tensor, x: torch.Tensor, segments: Segments,
     if T != segments.num_tokens:
         raise ValueError("x / y shapes do not match the segments")
     _check_segments(segments, packed)
+    h = packed._host_tables()
     _lib.call("gs_switched_lora_noalloc", _dtype_code(x2), x2.data_ptr(), x2.stride(0), y2.data_ptr(), y2.stride(0),
-              T, packed.hidden, packed.out_total, _i32_array(packed.slice_bounds), packed.num_slices,
+              T, packed.hidden, h.bounds_list[-1], h.bounds, packed.num_slices,
               packed.a_pack.data_ptr(), packed.a_off.data_ptr(), packed.b_pack.data_ptr(), packed.b_off.data_ptr(),
-              packed.ranks.data_ptr(), packed.num_adapters, packed.max_rank, _i32_array(packed.ranks_host),
+              packed.ranks.data_ptr(), packed.num_adapters, packed.max_rank, h.ranks,
               segments.seg_offsets.data_ptr(), segments.perm.data_ptr(), _lib.stream_ptr(x2.device))
     return y
 
@@ -966,6 +1067,10 @@ def _check_segments(segments: Segments, packed: PackedAdapters) -> None:
 def _i32_array(vals):
     """Host int32 array for the C ABI's host-side table arguments."""
     return (ctypes.c_int32 * len(vals))(*[int(v) for v in vals])
+
+
+def _i64_array(vals):
+    return (ctypes.c_int64 * len(vals))(*[int(v) for v in vals])
 
 
 def linear_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:

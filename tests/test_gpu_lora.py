@@ -148,6 +148,23 @@ def test_shrink_matches_oracle(dev):
         _close(got[lo:hi, :rr], olora.bf16_round(ref[lo:hi, :rr]), 2e-2, f"z adapter {g}")
 
 
+def test_shrink_and_expand_ops_without_host_ranks(dev):
+    """The torch ops have no host rank table: one class up to max_rank, the same values."""
+    from granite_switch_amd import ops
+
+    T, NA = 300, 20
+    spec = workloads.ModuleSpec("ops", 512, (256, 128), [8, 16, 32, 24] * 5, 32)
+    md = workloads.make_module(spec, T, NA, torch.bfloat16, dev, seed=21)
+    ids = torch.randint(0, NA + 1, (T,), device=dev)
+    segs = switched.build_segments(ids, NA)
+    pk = switched.PackedAdapters.from_slices(md.lora_A_slices, md.lora_B_slices, spec.ranks)
+    z = ops.op("switched_lora_shrink")(md.x, segs.seg_offsets, segs.perm, pk.a_pack, pk.a_off, pk.ranks, 2, 32)
+    y = md.y.clone()
+    ops.op("switched_lora_expand_add")(y, z, segs.seg_offsets, segs.perm, pk.b_pack, pk.b_off, pk.ranks,
+                                       pk.slice_bounds, 32)
+    _check_module(md, y, ids.cpu().numpy(), slice(0, T), torch.bfloat16, hf_too=False)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_identity_known_answer(dev, dtype):
     """A_a = eye*0.1(a+1), B_a = eye*0.2(a+1) -> delta[:, j<r] = x[:, j] * 0.02(a+1)^2 (lora_cases.py:346-426)."""

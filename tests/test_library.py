@@ -313,6 +313,40 @@ def test_workload_module_on_cpu():
     assert md.lora_B_slices[0][1, 0].std().item() < 0.05
 
 
+def test_host_tables_follow_the_pack():
+    """The tables kept with a pack are made again after any field they follow
+    from changes, in place or by assignment; the class views after a device
+    tensor is replaced."""
+    import copy
+    import pickle
+
+    A = [torch.ones(3, 1, 128, 16)]
+    B = [torch.ones(3, 1, 32, 128)]
+    pk = switched.PackedAdapters.from_slices(A, B, [16, 128, 64])
+    h = pk._host_tables()
+    assert pk._host_tables() is h and list(h.ranks) == pk.ranks_host and list(h.bounds) == [0, 32]
+    small, large = pk.rank_split()
+    assert pk.rank_split()[0] is small and small.ranks_host == [0, 16, 0, 64] and large.ranks_host == [0, 0, 128, 0]
+    pk.ranks_host[1] = 8
+    assert list(pk._host_tables().ranks) == [0, 8, 128, 64] and pk.rank_split()[0].ranks_host == [0, 8, 0, 64]
+    pk.b_pack = pk.b_pack.clone()
+    assert pk.rank_split()[0].b_pack is pk.b_pack and pk.rank_split()[1].b_pack is pk.b_pack
+    for twin in (copy.deepcopy(pk), pickle.loads(pickle.dumps(pk))):
+        assert "_host" not in vars(twin) and list(twin._host_tables().ranks) == pk.ranks_host
+    pk.b_off_host[3] += 1
+    assert list(pk._host_tables().b_off) == pk.b_off_host
+    pk.output_slices = (16, 16)
+    assert list(pk._host_tables().bounds) == [0, 16, 32]
+    one = switched.PackedAdapters.from_slices(A, B, [16, 8, 64])
+    assert one.rank_split() == (one, None) and one.rank_split()[0] is one
+    wide = switched.PackedAdapters.from_slices(A, B, [128, 72, 0])
+    assert wide.rank_split()[0] is None and wide.rank_split()[1] is wide
+    one.max_rank = 128                       # wider than its ranks: the views carry their own largest rank
+    assert one.rank_split()[0].max_rank == 64 and one.rank_split()[1] is None
+    one.ranks_host = []
+    assert one._host_tables().ranks is None and one.rank_split() == (None, None)
+
+
 def _packed_stub(H, slices, NA, max_rank, dtype=torch.bfloat16):
     """The attributes the small-path plan reads, without device memory."""
     from types import SimpleNamespace
