@@ -97,6 +97,9 @@ GS_HD int k_or_zero(int k0, int r) { return k0 < r ? k0 : 0; }
 GS_HD int stage_row(int it, int per_row) { return it / per_row; }
 GS_HD int stage_col(int it, int row, int per_row, int col_base) { return col_base + (it - row * per_row) * 4; }
 
+// Workgroups of `threads` that sum a tile's partials (tm rows of cols values), 4 values a thread.
+GS_HD int sum_wgs_per_tile(int tm, int cols, int threads) { return (tm * (cols >> 2) + threads - 1) / threads; }
+
 // ---- reference-semantics ops over x_ext (gs_xext.hip) ----------------------
 // Tier of kernel-local id kid (ids are numbered 1.. across the six tiers in
 // ascending-rank order; tier t holds na[t] adapters of rank 16 << t): its

@@ -287,8 +287,14 @@ __device__ __forceinline__ void wait_stages(int after) {
   }
 }
 
+// A 4-element bf16 piece of z that no workgroup has summed yet (NaNs; a piece
+// that truly sums to these bits is summed again by its reader).
+constexpr uint64_t kUnsummed = ~uint64_t(0);
+
 // One work item of shrink_dma_kernel: tile tr, sub = (k-chunk, column chunk).
-template <int NB>
+// MARK: the launch's expand sums the split-K partials into z (sum_partials);
+// the first k-chunk's workgroups mark its pieces as not yet summed.
+template <int NB, bool MARK = false>
 __device__ __forceinline__ void shrink_dma_item(const ShrinkParams& p, const TileRef& tr, int sub, int KS,
                                                 char* ring) {
   constexpr int COLS = 32 * NB;
@@ -398,6 +404,8 @@ __device__ __forceinline__ void shrink_dma_item(const ShrinkParams& p, const Til
           make_uint2(pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w));
     } else {
       *reinterpret_cast<f32x4*>(p.part + static_cast<int64_t>(ks) * p.part_stride + slot * p.zw + col0 + c4) = v;
+      if (MARK && ks == 0 && p.z != nullptr)
+        *reinterpret_cast<uint64_t*>(static_cast<uint16_t*>(p.z) + slot * p.ldz + col0 + c4) = kUnsummed;
     }
   }
 }
@@ -534,6 +542,7 @@ struct ExpandParams {
   int flat;               // flat item layout, one sub-tile per item (work_item)
   int ks_target;          // > 0: the shrink chose its k-split on the device (dyn_ksplit over
   int ks_chunks;          //   its 64-slot tiles, ks_chunks column chunks, at most nparts)
+  int sum_wgs;            // pair expand: workgroups that first sum split-K partials into z (sum_partials)
 };
 
 // Shrink values of the tile for slices s_lo..s_hi (the ones the workgroup's
@@ -903,7 +912,8 @@ constexpr int kSpNT = 128;                   // columns per item of expand_spars
 // columns (inside one slice).  red: the waves' partial deltas.  Each output
 // element is the same sum in the same order whatever QB: wave w's k-groups
 // [w*KG, (w+1)*KG) in order, then (w0 + w2) + (w1 + w3).
-template <int KG, int QB>
+// SUMMED: split-K partials may be summed in z already (sum_partials).
+template <int KG, int QB, bool SUMMED = false>
 __device__ __forceinline__ void expand_sparse_item(const ExpandParams& p, const TileRef& tr, int sub, int nparts,
                                                    float (&red)[2][kTM][32 * QB + kOutPad], char* zs) {
   constexpr int NTC = 32 * QB;               // columns per item
@@ -954,7 +964,7 @@ __device__ __forceinline__ void expand_sparse_item(const ExpandParams& p, const 
     // (pieces past the rank read the row's first piece and are masked) and
     // the y pieces
     uint2 w[ZIT];
-    if (nparts == 0) {
+    if (!SUMMED && nparts == 0) {   // uniform
       const uint16_t* zp = static_cast<const uint16_t*>(p.z) + zo + s * r;
 #pragma unroll
       for (int j = 0; j < ZIT; ++j) {
@@ -977,10 +987,37 @@ __device__ __forceinline__ void expand_sparse_item(const ExpandParams& p, const 
     u32x4 yv[PASSES];
 #pragma unroll
     for (int ps = 0; ps < PASSES; ++ps) yv[ps] = ld16(static_cast<const char*>(p.y) + (yrow[ps] + n_tile0 + cx) * 2);
+    uint32_t unsummed = ~0u;               // pieces j of this thread whose partials it sums itself
+    if constexpr (SUMMED) {
+      // the summed pieces (or z, when the shrink was not split), the youngest
+      // loads: the sums have had the longest time.  Agent scope: another XCD
+      // may have stored them in this launch.  zo is 0: the pair's z is by slot
+      if (nparts == 0 || p.sum_wgs > 0) {   // uniform
+        const uint16_t* zp = static_cast<const uint16_t*>(p.z) + s * r;
+        uint64_t zv[ZIT];
+#pragma unroll
+        for (int j = 0; j < ZIT; ++j) {
+          const int it = tid + j * kThreads;
+          const int c4 = it < kTM * per_row ? addr::stage_col(it, addr::stage_row(it, per_row), per_row, 0) : 0;
+          zv[j] = __hip_atomic_load(
+              reinterpret_cast<uint64_t*>(const_cast<uint16_t*>(zp) + static_cast<int64_t>(zrow[j]) * p.ldz + c4),
+              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+#pragma unroll
+        for (int j = 0; j < ZIT; ++j) {
+          const int it = tid + j * kThreads;
+          const int row = addr::stage_row(it, per_row);
+          if (zv[j] != kUnsummed) unsummed &= ~(1u << j);
+          if (it < kTM * per_row)
+            *reinterpret_cast<uint64_t*>(zs + (static_cast<int64_t>(row) * zs_ld +
+                                               addr::stage_col(it, row, per_row, 0)) * 2) = zv[j];
+        }
+      }
+    }
     // the slice's shrink values of the tile's rows in LDS: the z pieces
     // loaded above, or split-K partials summed in ks order (kPartGroup at a
     // time) and rounded to bf16 as a stored z would be
-    if (nparts == 0) {
+    if (!SUMMED && nparts == 0) {
 #pragma unroll
       for (int j = 0; j < ZIT; ++j) {
         const int it = tid + j * kThreads;
@@ -1000,6 +1037,10 @@ __device__ __forceinline__ void expand_sparse_item(const ExpandParams& p, const 
     constexpr int UNR = KG >= 8 && QB == 4 ? 2 : 1;
     const int npieces = nparts == 0 ? 0 : tr.nrows * per_row;
     for (int it0 = tid; it0 < npieces; it0 += UNR * kThreads) {
+      if constexpr (SUMMED) {
+        static_assert(UNR == 1 && ZIT <= 32, "a piece of a thread is one bit of its mask");
+        if (!(unsummed >> ((it0 - tid) / kThreads) & 1u)) continue;
+      }
       float v[UNR][4];
       const float* src[UNR];
 #pragma unroll
@@ -1086,6 +1127,54 @@ __device__ __forceinline__ int sparse_nparts(const ExpandParams& p) {
   return ks > 1 ? ks : 0;
 }
 
+// The first p.sum_wgs workgroups of a pair expand sum the large class's
+// split-K partials into z, 1 KB pieces a workgroup, before their own items:
+// every item of the class (one per 64 columns) reads the same sums, and each
+// used to add up to 16 partials of its 32 x r values for itself.  Nobody
+// waits: a reader takes the pieces that are there and sums the ones still
+// marked kUnsummed as before, in the same order, so the bits are the same
+// either way.  Pieces are 8 bytes, stored and loaded whole at agent scope.
+// Pair expand of 256 tokens, 12 rank-32 adapters and one of rank 512: 4096 ->
+// 4096 20.5 -> 13.2 us, 4096 -> 6144 18.6 -> 13.7, 4096 -> 25600 30.0 -> 24.6.
+// A deeper k-split, which the cheaper sums would allow, lost in the shrink
+// what it gained (4096 -> 6144: 13.6 -> 17.6 us).
+__device__ __forceinline__ void sum_partials(const ExpandParams& p) {
+  const int u = static_cast<int>(blockIdx.x);
+  if (u >= p.sum_wgs) return;
+  const int nparts = sparse_nparts(p);
+  if (nparts == 0) return;
+  const int wpt = addr::sum_wgs_per_tile(kTM, p.si.S * p.max_rank, kThreads);
+  const TileRef tr = find_tile<kTM, kExpandBalanced>(p.seg, p.ranks, p.b_off, p.NA, p.rw, u / wpt);
+  if (tr.g == 0) return;
+  const int per_row = (p.si.S * tr.rank) >> 2;
+  const int it = (u % wpt) * kThreads + static_cast<int>(threadIdx.x);
+  const int row = addr::stage_row(it, per_row);
+  if (row >= tr.nrows) return;
+  const int c4 = addr::stage_col(it, row, per_row, 0);
+  const int64_t slot = tr.slot0 + row;
+  const float* src = p.part + slot * p.zw + c4;
+  float v[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int ks0 = 0; ks0 < nparts; ks0 += kPartGroup) {
+    f32x4 a[kPartGroup];
+#pragma unroll
+    for (int k = 0; k < kPartGroup; ++k)
+      if (ks0 + k < nparts) a[k] = *reinterpret_cast<const f32x4*>(src + (ks0 + k) * p.part_stride);
+#pragma unroll
+    for (int k = 0; k < kPartGroup; ++k)
+      if (ks0 + k < nparts) {
+        v[0] += a[k].x;
+        v[1] += a[k].y;
+        v[2] += a[k].z;
+        v[3] += a[k].w;
+      }
+  }
+  const uint64_t sum = static_cast<uint64_t>(pack_bf16x2(v[0], v[1])) |
+                       (static_cast<uint64_t>(pack_bf16x2(v[2], v[3])) << 32);
+  __hip_atomic_store(reinterpret_cast<uint64_t*>(const_cast<uint16_t*>(static_cast<const uint16_t*>(p.z)) +
+                                                 slot * p.ldz + c4),
+                     sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 template <int KG>
 __global__ __launch_bounds__(kThreads) void expand_sparse_kernel(ExpandParams p) {
   __shared__ float red[2][kTM][kSpNT + kOutPad];
@@ -1119,7 +1208,8 @@ __global__ __launch_bounds__(kThreads) void expand_sparse_kernel(ExpandParams p)
 //   expand_pair_kernel: workgroup b expands its small-class item, then takes
 //     large-class items (64-column sub-tiles of the rank-split form) from that
 //     counter until none are left, so the workgroups that finish first take
-//     them and they fill the launch's end.
+//     them and they fill the launch's end.  Its first workgroups sum the
+//     large class's split-K partials for all of them (sum_partials).
 // Every output element is computed as by the separate launches (the same
 // item functions, the same sums in the same order).
 // ----------------------------------------------------------------------------
@@ -1159,7 +1249,7 @@ __global__ __launch_bounds__(kThreads) void shrink_dma_pair_kernel(ShrinkParams 
   const int items = work_items(total, p1.n_chunks * KS, true);
   while (lin < items) {
     lds_barrier();                         // every wave is done with the ring before the item's transfers
-    if (tr.g != 0) shrink_dma_item<1>(p1, tr, sub, KS, ring);
+    if (tr.g != 0) shrink_dma_item<1, true>(p1, tr, sub, KS, ring);
     lin += static_cast<int>(gridDim.x);
     if (lin >= items) break;
     tr = tile_at<kTMS>(p1.seg, p1.ranks, p1.a_off, p1.NA, p1.rw, lin, true, total, p1.n_chunks * KS, sub);
@@ -1167,7 +1257,7 @@ __global__ __launch_bounds__(kThreads) void shrink_dma_pair_kernel(ShrinkParams 
 }
 
 template <int NBW, int PRE, int KG>
-__global__ __launch_bounds__(kThreads) void expand_pair_kernel(ExpandParams p0, ExpandParams p1, int* claim) {
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void expand_pair_kernel(ExpandParams p0, ExpandParams p1, int* claim) {
   constexpr int NT = 4 * NBW * 32;
   constexpr int kD = static_cast<int>(sizeof(float)) * kTM * (NT + kOutPad);
   constexpr int kR = static_cast<int>(sizeof(float)) * 2 * kTM * (32 * kPairQB + kOutPad);
@@ -1176,6 +1266,7 @@ __global__ __launch_bounds__(kThreads) void expand_pair_kernel(ExpandParams p0, 
   extern __shared__ __align__(16) char zs[];   // either class's shrink values
   auto& dtile = *reinterpret_cast<float(*)[kTM][NT + kOutPad]>(buf);
   auto& red = *reinterpret_cast<float(*)[2][kTM][32 * kPairQB + kOutPad]>(buf);
+  sum_partials(p1);
   int ticket = 0;
   bool early = false;                      // uniform: the small items ran and claimed
   // the first claim goes out before the small class's last sub-tile, so its
@@ -1196,7 +1287,7 @@ __global__ __launch_bounds__(kThreads) void expand_pair_kernel(ExpandParams p0, 
   while (it < items1) {
     int sub = 0;
     const TileRef tr = tile_at<kTM, kExpandBalanced>(p1.seg, p1.ranks, p1.b_off, p1.NA, p1.rw, it, true, total1, n_sub1, sub);
-    if (tr.g != 0) expand_sparse_item<KG, kPairQB>(p1, tr, sub, nparts1, red, zs);
+    if (tr.g != 0) expand_sparse_item<KG, kPairQB, true>(p1, tr, sub, nparts1, red, zs);
     lds_barrier();                         // zs, buf and `claimed` are free
     if (threadIdx.x == 0) claimed = claim_next(claim);
     lds_barrier();
@@ -1232,7 +1323,8 @@ struct ShrinkPlan {
 // workgroup target: its expand stages the split-K partials of every row for
 // each 128-column item, so fewer, longer k-chunks measured faster overall
 // (with one rank-512 adapter: decode QKV 46.0 us at the full target, 40.7 at
-// half, 40.2 at a quarter; decoder step 8.87 / 8.85 / 8.90 ms).
+// half, 40.2 at a quarter; decoder step 8.87 / 8.85 / 8.90 ms; with the pair
+// expand summing them once the full target still loses, sum_partials).
 #ifndef GS_SPARSE_KS_DIV
 #define GS_SPARSE_KS_DIV 2
 #endif
@@ -1704,6 +1796,15 @@ int64_t pair_expand_grid(const PairForm& f, int64_t T, int adapters0, size_t lds
   return expand_grid(wt, max_tiles_for(T, adapters0), (e0.out_total + NT - 1) / NT);
 }
 
+// Workgroups that sum the large class's partials (sum_partials): for the tiles
+// it is expected to hold, a part-filled one among them; the items of any
+// further tile sum for themselves.  0 without a z to sum into.
+int pair_sum_wgs(const ExpandParams& e1, const RankClass& k, int64_t grid) {
+  if (e1.z == nullptr || e1.nparts == 0) return 0;
+  const int64_t tiles = (k.est_tokens + kTM - 1) / kTM + std::min<int64_t>(k.adapters, k.est_tokens);
+  return static_cast<int>(std::min(grid, tiles * addr::sum_wgs_per_tile(kTM, e1.si.S * e1.max_rank, kThreads)));
+}
+
 void launch_shrink_pair(const PairForm& f, int64_t grid, const ShrinkParams& p0, const ShrinkParams& p1, int* claim,
                         hipStream_t st) {
   const dim3 g(static_cast<unsigned>(grid));
@@ -1964,6 +2065,38 @@ struct AddrModel {
     }
   }
 
+  // ---- sum_partials (pair expand) and the marks its shrink leaves in z -------
+  void sums(const ExpandParams& e, int64_t z_elems, int64_t part_elems) {
+    const std::vector<TileRef> tl = tiles<kTM, kExpandBalanced>(e.rw, b_off);
+    const int ks = e.ks_target > 0 ? dyn_ksplit(static_cast<int>(tiles<kTMS, false>(e.rw, a_off).size()), e.ks_chunks,
+                                                e.ks_target, e.nparts)
+                                   : e.nparts;
+    if (ks <= 1) return;
+    for (const TileRef& tr : tl) {
+      in("pair mark column", static_cast<int64_t>(si.S) * tr.rank - 1, 1, e.ldz);
+      in("pair mark", (tr.slot0 + tr.nrows - 1) * e.ldz + static_cast<int64_t>(si.S) * tr.rank - 1, 1, z_elems);
+    }
+    const int wpt = addr::sum_wgs_per_tile(kTM, si.S * e.max_rank, kThreads);
+    for (int u = 0; u < e.sum_wgs; ++u) {
+      if (u / wpt >= static_cast<int>(tl.size())) break;
+      const TileRef& tr = tl[u / wpt];
+      const int per_row = (si.S * tr.rank) >> 2;
+      for (int tid = 0; tid < kThreads; ++tid) {
+        const int it = (u % wpt) * kThreads + tid, row = addr::stage_row(it, per_row);
+        if (row >= tr.nrows) continue;
+        const int c4 = addr::stage_col(it, row, per_row, 0);
+        const int64_t slot = tr.slot0 + row;
+        for (int k = 0; k < ks; ++k) in("pair partials", k * e.part_stride + slot * e.zw + c4, 4, part_elems);
+        in("pair sum column", c4, 4, e.ldz);
+        in("pair sum", slot * e.ldz + c4, 4, z_elems);
+      }
+    }
+    // with as many workgroups as a tile needs, all of its values are summed
+    for (const TileRef& tr : tl)
+      if (static_cast<int64_t>(wpt) * kThreads < static_cast<int64_t>(tr.nrows) * ((si.S * tr.rank) >> 2))
+        fail("sum_partials: %d workgroups leave values of a tile of %d rows", wpt, tr.nrows);
+  }
+
   // ---- expand_kernel and expand_sparse_kernel --------------------------------
   // z source: partials [nparts][T][zw] (nparts > 0), else z [z_rows, ldz]
   // by slot or by token (z_by_token), columns from z_off[g].
@@ -2038,9 +2171,8 @@ struct AddrModel {
             const int tok = token_at(tr.slot0 + addr::tile_row(row, tr.nrows));
             row_piece("sparse y", tok, n_tile0 + cx, 8, out_total);
           }
-        if (nparts > 0) {
-          stage(tr, s, s, 0, zs_ld, lds, nparts);
-        } else {
+        if (nparts > 0) stage(tr, s, s, 0, zs_ld, lds, nparts);
+        if (nparts == 0 || (claimed && e.sum_wgs > 0)) {
           // every piece of the 2 KG per thread loaded (rows past the tile
           // and pieces past the rank read clamped addresses), then stored
           const int per_row = r >> 2, ZIT = 2 * f.KG, zo = z_off ? z_off[tr.g] : 0;
@@ -2327,13 +2459,14 @@ int switched_lora_impl(const char* who, int32_t dtype, const void* x, int64_t ld
     const ShrinkPlan pl1 = plan_class(num_tokens, hidden, num_slices, cls[1], bf16, max_part_bytes);
     const ShrinkParams sp0 = shrink_params(cls[0], pl0, L.off[0], ldz);
     const ShrinkParams sp1 = shrink_params(cls[1], pl1, L.off[1], ldz);
-    ExpandParams e0 = expand_params(cls[0], pl0, sp0, ldz);
-    const ExpandParams e1 = expand_params(cls[1], pl1, sp1, ldz);
+    const ExpandParams e0 = expand_params(cls[0], pl0, sp0, ldz);
+    ExpandParams e1 = expand_params(cls[1], pl1, sp1, ldz);
     const PairForm f = pair_form(bf16, num_tokens, pl0, pl1, e0, e1);
     if (f.ok) {
       int* claim = reinterpret_cast<int*>(static_cast<char*>(workspace) + L.claim);
       const size_t lds = pair_lds_bytes(num_slices, cls[0].max_rank, cls[1].max_rank);
       const int64_t egrid = pair_expand_grid(f, num_tokens, cls[0].adapters, lds, e0);
+      e1.sum_wgs = pair_sum_wgs(e1, cls[1], egrid);
       launch_shrink_pair(f, pl0.grid, sp0, sp1, claim, st);
       GS_CHECK_LAUNCH(who);
       launch_expand_pair(f, egrid, lds, e0, e1, claim, st);
@@ -2624,7 +2757,7 @@ int64_t gs_check_segment_addresses(int32_t dtype, int64_t num_tokens, int32_t hi
         const ShrinkPlan pl0 = plan_class(T, hidden, num_slices, cls[0], bf16, budget);
         const ShrinkPlan pl1 = plan_class(T, hidden, num_slices, cls[1], bf16, budget);
         const ExpandParams e0 = class_expand_plan(m.si, out_total, cls[0], pl0, T, zl);
-        const ExpandParams e1 = class_expand_plan(m.si, out_total, cls[1], pl1, T, zl);
+        ExpandParams e1 = class_expand_plan(m.si, out_total, cls[1], pl1, T, zl);
         const PairForm pf = pair_form(bf16, T, pl0, pl1, e0, e1);
         if (pf.ok) {
           m.in("pair item counter", L.claim / 4, 1, ws_elems);
@@ -2634,6 +2767,9 @@ int64_t gs_check_segment_addresses(int32_t dtype, int64_t num_tokens, int32_t hi
           for (int occ = 1; occ <= 4; ++occ)
             m.expand(e0, pf.f0, cls[0].adapters, int64_t(occ) * cus, z_elems, part0, nullptr);
           const ExpandForm f1{true, 1, 2, pf.KG1};
+          e1.z = &m;           // a call's z (only its presence is read)
+          e1.sum_wgs = pair_sum_wgs(e1, cls[1], INT64_MAX);
+          m.sums(e1, z_elems, part1);
           m.expand(e1, f1, cls[1].adapters, cus, z_elems, part1, nullptr, kPairQB, true);
           continue;
         }

@@ -251,7 +251,8 @@ int gs_expand_add(int32_t dtype, void* y, int64_t ldy, int64_t num_tokens, int32
  * A module of two rank classes with a workspace of gs_shrink_workspace_bytes:
  *   - bf16 with a sparse large class (e.g. one rank-512 adapter among rank-32
  *     ones): both classes in the same two launches, the small class's
- *     workgroups taking the large class's items once their own are done;
+ *     workgroups taking the large class's items once their own are done (z
+ *     holds the large class's summed partials, when given);
  *   - otherwise, when `stream` belongs to the current device: the large class
  *     on the library's side stream of the current device (default priority,
  *     created on the first such call: make it eagerly, outside graph capture),

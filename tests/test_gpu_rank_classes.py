@@ -397,3 +397,40 @@ def test_step_population_with_a_rank512_adapter(dev, proj):
     torch.cuda.synchronize()
     err = _check(md, y, eff, torch.bfloat16, f"step r512 {spec.name}")
     _say(f"  max abs err {err:.3e}")
+
+
+@pytest.mark.parametrize("slices,on_large", [((2048, 1024, 1024), 300), ((4096,), 33), ((256, 256), 1)])
+def test_pair_sums_beyond_the_expected_tiles_and_nan(dev, slices, on_large):
+    """The pair expand sums the large class's partials once for the tiles it is
+    expected to hold; the items of further tiles (300 tokens where ~24 are
+    expected), and pieces whose sum has the bits of the not-yet-summed mark
+    (NaN), sum for themselves: the same bits as the classes in turn, also on
+    replays of a graph over the same scratch."""
+    ranks = [32] * 24 + [512]
+    NA, T = len(ranks), 600
+    spec = workloads.ModuleSpec("m", 4096, slices, ranks, 512)
+    md = workloads.make_module(spec, T, NA, torch.bfloat16, dev, seed=on_large)
+    pk = switched.PackedAdapters.from_slices(md.lora_A_slices, md.lora_B_slices, ranks)
+    assert switched.pair_launches(pk, T)
+    rng = np.random.default_rng(on_large)
+    req = rng.integers(0, NA, size=T)
+    at = rng.permutation(T)[:on_large]
+    req[at] = NA
+    md.x[int(at[0]), 5] = float("nan")
+    md.x.view(torch.int16)[int(at[-1]), 7] = -1            # NaN, all bits set
+    segs = switched.build_segments(torch.tensor(req, device=dev), NA)
+    full = int(switched._lib.load().gs_shrink_workspace_bytes(T, 4096, pk.num_slices, NA, 512,
+                                                              switched._i32_array(pk.ranks_host)))
+    pair = _run_with_workspace(md, pk, segs, T, spec, full)
+    turn = _run_with_workspace(md, pk, segs, T, spec, full - 512)
+    assert torch.equal(pair.view(torch.int16), turn.view(torch.int16))
+    y = md.y.clone()
+    switched.switched_lora_(y, md.x, segs, pk, path="segments")          # workspaces before the capture
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        switched.switched_lora_(y, md.x, segs, pk, path="segments")
+    for replay in range(3):
+        y.copy_(md.y)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int16), turn.view(torch.int16)), replay
