@@ -175,21 +175,22 @@ GS_HD bool gemm_tile(int bid, int tiles_m, int tiles_n, int group, int& tm, int&
   tn = rr / gm;
   return true;
 }
-// As gemm_tile, where the last tile row is thin (at most half its rows exist)
-// and its tiles cost half as much: they come after the others in every XCD's
-// range, shared out evenly, so that the XCDs end together.
-GS_HD int64_t gemm_thin_grid(int tiles_m, int tiles_n, int thin) {
-  const int64_t full = static_cast<int64_t>(tiles_m - thin) * tiles_n, t = thin ? tiles_n : 0;
-  return 8 * ((full + 7) / 8 + (t + 7) / 8);
+// Ping-pong form: `full` tile rows of 256, then what is left of M in tile rows
+// of 128, whose tiles come after the others in every XCD's range.
+GS_HD int gemm_half_rows(int64_t M, int full) {
+  const int64_t left = M - static_cast<int64_t>(full) * 256;
+  return left > 0 ? static_cast<int>((left + 127) / 128) : 0;
 }
-GS_HD bool gemm_tile_thin(int bid, int tiles_m, int tiles_n, int thin, int group, int& tm, int& tn, bool& half) {
-  const int full = (tiles_m - thin) * tiles_n;
-  const int per = (full + 7) >> 3;
+GS_HD int64_t gemm_mixed_grid(int full, int halves, int64_t tiles_n) {
+  return 8 * ((full * tiles_n + 7) / 8 + (halves * tiles_n + 7) / 8);
+}
+GS_HD bool gemm_tile_mixed(int bid, int full, int halves, int tiles_n, int group, int& first_row, int& tn, bool& half) {
+  const int per = (full * tiles_n + 7) >> 3;
   half = (bid >> 3) >= per;
-  if (!half) return gemm_tile(bid, tiles_m - thin, tiles_n, group, tm, tn);
-  tm = tiles_m - 1;
-  tn = (bid & 7) * ((tiles_n + 7) >> 3) + (bid >> 3) - per;
-  return thin && tn < tiles_n;
+  int tm = 0;
+  const bool ok = half ? gemm_tile(bid - 8 * per, halves, tiles_n, group, tm, tn) : gemm_tile(bid, full, tiles_n, group, tm, tn);
+  first_row = half ? 256 * full + 128 * tm : 256 * tm;
+  return ok;
 }
 // The tile column staged as row r (0 .. 127) of column half h: the 32 rows of
 // wave column r / 32 hold its columns h * 32 .. + 31, so ordered that matrix

@@ -20,6 +20,7 @@
 #include <stdarg.h>
 
 #include <algorithm>
+#include <set>
 #include <type_traits>
 #include <utility>
 #include <vector>
@@ -50,8 +51,8 @@ struct GemmParams {
   int64_t ldc;
   int M, N, K;
   int tiles_m, tiles_n;
-  int tile_rows;          // 256, or 128: every tile is one row half (ping-pong form)
-  int thin;               // the last tile row has at most 128 rows (the ping-pong form runs it at half the work)
+  int full_rows;          // ping-pong form: tile rows of 256, before
+  int half_rows;          // those of 128
 };
 
 // WM x WN waves over k-tiles of 64 in two LDS stages (one barrier per k-tile);
@@ -203,10 +204,11 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_tn_kernel(GemmParams p
 // memory part, until those older than six phases have landed: exactly the half
 // that the next phase reads.  So a transfer has ~3000 clocks to arrive.
 //
-// A last tile row of at most 128 rows runs the two phases of row half 0 only
-// (HALF), at two thirds of the time; those tiles come last in every XCD's
-// range.  Calls whose 256-row tiles would leave most CUs idle cut every tile
-// to that form (pick_gemm).
+// Tile rows of 128 run the two phases of row half 0 only (HALF), at 0.7 of the
+// time; those tiles come last in every XCD's range.  A last tile row of at most
+// 128 rows is one, and as many before it as shorten the last, part-filled
+// round of tiles -- all of them, where 256-row tiles would leave most CUs idle
+// (pick_gemm).
 //
 // Bound by LDS (64 KB of transfers in at 64 bytes per clock, 192 KB of operand
 // reads at 128: 2560 clocks per k-tile against 2048 of MFMAs; 1.1 us measured)
@@ -461,12 +463,12 @@ __device__ __forceinline__ void gemm_tile_pingpong(const GemmParams& p, char* sm
 
 __global__ __launch_bounds__(512) void gemm_bf16_tn_pingpong_kernel(GemmParams p) {
   __shared__ __align__(16) char smem[2 * kPStage];
-  int tm, tn;
+  int first, tn;
   bool half;
-  if (!addr::gemm_tile_thin(static_cast<int>(blockIdx.x), p.tiles_m, p.tiles_n, p.thin, kGGroup, tm, tn, half)) return;
-  half |= p.tile_rows == kGBM / 2;
-  if (half) gemm_tile_pingpong<true>(p, smem, tm * p.tile_rows, tn);
-  else gemm_tile_pingpong<false>(p, smem, tm * p.tile_rows, tn);
+  if (!addr::gemm_tile_mixed(static_cast<int>(blockIdx.x), p.full_rows, p.half_rows, p.tiles_n, kGGroup, first, tn, half))
+    return;
+  if (half) gemm_tile_pingpong<true>(p, smem, first, tn);
+  else gemm_tile_pingpong<false>(p, smem, first, tn);
 }
 
 // ---------------------------------------------------------------------------
@@ -674,7 +676,6 @@ __global__ __launch_bounds__(64 * W) void gemm_bf16_tn_stream_kernel(GemmParams 
 inline bool pingpong_form(int64_t K, int64_t lda, int64_t ldb) {
   return K % kPBK == 0 && K >= 2 * kPBK && lda <= kPMaxLd && ldb <= kPMaxLd;
 }
-inline int gemm_thin(int64_t M) { return M % kGBM >= 1 && M % kGBM <= kGBM / 2 ? 1 : 0; }
 
 struct StreamForm {
   int MB, NB, W, RS, LA;
@@ -704,20 +705,43 @@ const StreamForm kStreamForms[] = {
 //   256                                34.8      28.9                76
 //   512                                59.2      50.8                75
 //   777                                83.3      83.2      55        75
+constexpr int64_t kCus = 256, kFullClocks = 2400, kHalfClocks = 1700;
+// Clocks per 64 k of `full` 256-row tiles followed by `halves` 128-row ones on
+// kCus CUs, each taking the next tile when it is free.
+inline int64_t gemm_mixed_clocks(int64_t full, int64_t halves) {
+  const int64_t late = full % kCus, early = kCus - late;        // CUs that run one full tile more, and the others
+  const int64_t t_early = full / kCus * kFullClocks, t_late = t_early + kFullClocks;
+  const int64_t end = late > 0 ? t_late : t_early;
+  if (halves == 0) return end;
+  // halves done once the early CUs have run k: early * k + late * (k - 2) at
+  // their k-th end, early * k + late * (k - 1) at the late CUs' next one
+  static_assert(kFullClocks > kHalfClocks && kFullClocks < 2 * kHalfClocks, "the order of the two groups' ends");
+  for (int64_t k = std::max<int64_t>(1, halves / kCus - 1);; ++k) {
+    if (early * k + late * std::max<int64_t>(0, k - 2) >= halves) return std::max(end, t_early + k * kHalfClocks);
+    if (early * k + late * (k - 1) >= halves) return std::max(end, t_late + (k - 1) * kHalfClocks);
+  }
+}
 struct GemmPick {
   const StreamForm* stream;   // nullptr: the ping-pong form
-  int tile_rows;
+  int full_rows;              // its tile rows of 256
 };
+// Ping-pong, 4144 x 4864 x 12800 (17 x 19 tiles, the last row of 48): 461 us
+// with 16 full tile rows (304 tiles on 256 CUs, 48 in a second round) and one
+// half row, 392 us with 13 and 7; 4096 x 4480 x 12800 457 -> 381 us, 3333 x
+// 6150 x 4096 200 -> 172.
 inline GemmPick pick_gemm(int64_t M, int64_t N, int64_t K) {
-  constexpr int64_t kCus = 256;
   auto tiles = [&](int64_t tm, int64_t tn) { return ((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
   auto rounds = [&](int64_t n) { return (n + kCus - 1) / kCus; };
-  GemmPick best{nullptr, kGBM};
-  int64_t cost = 2400 * rounds(tiles(kGBM, kGBN));
-  const int64_t half = 1700 * rounds(tiles(kGBM / 2, kGBN));
-  if (half < cost) {
-    cost = half;
-    best.tile_rows = kGBM / 2;
+  const int64_t tiles_m = (M + kGBM - 1) / kGBM, tiles_n = (N + kGBN - 1) / kGBN;
+  GemmPick best{nullptr, static_cast<int>(tiles_m)};
+  int64_t cost = INT64_MAX;
+  // a tile row fewer at a time (16 of them level out any last round)
+  for (int64_t f = tiles_m; f >= std::max<int64_t>(0, tiles_m - 16); --f) {
+    const int64_t c = gemm_mixed_clocks(f * tiles_n, addr::gemm_half_rows(M, static_cast<int>(f)) * tiles_n);
+    if (c < cost) {
+      cost = c;
+      best.full_rows = static_cast<int>(f);
+    }
   }
   for (const StreamForm& f : kStreamForms) {
     const int64_t tc = (f.RS + f.MB + f.NB - 1) / (f.MB + f.NB);
@@ -826,9 +850,9 @@ struct GemmModel {
   // gemm_bf16_tn_pingpong_kernel: every workgroup's transfers, operand reads
   // and stores, each tile and each element of C once, and each operand read
   // landing on the rows and columns its result is stored at
-  void pingpong(int tile_rows) {
-    const int nk = static_cast<int>(K / kPBK), thin = tile_rows == kGBM ? gemm_thin(M) : 0;
-    tiles_m = static_cast<int>((M + tile_rows - 1) / tile_rows);
+  void pingpong(int full) {
+    const int nk = static_cast<int>(K / kPBK), halves = addr::gemm_half_rows(M, full);
+    const int slots = static_cast<int>((M + 127) / 128);       // tile rows of 128
     HalfLayout st;
     for (int wave = 0; wave < 8; ++wave)
       for (int l = 0; l < 64; ++l)
@@ -861,17 +885,16 @@ struct GemmModel {
               }
             }
       }
-    const int64_t total = int64_t(tiles_m) * tiles_n, grid = addr::gemm_thin_grid(tiles_m, tiles_n, thin);
+    const int64_t total = int64_t(slots) * tiles_n, grid = addr::gemm_mixed_grid(full, halves, tiles_n);
     std::vector<char> seen(total, 0);
     for (int64_t b = 0; b < grid; ++b) {
-      int tm, tn;
+      int first, tn;
       bool half;
-      if (!addr::gemm_tile_thin(static_cast<int>(b), tiles_m, tiles_n, thin, kGGroup, tm, tn, half)) continue;
-      if (!in("tile row", tm, 1, tiles_m) || !in("tile column", tn, 1, tiles_n)) continue;
-      if (seen[int64_t(tm) * tiles_n + tn]++) fail("tile (%d, %d) taken twice", tm, tn);
-      half |= tile_rows == kGBM / 2;
-      const int first = tm * tile_rows;
-      if (half && std::min<int64_t>(M - first, tile_rows) > kGBM / 2) fail("tile row %d has rows past the first half", tm);
+      if (!addr::gemm_tile_mixed(static_cast<int>(b), full, halves, tiles_n, kGGroup, first, tn, half)) continue;
+      if (!in("tile row", first / 128, 1, slots) || !in("tile column", tn, 1, tiles_n)) continue;
+      const int tile_rows = half ? kGBM / 2 : kGBM;
+      for (int r = first / 128; r < (first + tile_rows) / 128 && r < slots; ++r)
+        if (seen[int64_t(r) * tiles_n + tn]++) fail("rows %d on of tile column %d taken twice", 128 * r, tn);
       std::vector<char> cseen(kGBM * kGBN, 0);
       for (int wave = 0; wave < 8; ++wave)
         for (int l = 0; l < 64; ++l) {
@@ -903,7 +926,7 @@ struct GemmModel {
       for (int r = 0; r < tile_rows; ++r)
         for (int c = 0; c < kGBN; ++c)
           if (first + r < M && tn * kGBN + c < N && !cseen[r * kGBN + c]) {
-            fail("C element (%d, %d) of tile (%d, %d) is never stored", r, c, tm, tn);
+            fail("C element (%d, %d) of the tile at row %d, tile column %d is never stored", r, c, first, tn);
             r = kGBM;
             break;
           }
@@ -1085,10 +1108,9 @@ int gs_gemm_bf16_tn(const void* a, int64_t lda, const void* b, int64_t ldb, void
       GS_CHECK_LAUNCH(who);
       return GS_OK;
     }
-    p.tile_rows = pick.tile_rows;
-    p.tiles_m = static_cast<int>((M + p.tile_rows - 1) / p.tile_rows);
-    p.thin = p.tile_rows == kGBM ? gemm_thin(M) : 0;
-    const unsigned n = static_cast<unsigned>(addr::gemm_thin_grid(p.tiles_m, p.tiles_n, p.thin));
+    p.full_rows = pick.full_rows;
+    p.half_rows = addr::gemm_half_rows(M, p.full_rows);
+    const unsigned n = static_cast<unsigned>(addr::gemm_mixed_grid(p.full_rows, p.half_rows, p.tiles_n));
     hipLaunchKernelGGL(gemm_bf16_tn_pingpong_kernel, dim3(n), dim3(512), 0, st, p);
   } else if (K % kGBK == 0) launch_gemm<false>(grid, p, st);
   else launch_gemm<true>(grid, p, st);
@@ -1110,8 +1132,8 @@ int64_t gs_check_gemm_addresses(int64_t M, int64_t N, int64_t K, int64_t lda, in
   m.tiles_m = static_cast<int>((M + kGBM - 1) / kGBM);
   m.tiles_n = static_cast<int>((N + kGBN - 1) / kGBN);
   if (pingpong_form(K, lda, ldb)) {
-    m.pingpong(kGBM);
-    m.pingpong(kGBM / 2);
+    std::set<int> forms = {m.tiles_m, m.tiles_m - 1, m.tiles_m / 2, 0, pick_gemm(M, N, K).full_rows};
+    for (int full : forms) m.pingpong(full);
     for (const StreamForm& f : kStreamForms)
       if (K / kPBK / f.W >= (f.RS + f.MB + f.NB - 1) / (f.MB + f.NB)) m.stream(f);
     m.tiles_m = static_cast<int>((M + kGBM - 1) / kGBM);

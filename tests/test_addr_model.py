@@ -333,6 +333,7 @@ def test_builder_random_batches(T, NA, seed):
     (1100, 3000, 8, 0),
     (128, 264, 192, 0),            # a thin tile row alone
     (2049, 775, 128, 8),           # tile rows of 8, then one of one row
+    (2500, 8450, 192, 0),          # 256-row tiles, then 128-row ones
 ])
 def test_gemm_shapes(M, N, K, pad):
     msg = ctypes.create_string_buffer(512)

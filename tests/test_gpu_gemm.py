@@ -66,6 +66,8 @@ def test_gemm_pingpong_tile_edges(dev, M, N, K):
     (256, 7296, 512), (255, 7290, 1152), (300, 6149, 832),            # 128 x 64
     # 128-row tiles of the ping-pong form (too few 256-row ones to fill the CUs)
     (777, 7296, 256), (1100, 6001, 192), (129, 300, 128),
+    # 256-row tiles, then 128-row ones that level out the last round: a ragged last row, ragged columns
+    (4144, 4864, 128), (2500, 8450, 192), (3333, 6150, 128),
 ])
 def test_gemm_forms_for_few_tiles(dev, M, N, K):
     test_gemm_matches_fp32_reference(dev, M, N, K, M + N + K)
