@@ -75,13 +75,31 @@ GS_HD void even_range(int n, int parts, int i, int& lo, int& count) {
   count = q + (i < r ? 1 : 0);
 }
 // The sub-tiles of workgroup b of an expand launch of `grid` (a multiple of 8)
-// workgroups, as positions tile * n_sub + sub of `total` tiles: XCD b % 8
-// takes an eighth of them, its workgroups near-equal shares of that.
-GS_HD void expand_span(int b, int grid, int total, int n_sub, int& lo, int& count) {
+// workgroups: `count` from sub-tile `sub` of tile `tile` on, tile after tile, of
+// `total` tiles (count 0: none).  XCD b % 8 takes an eighth of them, its
+// workgroups near-equal shares of that.  With
+// whole groups, every XCD takes whole tiles and every tile is cut into as many
+// equal spans as fit, so that no span crosses into a second tile: always (the
+// grid then holds 8 * ceil(total / 8)), or from kExpandWholeTiles tiles on
+// while the grid holds them.
+enum ExpandCut { kCutSpans, kCutWholeFrom64, kCutWhole };
+constexpr int kExpandWholeTiles = 64;
+GS_HD void expand_span(int b, int grid, int total, int n_sub, ExpandCut cut, int& tile, int& sub, int& count) {
+  const int tpx = (total + 7) >> 3;
+  if (total > 0 && (cut == kCutWhole || (cut == kCutWholeFrom64 && total >= kExpandWholeTiles && 8 * tpx <= grid))) {
+    const int groups = imin(grid / (8 * tpx), n_sub);
+    const int j = b >> 3, g = j / tpx;
+    tile = (b & 7) * tpx + j - g * tpx;
+    sub = (g * n_sub) / groups;
+    count = g < groups && tile < total ? ((g + 1) * n_sub) / groups - sub : 0;
+    return;
+  }
   int xlo, xn;
   even_range(total * n_sub, 8, b & 7, xlo, xn);
+  int lo;
   even_range(xn, grid >> 3, b >> 3, lo, count);
-  lo += xlo;
+  tile = (xlo + lo) / n_sub;
+  sub = xlo + lo - tile * n_sub;
 }
 // First output column of the lane's 16-byte y piece in sub-tile sub of NT
 // columns (the last piece of a partial sub-tile re-reads the row's last one).

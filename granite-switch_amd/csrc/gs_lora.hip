@@ -506,9 +506,11 @@ __global__ __launch_bounds__(kThreads) void reduce_parts_kernel(const float* __r
 // Whole column groups per tile in place of spans left workgroup slots without
 // work and XCDs with fewer tiles than others: 4096 rows x 4096 of 48 adapters
 // 17.5 -> 16.1 us, 256 x 6144 of 12 (13 tiles) 7.0 -> 6.3, and 22.2 -> 18.6
-// in the pair expand.  From there it is bound by the y stream: 4500 rows x
-// 25600 take 97 us, 4.76 TB/s read + written, the rate of a bare
-// read-modify-write of the same rows (4.7 TB/s).
+// in the pair expand.  The 256-column form, whose start costs about three of
+// its sub-tiles, keeps whole groups (in the pair expand from 64 tiles on): 125
+// tiles x 4096 16.2 us against 17.0, x 25600 82.5 against 84.5 with spans.  From there it is bound by the y stream: 4500 rows x 25600
+// take 97 us, 4.76 TB/s read + written, the rate of a bare read-modify-write
+// of the same rows (4.7 TB/s).
 // The tile's shrink values for every slice (z rows, or the sum of
 // the split-K partials rounded to the element type exactly like a
 // materialised z) are staged in LDS once.  Per sub-tile each wave computes NBW
@@ -825,22 +827,34 @@ __device__ __forceinline__ void expand_item(const ExpandParams& p, const TileRef
   compute(sub0 + nsub - 1, bc, yc);
 }
 
-// A workgroup's span of a launch of `grid` workgroups (addr::expand_span).
-// before_last() runs before the span's last sub-tile's products.
-template <bool BF16, int NBW, int PRE, typename Hook = NoHook>
+// The cut of an expand launch: whole groups for the 256-column form (one item
+// per workgroup, compiled without the walk), which in the pair expand takes
+// spans below 64 tiles.
+constexpr addr::ExpandCut expand_cut(int NBW, bool pair) {
+  return NBW == 1 ? addr::kCutSpans : (pair ? addr::kCutWholeFrom64 : addr::kCutWhole);
+}
+
+// A workgroup's span of the launch (addr::expand_span).  before_last() runs
+// before the span's last sub-tile's products.
+template <bool BF16, int NBW, int PRE, bool PAIR, typename Hook = NoHook>
 __device__ __forceinline__ void expand_walk(const ExpandParams& p, float (&dtile)[kTM][4 * NBW * 32 + kOutPad],
                                             char* zs, Hook before_last = Hook{}) {
   constexpr int NT = 4 * NBW * 32;
   const int n_sub = (p.out_total + NT - 1) / NT;
-  int lo = 0, left = 0, sub = 0, total = 0;
+  int tile = 0, left = 0, sub = 0, total = 0;
   TileRef tr = locate_item<kTM, kExpandBalanced>(p.seg, p.ranks, p.b_off, p.NA, p.rw,
                                                  [&](int tot) {
+                                                   int first;
                                                    addr::expand_span(static_cast<int>(blockIdx.x),
-                                                                     static_cast<int>(gridDim.x), tot, n_sub, lo, left);
-                                                   return left > 0 ? XcdItem{lo / n_sub, lo % n_sub} : XcdItem{-1, 0};
+                                                                     static_cast<int>(gridDim.x), tot, n_sub,
+                                                                     expand_cut(NBW, PAIR), tile, first, left);
+                                                   return XcdItem{left > 0 ? tile : -1, first};
                                                  }, sub, total);
   if (left <= 0) return;
-  int tile = lo / n_sub;
+  if constexpr (expand_cut(NBW, PAIR) == addr::kCutWhole) {
+    expand_item<BF16, NBW, PRE, false>(p, tr, sub, left, p.nparts, dtile, zs, before_last);
+    return;
+  }
   for (;;) {
     const int n = min(left, n_sub - sub);
     left -= n;
@@ -862,13 +876,13 @@ __device__ __forceinline__ void expand_walk(const ExpandParams& p, float (&dtile
 // registers per lane; the rank-64 multiswitch projection measured faster at
 // 4 than at 3).
 template <bool BF16, int NBW, int PRE, bool LOOP>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(!BF16 || LOOP || PRE > 4 ? 1 : (NBW == 1 ? 4 : 3))))
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BF16 && NBW == 1 && PRE <= 4 && !LOOP ? 4 : 1)))
 void expand_kernel(ExpandParams p) {
   constexpr int NT = 4 * NBW * 32;
   __shared__ float dtile[kTM][NT + kOutPad];
   extern __shared__ __align__(16) char zs[];   // [32][S*max_rank + 8] element type
   if constexpr (!LOOP) {
-    expand_walk<BF16, NBW, PRE>(p, dtile, zs);
+    expand_walk<BF16, NBW, PRE, false>(p, dtile, zs);
     return;
   }
   const int n_sub = (p.out_total + NT - 1) / NT;
@@ -1272,7 +1286,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   // the first claim goes out before the small class's last sub-tile, so its
   // round trip passes while that sub-tile is computed; its result is written
   // to LDS only afterwards (no wait for it before)
-  expand_walk<true, NBW, PRE>(p0, dtile, zs, [&]() {
+  expand_walk<true, NBW, PRE, true>(p0, dtile, zs, [&]() {
     if (threadIdx.x == 0) ticket = claim_next(claim);
     early = true;
   });
@@ -1595,8 +1609,11 @@ int prepare_expand(ExpandParams& p, const char* who, int32_t dtype, void* y, int
 }
 
 // Workgroups of a column-split expand launch: one round (wt), at most one per
-// (tile slot, sub-tile); a multiple of 8 (addr::expand_span).
-int64_t expand_grid(int64_t wt, int max_tiles, int64_t n_sub) {
+// (tile slot, sub-tile), a multiple of 8 (addr::expand_span); cut into whole
+// groups, one per tile slot when those alone exceed a round.
+int64_t expand_grid(int64_t wt, int max_tiles, int64_t n_sub, addr::ExpandCut cut) {
+  const int64_t t8 = (static_cast<int64_t>(max_tiles) + 7) / 8 * 8;
+  if (cut == addr::kCutWhole) return (std::min<int64_t>(std::max(wt, t8), t8 * n_sub) + 7) / 8 * 8;
   return (std::min<int64_t>(wt, static_cast<int64_t>(max_tiles) * n_sub) + 7) / 8 * 8;
 }
 
@@ -1624,7 +1641,8 @@ void launch_expand_t(int max_tiles, size_t lds, ExpandParams p, hipStream_t st) 
   }
   constexpr int NT = 4 * NBW * 32;
   const int grid = static_cast<int>(expand_grid(static_cast<int64_t>(o & 0xffff) * device_cus(), max_tiles,
-                                                (p.out_total + NT - 1) / NT));
+                                                (p.out_total + NT - 1) / NT,
+                                                p.flat ? addr::kCutSpans : expand_cut(NBW, false)));
   hipLaunchKernelGGL(kern, dim3(grid), dim3(kThreads), lds, st, p);
 }
 
@@ -1793,7 +1811,7 @@ int pair_expand_occupancy(const void* kern, size_t lds) {
 int64_t pair_expand_grid(const PairForm& f, int64_t T, int adapters0, size_t lds, const ExpandParams& e0) {
   const int64_t wt = static_cast<int64_t>(pair_expand_occupancy(expand_pair_fn_of(f), lds)) * device_cus();
   const int NT = 4 * f.f0.NBW * 32;
-  return expand_grid(wt, max_tiles_for(T, adapters0), (e0.out_total + NT - 1) / NT);
+  return expand_grid(wt, max_tiles_for(T, adapters0), (e0.out_total + NT - 1) / NT, expand_cut(f.f0.NBW, true));
 }
 
 // Workgroups that sum the large class's partials (sum_partials): for the tiles
@@ -2104,7 +2122,7 @@ struct AddrModel {
   // claimed: the items are taken from a counter (each exactly once) instead
   // of by a grid.
   void expand(const ExpandParams& e, const ExpandForm& f, int adapters, int64_t wt, int64_t z_elems,
-              int64_t part_elems, const int32_t* z_off, int qb = kSpNT / 32, bool claimed = false) {
+              int64_t part_elems, const int32_t* z_off, int qb = kSpNT / 32, bool claimed = false, bool pair = false) {
     const bool flat = e.flat != 0;
     const int max_tiles = max_tiles_for(T, adapters);
     const std::vector<TileRef> tl = tiles<kTM, kExpandBalanced>(e.rw, b_off);
@@ -2230,7 +2248,8 @@ struct AddrModel {
       while (s_hi + 1 < si.S && c_last >= si.bounds[s_hi + 1]) ++s_hi;
       stage(tr, s_lo, s_hi, s_lo * r, zs_ld, lds, nparts);
     };
-    const int64_t grid = expand_grid(wt, max_tiles, n_sub);
+    const addr::ExpandCut cut = flat ? addr::kCutSpans : expand_cut(f.NBW, pair);
+    const int64_t grid = expand_grid(wt, max_tiles, n_sub, cut);
     if (flat) {
       for_items("expand_kernel", grid, true, work_items(total, n_sub, true), [&](int lin) {
         const XcdItem it = work_item(lin, total, n_sub, true);
@@ -2241,15 +2260,17 @@ struct AddrModel {
     // the workgroups' spans: each (tile, sub-tile) exactly once, in order per XCD
     std::vector<char> seen(static_cast<size_t>(total) * n_sub, 0);
     for (int64_t b = 0; b < grid; ++b) {
-      int lo = 0, left = 0;
-      addr::expand_span(static_cast<int>(b), static_cast<int>(grid), total, n_sub, lo, left);
+      int tile = 0, sub = 0, left = 0;
+      addr::expand_span(static_cast<int>(b), static_cast<int>(grid), total, n_sub, cut, tile, sub, left);
       while (left > 0) {
-        const int tile = lo / n_sub, sub = lo % n_sub, n = std::min(left, n_sub - sub);
+        const int n = std::min(left, n_sub - sub);
+        const int64_t lo = static_cast<int64_t>(tile) * n_sub + sub;
         if (!in("expand span", lo, n, static_cast<int64_t>(total) * n_sub)) break;
         for (int k = 0; k < n; ++k)
           if (seen[lo + k]++) fail("expand_kernel: (tile %d, sub-tile %d) is taken twice", tile, sub + k);
         item(tl[tile], sub, n);
-        lo += n;
+        ++tile;
+        sub = 0;
         left -= n;
       }
     }
@@ -2765,7 +2786,7 @@ int64_t gs_check_segment_addresses(int32_t dtype, int64_t num_tokens, int32_t hi
           m.shrink_dma(pl0, cls[0].rw, zl, z_elems, part0);
           m.shrink_dma(pl1, cls[1].rw, zl, z_elems, part1, pl0.grid, 1);
           for (int occ = 1; occ <= 4; ++occ)
-            m.expand(e0, pf.f0, cls[0].adapters, int64_t(occ) * cus, z_elems, part0, nullptr);
+            m.expand(e0, pf.f0, cls[0].adapters, int64_t(occ) * cus, z_elems, part0, nullptr, kSpNT / 32, false, true);
           const ExpandForm f1{true, 1, 2, pf.KG1};
           e1.z = &m;           // a call's z (only its presence is read)
           e1.sum_wgs = pair_sum_wgs(e1, cls[1], INT64_MAX);
