@@ -12,9 +12,10 @@
 // tiles running together on one XCD share its L2.  Partial tiles clamp their
 // loads to the last row and mask their stores.
 //
-// Two kernels: for K % 64 == 0 (and K >= 128) the k-tiles go from global memory
+// Three kernels: for K % 64 == 0 (and K >= 128) the k-tiles go from global memory
 // straight into LDS and the two waves of a SIMD alternate between reading and
-// multiplying (gemm_bf16_tn_pingpong_kernel); otherwise they are loaded into
+// multiplying (gemm_bf16_tn_pingpong_kernel), or, for few tiles, smaller ones
+// split K over their waves (gemm_bf16_tn_stream_kernel); otherwise they are loaded into
 // registers, zero-filled past K, and written to padded LDS rows
 // (gemm_bf16_tn_kernel).
 #include <stdarg.h>

@@ -872,6 +872,8 @@ int gs_build_segments(const int64_t* req_ids, const int64_t* positions, const in
 int gs_route_latest_wins(const int64_t* input_ids, const int32_t* cu_seqlens, int64_t num_tokens,
                          int32_t num_seqs, const int64_t* control_tokens, int32_t num_control, int32_t id_offset,
                          const int64_t* start_ids, int64_t* out_ids, void* stream) {
+  GS_CHECK_ARG(num_tokens <= 0 || out_ids + num_tokens <= input_ids || input_ids + num_tokens <= out_ids,
+               "gs_route_latest_wins: out_ids overlaps input_ids");
   GS_CHECK_ARG(num_control >= 0 && num_control <= GS_MAX_ADAPTERS + 1, "gs_route_latest_wins: num_control=%d",
                num_control);
   GS_CHECK_ARG(num_tokens >= 0 && num_tokens < (int64_t(1) << 31), "gs_route_latest_wins: num_tokens out of range");
