@@ -79,6 +79,7 @@ SIGNATURES = {
                                        c_void_p, c_i64, c_i32, c_i32, c_void_p]),
     "gs_compute_bitmasks": (c_i32, [c_void_p, c_i32, c_i64, c_void_p, c_i32, c_i32, c_i32, c_void_p, c_void_p,
                                     c_void_p]),
+    "gs_bitmask_table_form": (c_i32, [c_i64, c_i32, c_i32, c_i32]),
     "gs_switch_lora_expand": (c_i32, [c_void_p, c_i64, c_i64, c_i64, c_void_p, c_i32, c_void_p, c_i64, c_void_p,
                                       c_void_p, c_void_p, c_void_p, c_i32, c_i32, c_i32, c_void_p]),
     "gs_switch_lora_expand_swiglu": (c_i32, [c_void_p, c_i64, c_i64, c_void_p, c_i64, c_i64, c_i64, c_void_p, c_i32,

@@ -427,7 +427,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_latest_wins_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Reference bitmasks and remap gather, two forms (gs_compute_bitmasks picks).
+// Reference bitmasks and remap gather, two forms (remap_lds_form picks).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int64_t load_idx(const void* p, int bytes, int64_t i) {
   return bytes == 8 ? static_cast<const int64_t*>(p)[i] : static_cast<int64_t>(static_cast<const int32_t*>(p)[i]);
@@ -437,7 +437,7 @@ __device__ __forceinline__ uint64_t loc_bit(int64_t loc) {
   return (loc > 0 && loc <= 64) ? (1ull << (loc - 1)) : 0ull;
 }
 
-// The form for the sizes in use (tiles of a power of two from 8 to 512 tokens,
+// The form for large calls (tiles of a power of two from 8 to 512 tokens,
 // tables of at most GS_MAX_ADAPTERS + 1 ids): a workgroup takes kRemapTok
 // tokens and `mg` modules.  It stages those modules' tables in LDS and reads
 // its tokens' ids once for all of them; a module then costs a token one LDS
@@ -447,13 +447,30 @@ __device__ __forceinline__ uint64_t loc_bit(int64_t loc) {
 // Bound by the stores: 8 bytes per token and module.  32768 tokens, 160
 // modules, 24 adapters (43 MB written): 10.8 us (4.1 TB/s); with one thread per (token,
 // module), its gather from L2 and a 64-bit OR over lanes for each, 19.7 us.
+// Its chain (tables, id sets, then up to a tile's worth of ids one after the
+// other) is longer than the general form's, so small calls are that one's
+// (remap_lds_form).
 constexpr int kRemapTok = 512;                   // tokens per workgroup
 constexpr int kRemapMods = 16;                   // modules per workgroup at most
 constexpr int kRemapWords = (GS_MAX_ADAPTERS + 1 + 63) / 64;
 
 // Tiles must not cross workgroups, and the tables and id sets fit their LDS.
-inline bool remap_lds_form(int block_m, int na_plus_1) {
+inline bool remap_lds_takes(int block_m, int na_plus_1) {
   return block_m >= 8 && block_m <= kRemapTok && (block_m & (block_m - 1)) == 0 && na_plus_1 <= GS_MAX_ADAPTERS + 1;
+}
+// ... and the call is large enough for it: its fixed chain grows with the
+// ids that a tile can hold.  us, general / LDS form, tiles of 32 tokens:
+//   tokens x modules   24 adapters   64             255
+//   256 x 160          3.3 / 4.8     3.3 / 5.6      3.4 / 6.9
+//   4144 x 160         5.8 / 6.5     5.9 / 7.2      6.2 / 8.7
+//   8192 x 160         8.4 / 7.8     8.3 / 8.5      8.6 / 9.7
+//   16384 x 160        12.8 / 9.6    12.9 / 10.6    12.8 / 12.3
+//   32768 x 160        22.3 / 12.8   22.3 / 14.2    22.6 / 18.1
+// The general form reads a tile of more than 64 tokens with one thread: from
+// 4 tokens on (3: 2.5 / 2.5, 5: 2.8 / 2.6, 256: 46 / 5.4) it is the slower one.
+inline bool remap_lds_form(int64_t M, int num_modules, int block_m, int na_plus_1) {
+  if (!remap_lds_takes(block_m, na_plus_1)) return false;
+  return block_m > 64 ? M > 3 : M * num_modules >= (int64_t(1) << 20) + (int64_t(na_plus_1) << 13);
 }
 
 // Modules per workgroup: about 1024 workgroups (4 per CU), at most kRemapMods.
@@ -888,6 +905,10 @@ int gs_route_latest_wins(const int64_t* input_ids, const int32_t* cu_seqlens, in
   return GS_OK;
 }
 
+int gs_bitmask_table_form(int64_t M, int32_t na_plus_1, int32_t num_modules, int32_t block_m) {
+  return remap_lds_form(M, num_modules, block_m, na_plus_1) ? 1 : 0;
+}
+
 int gs_compute_bitmasks(const void* adapter_indices, int32_t idx_bytes, int64_t M, const int64_t* remap_tables_t,
                         int32_t na_plus_1, int32_t num_modules, int32_t block_m, int64_t* bitmasks,
                         int64_t* remapped, void* stream) {
@@ -896,7 +917,7 @@ int gs_compute_bitmasks(const void* adapter_indices, int32_t idx_bytes, int64_t 
   GS_CHECK_ARG(na_plus_1 >= 1 && num_modules >= 1, "gs_compute_bitmasks: bad remap table shape");
   GS_CHECK_ARG(M >= 0 && M < (int64_t(1) << 31), "gs_compute_bitmasks: M out of range");
   if (M == 0) return GS_OK;
-  if (remap_lds_form(block_m, na_plus_1)) {
+  if (remap_lds_form(M, num_modules, block_m, na_plus_1)) {
     const int mg = remap_group(M, num_modules);
     const dim3 grid(static_cast<unsigned>((M + kRemapTok - 1) / kRemapTok),
                     static_cast<unsigned>((num_modules + mg - 1) / mg));
@@ -949,7 +970,7 @@ int64_t gs_check_token_addresses(int64_t num_tokens, int32_t num_seqs, const int
   if (num_tokens > 0) {
     m.route(num_control);
     m.bitmask(ids, na_plus_1, num_modules, block_m);
-    if (remap_lds_form(block_m, na_plus_1)) m.remap_bitmask(ids, na_plus_1, num_modules, block_m);
+    if (remap_lds_takes(block_m, na_plus_1)) m.remap_bitmask(ids, na_plus_1, num_modules, block_m);
     m.split(ids, lut_len);
   }
   if (checked) *checked = m.checked;

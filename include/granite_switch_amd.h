@@ -431,6 +431,9 @@ int gs_switched_lora_small(int32_t dtype, const int64_t* req_ids, const int64_t*
 int gs_compute_bitmasks(const void* adapter_indices, int32_t idx_bytes, int64_t M, const int64_t* remap_tables_t,
                         int32_t na_plus_1, int32_t num_modules, int32_t block_m, int64_t* bitmasks,
                         int64_t* remapped, void* stream);
+/* 1 if a call of these sizes takes the kernel that stages the tables in LDS
+ * (large calls), 0 for the general one.  Both give the same outputs. */
+int gs_bitmask_table_form(int64_t M, int32_t na_plus_1, int32_t num_modules, int32_t block_m);
 
 /* ------------------------------------------------------------------------
  * Reference op: in-place expand over x_ext (bf16), reference semantics.

@@ -193,6 +193,21 @@ def test_bitmask_and_remap_table_form(dev, M, block_m, NA, modules):
         assert np.array_equal(out.cpu().numpy(), remap[:, np.clip(ids, 0, NA)])
 
 
+@pytest.mark.parametrize("M,block_m,NA,modules", [
+    (8197, 32, 24, 200), (2625, 8, 64, 700), (5003, 64, 255, 700), (3100, 16, 2, 357), (4099, 512, 24, 3), (4, 128, 7, 2)])
+def test_bitmask_table_kernel_at_its_sizes(dev, M, block_m, NA, modules):
+    assert switched._lib.load().gs_bitmask_table_form(M, NA + 1, modules, block_m) == 1
+    rng = np.random.default_rng(M + block_m)
+    ids = rng.integers(-2, NA + 3, size=M)
+    remap = rng.integers(0, 65, size=(modules, NA + 1))
+    remap[:, 0] = 0
+    out = torch.full((modules, M), -1, dtype=torch.int64, device=dev)
+    got = kernels.compute_per_module_bitmasks(torch.tensor(ids, device=dev), torch.tensor(remap, device=dev).T.contiguous(),
+                                              block_m, remapped_out=out)
+    assert np.array_equal(got.cpu().numpy(), omap.compute_bitmasks(np.clip(ids, 0, NA), remap.T, block_m))
+    assert np.array_equal(out.cpu().numpy(), remap[:, np.clip(ids, 0, NA)])
+
+
 def test_bitmask_hand_derived(dev, kats):
     k = kats["bitmask"]
     ids = torch.tensor(k["adapter_indices"], device=dev)

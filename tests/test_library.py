@@ -313,6 +313,16 @@ def test_workload_module_on_cpu():
     assert md.lora_B_slices[0][1, 0].std().item() < 0.05
 
 
+@pytest.mark.parametrize("M,na,modules,block_m,table", [
+    (7, 24, 160, 32, False), (256, 24, 160, 32, False), (256, 255, 160, 32, False), (1024, 24, 500, 8, False),
+    (4144, 24, 160, 32, False), (8192, 24, 160, 32, True), (8192, 64, 160, 32, False), (32768, 24, 160, 32, True),
+    (32768, 255, 80, 32, False), (32768, 255, 160, 32, True), (32768, 24, 160, 24, False), (32768, 24, 160, 1024, False),
+    (32768, 300, 160, 32, False), (3, 24, 1, 128, False), (256, 24, 1, 512, True)])
+def test_bitmask_kernel_choice(M, na, modules, block_m, table):
+    """The table kernel's fixed chain is longer than the general kernel's whole run at serving sizes."""
+    assert switched._lib.load().gs_bitmask_table_form(M, na + 1, modules, block_m) == int(table)
+
+
 def test_host_tables_follow_the_pack():
     """The tables kept with a pack are made again after any field they follow
     from changes, in place or by assignment; the class views after a device
