@@ -426,6 +426,85 @@ __global__ __launch_bounds__(kRouteThreads) void route_latest_wins_kernel(
   out[t] = id;
 }
 
+// The form for an out that overlaps input_ids (routing in place): one workgroup
+// per sequence, which has read every token of a step of kRouteSeqThreads before
+// it writes the step, and needs none of the earlier ones again (the latest
+// control token so far is carried along).  The workgroups of the form above
+// look back at tokens that others may have written already.
+constexpr int kRouteSeqThreads = 256;
+
+__global__ __launch_bounds__(kRouteSeqThreads) void route_latest_wins_in_place_kernel(
+    const int64_t* input_ids, const int32_t* __restrict__ cu, int T, const int64_t* __restrict__ ctl, int num_control,
+    int id_offset, const int64_t* __restrict__ start_ids, int64_t* out) {
+  __shared__ int64_t ctl_s[GS_MAX_ADAPTERS + 1];
+  __shared__ int wave_max[kRouteSeqThreads / 64];
+  __shared__ int wave_id[kRouteSeqThreads / 64];
+  const int s = blockIdx.x;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  for (int i = tid; i < num_control; i += kRouteSeqThreads) ctl_s[i] = ctl[i];
+  lds_barrier();
+  const int lo = (cu != nullptr) ? cu[s] : 0;
+  const int hi = (cu != nullptr) ? cu[s + 1] : T;
+  // carry: (index of last control token so far, its fired id); index -1 = none
+  int carry_idx = -1;
+  int carry_id = (start_ids != nullptr) ? static_cast<int>(start_ids[s]) : 0;
+  for (int base = lo; base < hi; base += kRouteSeqThreads) {
+    const int t = base + tid;
+    int my_idx = -1, my_id = 0;
+    if (t < hi) {
+      const int64_t tok = input_ids[t];
+      for (int k = 0; k < num_control; ++k) {
+        if (ctl_s[k] == tok) {  // the first matching slot, like list.index
+          my_idx = t;
+          my_id = k + id_offset;
+          break;
+        }
+      }
+    }
+    // inclusive max-scan of (idx, id) by idx inside the wave
+    int sidx = my_idx, sid = my_id;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      int oi = __shfl_up(sidx, d, 64);
+      int od = __shfl_up(sid, d, 64);
+      if (lane >= d && oi > sidx) {
+        sidx = oi;
+        sid = od;
+      }
+    }
+    if (lane == 63) {
+      wave_max[wave] = sidx;
+      wave_id[wave] = sid;
+    }
+    lds_barrier();
+    // combine with earlier waves of this step, then with the carry
+    for (int w = 0; w < wave; ++w) {
+      if (wave_max[w] > sidx) {
+        sidx = wave_max[w];
+        sid = wave_id[w];
+      }
+    }
+    if (carry_idx > sidx) {
+      sidx = carry_idx;
+      sid = carry_id;
+    }
+    if (t < hi) out[t] = (sidx >= 0) ? sid : carry_id;
+    // new carry: the max over the whole step
+    int cidx = carry_idx, cid = carry_id;
+    for (int w = 0; w < kRouteSeqThreads / 64; ++w) {
+      if (wave_max[w] > cidx) {
+        cidx = wave_max[w];
+        cid = wave_id[w];
+      }
+    }
+    lds_barrier();
+    carry_idx = cidx;
+    carry_id = cid;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Reference bitmasks and remap gather, two forms (remap_lds_form picks).
 // ---------------------------------------------------------------------------
@@ -738,6 +817,25 @@ struct MetaModel {
       }
     }
   }
+  // ---- route_latest_wins_in_place_kernel: one workgroup per sequence --------
+  void route_in_place(int num_control) {
+    for (int sq = 0; sq < nseq; ++sq) {
+      for (int i = 0; i < num_control; ++i) {
+        in("control tokens", i, 1, num_control);
+        in("control tokens (LDS)", i, 1, GS_MAX_ADAPTERS + 1);
+      }
+      int lo = 0, hi = T;
+      if (cu != nullptr) {
+        in("cu_seqlens", sq, 2, nseq + 1);
+        lo = cu[sq];
+        hi = cu[sq + 1];
+      }
+      in("start ids (when given)", sq, 1, nseq);
+      for (int base = lo; base < hi; base += kRouteSeqThreads)
+        for (int tid = 0; tid < kRouteSeqThreads; ++tid)
+          if (base + tid < hi) in("tokens and routed ids", base + tid, 1, T);
+    }
+  }
   // ---- remap_bitmask_kernel: grid (token chunks, module groups) --------------
   void remap_bitmask(const int64_t* ids, int na_plus_1, int num_modules, int block_m) {
     const int M = T, mg = remap_group(T, num_modules), lb = __builtin_ctz(block_m);
@@ -889,14 +987,21 @@ int gs_build_segments(const int64_t* req_ids, const int64_t* positions, const in
 int gs_route_latest_wins(const int64_t* input_ids, const int32_t* cu_seqlens, int64_t num_tokens,
                          int32_t num_seqs, const int64_t* control_tokens, int32_t num_control, int32_t id_offset,
                          const int64_t* start_ids, int64_t* out_ids, void* stream) {
-  GS_CHECK_ARG(num_tokens <= 0 || out_ids + num_tokens <= input_ids || input_ids + num_tokens <= out_ids,
-               "gs_route_latest_wins: out_ids overlaps input_ids");
   GS_CHECK_ARG(num_control >= 0 && num_control <= GS_MAX_ADAPTERS + 1, "gs_route_latest_wins: num_control=%d",
                num_control);
   GS_CHECK_ARG(num_tokens >= 0 && num_tokens < (int64_t(1) << 31), "gs_route_latest_wins: num_tokens out of range");
   const int nseq = cu_seqlens ? num_seqs : 1;
   GS_CHECK_ARG(nseq >= 1, "gs_route_latest_wins: num_seqs=%d", num_seqs);
   if (num_tokens == 0) return GS_OK;
+  const uintptr_t in0 = reinterpret_cast<uintptr_t>(input_ids), out0 = reinterpret_cast<uintptr_t>(out_ids);
+  const uintptr_t bytes = static_cast<uintptr_t>(num_tokens) * sizeof(int64_t);
+  if (out0 < in0 + bytes && in0 < out0 + bytes) {
+    hipLaunchKernelGGL(route_latest_wins_in_place_kernel, dim3(nseq), dim3(kRouteSeqThreads), 0,
+                       static_cast<hipStream_t>(stream), input_ids, cu_seqlens, static_cast<int>(num_tokens),
+                       control_tokens, num_control, id_offset, start_ids, out_ids);
+    GS_CHECK_LAUNCH("gs_route_latest_wins");
+    return GS_OK;
+  }
   const int64_t chunks = (num_tokens + kRouteThreads - 1) / kRouteThreads;
   hipLaunchKernelGGL(route_latest_wins_kernel, dim3(static_cast<unsigned>(chunks)), dim3(kRouteThreads), 0,
                      static_cast<hipStream_t>(stream), input_ids, cu_seqlens, nseq, static_cast<int>(num_tokens),
@@ -969,6 +1074,7 @@ int64_t gs_check_token_addresses(int64_t num_tokens, int32_t num_seqs, const int
   m.cu = cu_seqlens;
   if (num_tokens > 0) {
     m.route(num_control);
+    m.route_in_place(num_control);
     m.bitmask(ids, na_plus_1, num_modules, block_m);
     if (remap_lds_takes(block_m, na_plus_1)) m.remap_bitmask(ids, na_plus_1, num_modules, block_m);
     m.split(ids, lut_len);

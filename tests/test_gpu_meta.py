@@ -178,6 +178,24 @@ def test_route_latest_wins_across_chunks(dev, lens, rate):
             assert list(got[cu[s]:cu[s + 1]]) == omap.latest_wins_ids(list(toks[cu[s]:cu[s + 1]]), atok, False, start[s]), s
 
 
+@pytest.mark.parametrize("lens,rate", [([9217, 40, 1, 3000], 0.001), ([1] * 300, 0.3), ([0, 257, 2100], 0.0)])
+def test_route_latest_wins_in_place(dev, lens, rate):
+    """out_ids may be input_ids."""
+    rng = np.random.default_rng(sum(lens))
+    atok = [500, 90007, 41]
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    toks = rng.integers(1000, 40000, size=int(cu[-1]))
+    ctl = rng.random(toks.size) < rate
+    toks[ctl] = rng.choice(atok, size=int(ctl.sum()))
+    start = rng.integers(0, 4, size=len(lens))
+    ids, c, s = torch.tensor(toks, device=dev), torch.tensor(atok, device=dev), torch.tensor(start, device=dev)
+    cut = torch.tensor(cu, device=dev)
+    exp = switched.route_latest_wins(ids, atok, 1, cut, s)
+    switched._lib.call("gs_route_latest_wins", ids.data_ptr(), cut.data_ptr(), ids.numel(), len(lens), c.data_ptr(),
+                       len(atok), 1, s.data_ptr(), ids.data_ptr(), switched._lib.stream_ptr(dev))
+    assert torch.equal(ids, exp)
+
+
 @pytest.mark.parametrize("M", [1, 511, 512, 513, 1300])
 @pytest.mark.parametrize("block_m,NA,modules", [(8, 40, 33), (32, 64, 161), (128, 256, 3), (512, 7, 1)])
 def test_bitmask_and_remap_table_form(dev, M, block_m, NA, modules):
