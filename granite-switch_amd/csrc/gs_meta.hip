@@ -314,9 +314,14 @@ __global__ __launch_bounds__(kBuildThreads) void build_scatter_kernel(BuildArgs 
 // sit at the end of a vocabulary).
 //
 // Bound by the chain of dependent memory trips, not by bytes: ids and tables,
-// then the look-back.  One workgroup per sequence (the earlier form, 256
-// tokens per step) left a 32768-token prompt batch of 5 sequences on 5 CUs:
-// 249 us, now 8.4 us.
+// then the look-back.  One workgroup per sequence (256 tokens per step, the
+// in-place form below) leaves a 32768-token prompt batch of 5 sequences on 5
+// CUs: 249 us, 8.4 here; 1024 one-token sequences 5.8 us, 5.3 here (5.6 with a
+// control token among them: its list is read 8 entries at a time).
+// A chunk whose sequence has no earlier control token reads all of the sequence
+// before it: for n tokens n^2 / 2048 reads, and n / 8192 trips for the last
+// chunk.  One sequence without any: 262144 tokens 60 us, 1 M 420 us, 4 M 4.9 ms
+// (per sequence: 2.98, 12.4 and 49.6 ms).
 // ---------------------------------------------------------------------------
 constexpr int kRouteThreads = 1024;              // threads, and tokens per chunk
 constexpr int kRouteWaves = kRouteThreads / 64;
@@ -330,8 +335,16 @@ __device__ __forceinline__ int route_slot(const int64_t* ctl_s, int num_control,
                                           bool active) {
   int slot = -1;
   if (__any(active && tok >= lo && tok <= hi)) {
-    for (int k = num_control - 1; k >= 0; --k)
-      if (active && ctl_s[k] == tok) slot = k;   // downwards: the first matching slot stays, like list.index
+    // downwards: the first matching slot stays, like list.index.  8 list reads in
+    // flight (entries below the first are read as the first, whose slot then wins)
+    for (int k0 = num_control - 1; k0 >= 0; k0 -= 8) {
+      int64_t c[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) c[u] = ctl_s[max(k0 - u, 0)];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) slot = c[u] == tok ? max(k0 - u, 0) : slot;
+    }
+    if (!active) slot = -1;
   }
   return slot;
 }
@@ -343,6 +356,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_latest_wins_kernel(
   __shared__ int64_t ctl_s[GS_MAX_ADAPTERS + 1];
   __shared__ int64_t rng_s[2];
   __shared__ int32_t cu_s[kCuCap + 1];
+  __shared__ int32_t first_lo_s;
   __shared__ int wave_last[kRouteWaves];
   __shared__ unsigned long long back_s;
   const int tid = threadIdx.x;
@@ -357,7 +371,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_latest_wins_kernel(
     for (int i = tid; i <= num_seqs; i += kRouteThreads) cu_s[i] = cu[i];
   if (tid == 0) back_s = 0;
   lds_barrier();
-  if (wave == 0) {                               // range of the control tokens
+  if (wave == 0 && num_control > 0) {            // range of the control tokens
     int64_t lo = INT64_MAX, hi = INT64_MIN;
     for (int i = lane; i < num_control; i += 64) {
       lo = min(lo, ctl_s[i]);
@@ -373,17 +387,22 @@ __global__ __launch_bounds__(kRouteThreads) void route_latest_wins_kernel(
       rng_s[1] = hi;
     }
   }
-  // this token's sequence [seq_lo, seq_hi), and the start of the chunk's first
-  // token's (tokens outside every sequence are not written)
-  int seq = 0, seq_lo = 0, seq_hi = T, first_lo = 0;
+  // this token's sequence [seq_lo, seq_hi), the first token's also the chunk's
+  // first_lo (tokens outside every sequence are not written)
+  int seq = 0, seq_lo = 0, seq_hi = T;
   if (cu != nullptr) {
     const int32_t* tab = cu_in_lds ? cu_s : cu;
     seq = find_seq(tab, num_seqs, min(t, T - 1));
     seq_lo = tab[seq];
     seq_hi = tab[seq + 1];
-    first_lo = tab[find_seq(tab, num_seqs, c0)];
   }
+  if (num_control == 0) {                        // nothing fires: every token keeps its sequence's start
+    if (t < T && t >= seq_lo && t < seq_hi) out[t] = start_ids != nullptr ? static_cast<int>(start_ids[seq]) : 0;
+    return;
+  }
+  if (tid == 0) first_lo_s = seq_lo;
   lds_barrier();
+  const int first_lo = first_lo_s;
   const int64_t lo = rng_s[0], hi = rng_s[1];
 
   const int slot = route_slot(ctl_s, num_control, lo, hi, tok, t < T);

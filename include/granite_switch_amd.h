@@ -160,7 +160,9 @@ int gs_split_adapter_indices(const uint8_t* kind_lut, int32_t lut_len, const voi
  * input_ids [T] int64; cu_seqlens [num_seqs+1] int32 or NULL;
  * control_tokens [num_control] int64; start_ids [num_seqs] int64 or NULL;
  * out_ids [T] int64, may be input_ids (routing in place: one workgroup per
- * sequence).  Limits: num_control <= GS_MAX_ADAPTERS + 1.
+ * sequence).  Apart from input_ids, each 1024 tokens are a workgroup's, which
+ * re-reads its first sequence's earlier tokens back to the latest control
+ * token.  Limits: num_control <= GS_MAX_ADAPTERS + 1.
  * ---------------------------------------------------------------------- */
 int gs_route_latest_wins(const int64_t* input_ids, const int32_t* cu_seqlens, int64_t num_tokens,
                          int32_t num_seqs, const int64_t* control_tokens, int32_t num_control, int32_t id_offset,

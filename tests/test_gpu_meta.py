@@ -178,6 +178,22 @@ def test_route_latest_wins_across_chunks(dev, lens, rate):
             assert list(got[cu[s]:cu[s + 1]]) == omap.latest_wins_ids(list(toks[cu[s]:cu[s + 1]]), atok, False, start[s]), s
 
 
+@pytest.mark.parametrize("num_control", [0, 1, 7, 8, 9, 257])
+def test_route_latest_wins_control_list_lengths(dev, num_control):
+    """No control tokens (every token keeps its sequence's start), and list lengths around the 8 read at a time."""
+    lens = [1] * 700 + [2500, 0, 3]
+    rng = np.random.default_rng(num_control)
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    atok = list(range(90000, 90000 + num_control))
+    toks = rng.integers(89990, 90000 + num_control + 10, size=int(cu[-1]))
+    start = rng.integers(0, 6, size=len(lens))
+    got = switched.route_latest_wins(torch.tensor(toks, device=dev), torch.tensor(atok, dtype=torch.int64), 1,
+                                     torch.tensor(cu, device=dev), torch.tensor(start, device=dev)).cpu().numpy()
+    for s in range(len(lens)):
+        if lens[s]:
+            assert list(got[cu[s]:cu[s + 1]]) == omap.latest_wins_ids(list(toks[cu[s]:cu[s + 1]]), atok, False, start[s]), s
+
+
 @pytest.mark.parametrize("lens,rate", [([9217, 40, 1, 3000], 0.001), ([1] * 300, 0.3), ([0, 257, 2100], 0.0)])
 def test_route_latest_wins_in_place(dev, lens, rate):
     """out_ids may be input_ids."""
