@@ -216,11 +216,9 @@ GS_HD bool gemm_tile_mixed(int bid, int full, int halves, int tiles_n, int group
 GS_HD int gemm_b_row(int r, int h) {
   return (r >> 5) * 64 + h * 32 + ((r & 15) >> 2) * 8 + ((r >> 4) & 1) * 4 + (r & 3);
 }
-// Streaming form: the tile column of matrix row i of 16-column block j (of NB):
-// blocks pair up so that a lane's results are 8 consecutive columns.
-GS_HD int gemm_s_brow(int i, int j, int NB) {
-  return NB == 1 ? i : (j >> 1) * 32 + (i >> 2) * 8 + (j & 1) * 4 + (i & 3);
-}
+// Streaming form: the tile column of matrix row i of 16-column block j: blocks
+// pair up so that a lane's results are 8 consecutive columns.
+GS_HD int gemm_s_brow(int i, int j) { return (j >> 1) * 32 + (i >> 2) * 8 + (j & 1) * 4 + (i & 3); }
 // Of `full` chunks, those of wave w of W (chunks w, w + W, ...).
 GS_HD int gemm_s_chunks(int full, int w, int W) { return (full - w + W - 1) / W; }
 // An operand row a thread moves: rows past the matrix re-read its last.

@@ -56,6 +56,11 @@ struct GemmParams {
   int half_rows;          // those of 128
 };
 
+// C's rows start at 16 bytes: a lane stores 8 consecutive columns at once.
+__device__ __forceinline__ bool wide_rows(const GemmParams& p) {
+  return p.ldc % 8 == 0 && (reinterpret_cast<uintptr_t>(p.c) & 15) == 0;
+}
+
 // WM x WN waves over k-tiles of 64 in two LDS stages (one barrier per k-tile);
 // wave (wm, wn) owns rows wm*(256/WM) and columns wn*(256/WN)
 // of the tile as MI x NJ blocks of 32 x 32.
@@ -231,6 +236,9 @@ constexpr int kPRow = kPBK * 2;                 // bytes of one operand row per 
 constexpr int kPHalf = 128 * kPRow;             // one half-operand of one stage
 constexpr int kPStage = 4 * kPHalf;             // A0, A1, B0, B1
 constexpr int64_t kPMaxLd = int64_t(1) << 22;   // a tile's rows stay within 32-bit byte offsets
+constexpr int kPOutRow = 64 * 2 + 16;           // a wave's 64 x 64 results in LDS (rows 16-byte aligned, banks spread)
+constexpr int kPOutWave = 64 * kPOutRow;
+static_assert(8 * kPOutWave <= 2 * kPStage, "the results fit the operand stages");
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
@@ -435,31 +443,68 @@ __device__ __forceinline__ void gemm_tile_pingpong(const GemmParams& p, char* sm
 
   // lane l holds row l % 16 of each 16-row block and columns 8 * (l / 16) .. + 7
   // of each column half
-  const bool wide = p.ldc % 8 == 0 && (reinterpret_cast<uintptr_t>(p.c) & 15) == 0;
-  const int row0 = first_row + wm * 64 + (l & 15);
-  const int col0 = tn * kGBN + wn * 64 + (l >> 4) * 8;
+  auto result = [&](int h, int i, int c) {
+    const f32x4 lo = acc[h][c][i][0], hi = acc[h][c][i][1];
+    return u32x4{pack_bf16x2(lo[0], lo[1]), pack_bf16x2(lo[2], lo[3]), pack_bf16x2(hi[0], hi[1]),
+                 pack_bf16x2(hi[2], hi[3])};
+  };
+  if (wide_rows(p)) {
+    const int row0 = first_row + wm * 64 + (l & 15);
+    const int col0 = tn * kGBN + wn * 64 + (l >> 4) * 8;
 #pragma unroll
-  for (int h = 0; h < NA; ++h)
+    for (int h = 0; h < NA; ++h)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = row0 + h * 128 + i * 16;
-      if (row >= p.M) continue;
-      uint16_t* crow = p.c + static_cast<int64_t>(row) * p.ldc;
+      for (int i = 0; i < 4; ++i) {
+        const int row = row0 + h * 128 + i * 16;
+        if (row >= p.M) continue;
+        uint16_t* crow = p.c + static_cast<int64_t>(row) * p.ldc;
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        const int col = col0 + c * 32;
-        const f32x4 lo = acc[h][c][i][0], hi = acc[h][c][i][1];
-        const u32x4 v = {pack_bf16x2(lo[0], lo[1]), pack_bf16x2(lo[2], lo[3]), pack_bf16x2(hi[0], hi[1]),
-                         pack_bf16x2(hi[2], hi[3])};
-        if (wide && col + 8 <= p.N) {
-          st16(crow + col, v);
-        } else {
+        for (int c = 0; c < 2; ++c) {
+          const int col = col0 + c * 32;
+          const u32x4 v = result(h, i, c);
+          if (col + 8 <= p.N) {
+            st16(crow + col, v);
+          } else {
 #pragma unroll
-          for (int e = 0; e < 8; ++e)
-            if (col + e < p.N) crow[col + e] = static_cast<uint16_t>(v[e >> 1] >> (16 * (e & 1)));
+            for (int e = 0; e < 8; ++e)
+              if (col + e < p.N) crow[col + e] = static_cast<uint16_t>(v[e >> 1] >> (16 * (e & 1)));
+          }
         }
       }
+    return;
+  }
+  // rows of C that do not start at 16 bytes: 2-byte stores of a lane's 8 columns
+  // would scatter over 16 rows each (497 x 26543 x 128 41 us, 6991 x 11479 x 256
+  // 200, 4144 x 4866 x 1024 85), so a wave passes its 64 x 64 results through its
+  // part of the operand stages and stores 64 consecutive columns of a row at a
+  // time (16, 73 and 50 us)
+  lds_barrier();                                // no wave reads the stages, and no transfer lands in them, any more
+  char* const mine = smem + wave * kPOutWave;
+#pragma unroll
+  for (int h = 0; h < NA; ++h) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) st16(mine + (i * 16 + (l & 15)) * kPOutRow + c * 64 + (l >> 4) * 16, result(h, i, c));
+    const int row0 = first_row + h * 128 + wm * 64, col = tn * kGBN + wn * 64 + l;
+    uint16_t* crow = p.c + static_cast<int64_t>(row0) * p.ldc + col;
+    const int rows = min(64, p.M - row0);
+    auto copy = [&](int r, int n) {             // rows r .. r + 15, those below n
+      uint16_t v[16];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) v[u] = *reinterpret_cast<const uint16_t*>(mine + (r + u) * kPOutRow + l * 2);
+#pragma unroll
+      for (int u = 0; u < 16; ++u)
+        if (r + u < n) crow[(r + u) * p.ldc] = v[u];
+    };
+    if (col >= p.N) continue;
+    if (rows == 64) {
+#pragma unroll
+      for (int r = 0; r < 64; r += 16) copy(r, 64);
+    } else {
+      for (int r = 0; r < rows; r += 16) copy(r, rows);
     }
+  }
 }
 
 __global__ __launch_bounds__(512) void gemm_bf16_tn_pingpong_kernel(GemmParams p) {
@@ -501,6 +546,8 @@ __global__ __launch_bounds__(512) void gemm_bf16_tn_pingpong_kernel(GemmParams p
 // ---------------------------------------------------------------------------
 // s_waitcnt for "lgkmcnt <= n"
 constexpr int wait_lds(int n) { return 15 | (7 << 4) | (n << 8) | (3 << 14); }
+constexpr int kSOutRow = 32 * 2 + 16;           // a unit's 16 x 32 results in LDS
+static_assert(16 * kSOutRow <= 2048, "they fit a unit's partial");
 
 template <typename F, int... I>
 __device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
@@ -518,19 +565,18 @@ struct StreamShape {
   static constexpr int TC = (RS + NS - 1) / NS; // chunks at the end whose refills run out
   static constexpr int kSlot = 16 * kPRow;
   static constexpr int kRing = RS * kSlot;      // bytes per wave
-  static constexpr int NP = NB >= 2 ? NB / 2 : 1;   // column units of a row block: 2 (or 1) 16-column blocks
-  static constexpr int UB = NB >= 2 ? 2 : 1;        // blocks per unit
+  static constexpr int NP = NB / 2;                 // column units of a row block: 2 16-column blocks each
   static constexpr int U = MB * NP;
-  static constexpr int kSum = W * U * UB * 1024;    // the partial tiles
+  static constexpr int kSum = W * U * 2048;         // the partial tiles
   static constexpr int kLds = W * kRing > kSum ? W * kRing : kSum;
-  static_assert(NB == 1 || NB % 2 == 0, "column blocks pair up");
+  static_assert(NB % 2 == 0, "column blocks pair up");
   static_assert(RS >= NS && LA >= 1 && LA < NS && kLds <= 160 * 1024, "the ring holds a chunk, LDS holds the rings");
 };
 
 template <int MB, int NB, int W, int RS, int LA>
 __global__ __launch_bounds__(64 * W) void gemm_bf16_tn_stream_kernel(GemmParams p) {
   using S = StreamShape<MB, NB, W, RS, LA>;
-  constexpr int NS = S::NS, NP = S::NP, UB = S::UB, U = S::U, TC = S::TC;
+  constexpr int NS = S::NS, NP = S::NP, U = S::U, TC = S::TC;
   __shared__ __align__(16) char smem[S::kLds];
   int tm, tn;
   if (!addr::gemm_tile(static_cast<int>(blockIdx.x), p.tiles_m, p.tiles_n, p.tiles_m, tm, tn)) return;
@@ -549,7 +595,7 @@ __global__ __launch_bounds__(64 * W) void gemm_bf16_tn_stream_kernel(GemmParams 
       const int r = 8 * t + (l >> 3);
       const uint32_t piece = addr::gemm_piece(l, r) * 16;
       off[s][t] = piece + static_cast<uint32_t>(
-          s < NB ? (addr::gemm_row(tn * 16 * NB + addr::gemm_s_brow(r, s, NB), p.N) - tn * 16 * NB) * p.ldb * 2
+          s < NB ? (addr::gemm_row(tn * 16 * NB + addr::gemm_s_brow(r, s), p.N) - tn * 16 * NB) * p.ldb * 2
                  : (addr::gemm_row(tm * 16 * MB + 16 * (s - NB) + r, p.M) - tm * 16 * MB) * p.lda * 2);
     }
   const char* const basea = p.a + static_cast<int64_t>(tm) * 16 * MB * p.lda * 2;
@@ -640,32 +686,42 @@ __global__ __launch_bounds__(64 * W) void gemm_bf16_tn_stream_kernel(GemmParams 
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
-    for (int j = 0; j < NB; ++j) part[((wave * U + i * NP + j / UB) * UB + j % UB) * 64 + l] = acc[i][j];
+    for (int j = 0; j < NB; ++j) part[((wave * U + i * NP + j / 2) * 2 + j % 2) * 64 + l] = acc[i][j];
   lds_barrier();
-  const bool wide = p.ldc % 8 == 0 && (reinterpret_cast<uintptr_t>(p.c) & 15) == 0;
+  const bool wide = wide_rows(p);
   for (int u = wave; u < U; u += W) {
-    f32x4 v[UB];
+    f32x4 v[2];
 #pragma unroll
-    for (int e = 0; e < UB; ++e) v[e] = part[(u * UB + e) * 64 + l];
+    for (int e = 0; e < 2; ++e) v[e] = part[(u * 2 + e) * 64 + l];
 #pragma unroll
     for (int w = 1; w < W; ++w)
 #pragma unroll
-      for (int e = 0; e < UB; ++e) v[e] += part[((w * U + u) * UB + e) * 64 + l];
-    const int row = tm * 16 * MB + (u / NP) * 16 + i16;
-    const int col = tn * 16 * NB + (u % NP) * 32 + q * 4 * UB;
+      for (int e = 0; e < 2; ++e) v[e] += part[((w * U + u) * 2 + e) * 64 + l];
+    const int row0 = tm * 16 * MB + (u / NP) * 16, col0 = tn * 16 * NB + (u % NP) * 32;
+    const u32x4 o = {pack_bf16x2(v[0][0], v[0][1]), pack_bf16x2(v[0][2], v[0][3]), pack_bf16x2(v[1][0], v[1][1]),
+                     pack_bf16x2(v[1][2], v[1][3])};
+    if (!wide) {
+      // (as in the ping-pong form) through the place of the unit's first
+      // partial, which only this wave reads: 32 consecutive columns of 2 rows a store
+      char* const mine = reinterpret_cast<char*>(part + u * 128);
+      st16(mine + i16 * kSOutRow + q * 16, o);
+      const int col = col0 + (l & 31);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const int r = 2 * k + (l >> 5);
+        const uint16_t x = *reinterpret_cast<const uint16_t*>(mine + r * kSOutRow + (l & 31) * 2);
+        if (row0 + r < p.M && col < p.N) p.c[static_cast<int64_t>(row0 + r) * p.ldc + col] = x;
+      }
+      continue;
+    }
+    const int row = row0 + i16, col = col0 + q * 8;
     if (row >= p.M) continue;
     uint16_t* crow = p.c + static_cast<int64_t>(row) * p.ldc;
-    uint32_t o[2 * UB];
-#pragma unroll
-    for (int e = 0; e < UB; ++e) {
-      o[2 * e] = pack_bf16x2(v[e][0], v[e][1]);
-      o[2 * e + 1] = pack_bf16x2(v[e][2], v[e][3]);
-    }
-    if (UB == 2 && wide && col + 8 <= p.N) {
-      st16(crow + col, u32x4{o[0], o[1], o[2 * UB - 2], o[2 * UB - 1]});
+    if (col + 8 <= p.N) {
+      st16(crow + col, o);
     } else {
 #pragma unroll
-      for (int e = 0; e < 4 * UB; ++e)
+      for (int e = 0; e < 8; ++e)
         if (col + e < p.N) crow[col + e] = static_cast<uint16_t>(o[e >> 1] >> (16 * (e & 1)));
     }
   }
@@ -848,6 +904,27 @@ struct GemmModel {
           }
       }
   }
+  // A wave's results of rows x cols passed through LDS rows of out_row bytes
+  // (rows of C that do not start at 16 bytes): lane l of the writers gives row
+  // l % 16 of each 16-row block 16-byte pieces, the readers take single
+  // columns; each must find its own element.
+  void out_pass(const char* who, int rows, int cols, int out_row, int64_t lds) {
+    std::vector<int> held(lds / 2, -1);
+    for (int i = 0; i < rows / 16; ++i)
+      for (int c = 0; c < cols / 32; ++c)
+        for (int l = 0; l < 64; ++l)
+          for (int e = 0; e < 8; ++e) {
+            const int64_t at = (i * 16 + (l & 15)) * out_row + c * 64 + (l >> 4) * 16 + 2 * e;
+            if (!in(who, at, 2, lds)) continue;
+            if (held[at / 2] >= 0) fail("%s: byte %lld written twice", who, (long long)at);
+            held[at / 2] = (i * 16 + (l & 15)) * cols + c * 32 + (l >> 4) * 8 + e;
+          }
+    for (int r = 0; r < rows; ++r)
+      for (int col = 0; col < cols; ++col) {
+        const int64_t at = r * out_row + col * 2;
+        if (in(who, at, 2, lds) && held[at / 2] != r * cols + col) fail("%s: (%d, %d) is another element", who, r, col);
+      }
+  }
   // gemm_bf16_tn_pingpong_kernel: every workgroup's transfers, operand reads
   // and stores, each tile and each element of C once, and each operand read
   // landing on the rows and columns its result is stored at
@@ -886,6 +963,7 @@ struct GemmModel {
               }
             }
       }
+    out_pass("C through LDS", 64, 64, kPOutRow, kPOutWave);
     const int64_t total = int64_t(slots) * tiles_n, grid = addr::gemm_mixed_grid(full, halves, tiles_n);
     std::vector<char> seen(total, 0);
     for (int64_t b = 0; b < grid; ++b) {
@@ -990,6 +1068,7 @@ struct GemmModel {
         if ((addr::gemm_piece(l, r) ^ addr::lds_swz(r)) != (l & 7)) fail("transfer lands at another piece");
       }
     }
+    out_pass("C unit through LDS", 16, 32, kSOutRow, 2048);
     std::vector<char> cseen(static_cast<size_t>(M) * N, 0);
     const int64_t total = int64_t(tiles_m) * tiles_n;
     for (int64_t b = 0; b < 8 * ((total + 7) / 8); ++b) {
@@ -1001,7 +1080,7 @@ struct GemmModel {
           for (int t = 0; t < 2; ++t) {
             const int r = 8 * t + (l >> 3), piece = addr::gemm_piece(l, r);
             const bool isb = s < f.NB;
-            const int64_t row = isb ? addr::gemm_row(col0 + addr::gemm_s_brow(r, s, f.NB), static_cast<int>(N))
+            const int64_t row = isb ? addr::gemm_row(col0 + addr::gemm_s_brow(r, s), static_cast<int>(N))
                                     : addr::gemm_row(row0 + 16 * (s - f.NB) + r, static_cast<int>(M));
             const int64_t ld = isb ? ldb : lda;
             in("offset in 32 bits", (row - (isb ? col0 : row0)) * ld * 2 + piece * 16, 16, int64_t(1) << 32);
@@ -1013,7 +1092,7 @@ struct GemmModel {
           for (int e = 0; e < 8; ++e) {
             const int row = row0 + (u / NP) * 16 + (l & 15), col = col0 + (u % NP) * 32 + (l >> 4) * 8 + e;
             // element e of the lane: matrix row 4 (l / 16) + e % 4 of block 2 (u % NP) + e / 4
-            if (addr::gemm_s_brow(4 * (l >> 4) + (e & 3), 2 * (u % NP) + (e >> 2), f.NB) != col - col0)
+            if (addr::gemm_s_brow(4 * (l >> 4) + (e & 3), 2 * (u % NP) + (e >> 2)) != col - col0)
               fail("column %d is stored from another B row", col);
             if (row >= M || col >= N) continue;
             in("C", int64_t(row) * ldc + col, 1, (M - 1) * ldc + N);

@@ -73,6 +73,28 @@ def test_gemm_forms_for_few_tiles(dev, M, N, K):
     test_gemm_matches_fp32_reference(dev, M, N, K, M + N + K)
 
 
+@pytest.mark.parametrize("M,N,K,ldc,off", [
+    (497, 2543, 128, 2543, 0),        # odd rows of C, 128-row tiles
+    (300, 301, 256, 302, 0), (1, 255, 128, 255, 0), (129, 257, 192, 261, 0),
+    (4104, 250, 128, 251, 0),         # 256-row tiles, the last of 8 rows
+    (300, 512, 128, 520, 1),          # rows of whole 16 bytes that start off them
+    (7, 4481, 4096, 4481, 0), (27, 9001, 768, 9001, 0), (64, 7295, 1024, 7297, 0), (128, 7294, 576, 7294, 0),
+    (255, 7290, 1152, 7290, 0), (256, 7296, 512, 7304, 3),               # streaming forms
+])
+def test_gemm_rows_of_c_off_16_bytes(dev, M, N, K, ldc, off):
+    """Only C's own elements are written, whatever the alignment of its rows."""
+    g = torch.Generator(device=dev).manual_seed(M + N)
+    x = torch.randn(M, K, generator=g, device=dev).to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g, device=dev) / K ** 0.5).to(torch.bfloat16)
+    buf = torch.full((M * ldc + off + 8,), 7.0, dtype=torch.bfloat16, device=dev)
+    out = buf[off:].as_strided((M, N), (ldc, 1))
+    switched.linear_bf16(x, w, out)
+    _check(out, x, w)
+    written = torch.zeros_like(buf, dtype=torch.bool)
+    written[off:].as_strided((M, N), (ldc, 1)).fill_(True)
+    assert (buf[~written] == 7.0).all()
+
+
 @pytest.mark.parametrize("M,N,K", [(333, 520, 1024), (200, 9000, 640), (900, 7000, 320)])
 def test_gemm_strided_rows_and_output(dev, M, N, K):
     """x and out with row strides (a view into a wider buffer), as the layer's x_ext slices are."""
