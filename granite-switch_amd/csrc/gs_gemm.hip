@@ -688,8 +688,7 @@ __global__ __launch_bounds__(64 * W) void gemm_bf16_tn_stream_kernel(GemmParams 
 #pragma unroll
     for (int j = 0; j < NB; ++j) part[((wave * U + i * NP + j / 2) * 2 + j % 2) * 64 + l] = acc[i][j];
   lds_barrier();
-  const bool wide = wide_rows(p);
-  for (int u = wave; u < U; u += W) {
+  auto sum = [&](int u) {                       // lane l: row l % 16 of the unit, columns 8 * (l / 16) .. + 7
     f32x4 v[2];
 #pragma unroll
     for (int e = 0; e < 2; ++e) v[e] = part[(u * 2 + e) * 64 + l];
@@ -697,32 +696,37 @@ __global__ __launch_bounds__(64 * W) void gemm_bf16_tn_stream_kernel(GemmParams 
     for (int w = 1; w < W; ++w)
 #pragma unroll
       for (int e = 0; e < 2; ++e) v[e] += part[((w * U + u) * 2 + e) * 64 + l];
-    const int row0 = tm * 16 * MB + (u / NP) * 16, col0 = tn * 16 * NB + (u % NP) * 32;
-    const u32x4 o = {pack_bf16x2(v[0][0], v[0][1]), pack_bf16x2(v[0][2], v[0][3]), pack_bf16x2(v[1][0], v[1][1]),
-                     pack_bf16x2(v[1][2], v[1][3])};
-    if (!wide) {
-      // (as in the ping-pong form) through the place of the unit's first
-      // partial, which only this wave reads: 32 consecutive columns of 2 rows a store
-      char* const mine = reinterpret_cast<char*>(part + u * 128);
-      st16(mine + i16 * kSOutRow + q * 16, o);
-      const int col = col0 + (l & 31);
+    return u32x4{pack_bf16x2(v[0][0], v[0][1]), pack_bf16x2(v[0][2], v[0][3]), pack_bf16x2(v[1][0], v[1][1]),
+                 pack_bf16x2(v[1][2], v[1][3])};
+  };
+  if (wide_rows(p)) {
+    for (int u = wave; u < U; u += W) {
+      const u32x4 o = sum(u);
+      const int row = tm * 16 * MB + (u / NP) * 16 + i16;
+      const int col = tn * 16 * NB + (u % NP) * 32 + q * 8;
+      if (row >= p.M) continue;
+      uint16_t* crow = p.c + static_cast<int64_t>(row) * p.ldc;
+      if (col + 8 <= p.N) {
+        st16(crow + col, o);
+      } else {
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const int r = 2 * k + (l >> 5);
-        const uint16_t x = *reinterpret_cast<const uint16_t*>(mine + r * kSOutRow + (l & 31) * 2);
-        if (row0 + r < p.M && col < p.N) p.c[static_cast<int64_t>(row0 + r) * p.ldc + col] = x;
+        for (int e = 0; e < 8; ++e)
+          if (col + e < p.N) crow[col + e] = static_cast<uint16_t>(o[e >> 1] >> (16 * (e & 1)));
       }
-      continue;
     }
-    const int row = row0 + i16, col = col0 + q * 8;
-    if (row >= p.M) continue;
-    uint16_t* crow = p.c + static_cast<int64_t>(row) * p.ldc;
-    if (col + 8 <= p.N) {
-      st16(crow + col, o);
-    } else {
+    return;
+  }
+  // as in the ping-pong form, through the place of the unit's first partial,
+  // which only this wave reads: 32 consecutive columns of 2 rows a store
+  for (int u = wave; u < U; u += W) {
+    char* const mine = reinterpret_cast<char*>(part + u * 128);
+    st16(mine + i16 * kSOutRow + q * 16, sum(u));
+    const int row0 = tm * 16 * MB + (u / NP) * 16, col = tn * 16 * NB + (u % NP) * 32 + (l & 31);
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
-        if (col + e < p.N) crow[col + e] = static_cast<uint16_t>(o[e >> 1] >> (16 * (e & 1)));
+    for (int k = 0; k < 8; ++k) {
+      const int r = 2 * k + (l >> 5);
+      const uint16_t x = *reinterpret_cast<const uint16_t*>(mine + r * kSOutRow + (l & 31) * 2);
+      if (row0 + r < p.M && col < p.N) p.c[static_cast<int64_t>(row0 + r) * p.ldc + col] = x;
     }
   }
 }
