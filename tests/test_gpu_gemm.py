@@ -52,6 +52,7 @@ def test_gemm_matches_fp32_reference(dev, M, N, K, seed):
     (384, 1032, 320),           # full tiles, then thin ones, over two tile columns and a partial one
     (2049, 775, 128),           # one row in the thin row; columns that end inside an 8-column store
     (300, 301, 256),            # rows of C that are not 16-byte aligned
+    (1, 33, 64), (300, 7296, 64), (1025, 257, 64), (128, 264, 64),   # one k-tile
 ])
 def test_gemm_pingpong_tile_edges(dev, M, N, K):
     test_gemm_matches_fp32_reference(dev, M, N, K, M + N)
