@@ -90,6 +90,7 @@ SIGNATURES = {
                                              c_i32, c_void_p, c_i64, c_void_p, c_void_p, c_void_p, c_void_p, c_i32,
                                              c_i32, c_i32, c_void_p]),
     "gs_gemm_bf16_tn": (c_i32, [c_void_p, c_i64, c_void_p, c_i64, c_void_p, c_i64, c_i64, c_i64, c_i64, c_void_p]),
+    "gs_gemm_form": (c_i32, [c_i64, c_i64, c_i64, c_i64, c_i64, c_i32, c_void_p]),
 }
 
 

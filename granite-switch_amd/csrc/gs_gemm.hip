@@ -211,10 +211,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_tn_kernel(GemmParams p
 // that the next phase reads.  So a transfer has ~3000 clocks to arrive.
 //
 // Tile rows of 128 run the two phases of row half 0 only (HALF), at 0.7 of the
-// time; those tiles come last in every XCD's range.  A last tile row of at most
-// 128 rows is one, and as many before it as shorten the last, part-filled
-// round of tiles -- all of them, where 256-row tiles would leave most CUs idle
-// (pick_gemm).
+// time; those tiles come last in every XCD's range.  As many tile rows are such
+// as shorten the last, part-filled round of tiles -- all of them, where 256-row
+// tiles would leave most CUs idle (pick_gemm).  A last tile row of at most 128
+// rows is a 256-row one where that round is no shorter without it.
 //
 // Bound by LDS (64 KB of transfers in at 64 bytes per clock, 192 KB of operand
 // reads at 128: 2560 clocks per k-tile against 2048 of MFMAs; 1.1 us measured)
@@ -754,12 +754,12 @@ const StreamForm kStreamForms[] = {
     stream_form<4, 4, 4, 10, 3>(), stream_form<8, 4, 4, 16, 3>(),
 };
 
-// The form with the fewest clocks per 64 k on the busiest of 256 CUs: tiles
-// per CU times a tile's measured clocks, which follow its LDS time (transfers
-// in at 64 bytes per clock plus operand reads at 128).  A streaming form takes
-// 60 per 2 KB slot (48 of LDS), the 256 x 256 tile 2400, its 128-row form
-// 1700.  The HBM time of the operands is the same for all of them.  Every wave
-// of a streaming form needs TC chunks.
+// The form with the fewest clocks per 64 k on the busiest CU: tiles per CU
+// times a tile's weight, fitted to the forms' measured times (relative weights:
+// 60 for each 2 KB slot of a streaming form, 2400 for the 256 x 256 tile, 1700
+// for its 128-row form; their LDS time, transfers in at 64 bytes per clock plus
+// operand reads at 128, is 48, 2560 and 1792).  The HBM time of the operands is
+// the same for all of them.  Every wave of a streaming form needs TC chunks.
 // Measured, M x 7296 x 4096, us, every form (16*MB x 16*NB) that was close:
 //   M     16 x 32  32 x 32  64 x 32  64 x 64  128 x 64  128 x 256  256 x 256
 //   16      13.2                                                     47
@@ -769,18 +769,18 @@ const StreamForm kStreamForms[] = {
 //   256                                34.8      28.9                76
 //   512                                59.2      50.8                75
 //   777                                83.3      83.2      55        75
-constexpr int64_t kCus = 256, kFullClocks = 2400, kHalfClocks = 1700;
+constexpr int64_t kFullClocks = 2400, kHalfClocks = 1700;
 // Clocks per 64 k of `full` 256-row tiles followed by `halves` 128-row ones on
-// kCus CUs, each taking the next tile when it is free.
-inline int64_t gemm_mixed_clocks(int64_t full, int64_t halves) {
-  const int64_t late = full % kCus, early = kCus - late;        // CUs that run one full tile more, and the others
-  const int64_t t_early = full / kCus * kFullClocks, t_late = t_early + kFullClocks;
+// `cus` CUs, each taking the next tile when it is free.
+inline int64_t gemm_mixed_clocks(int64_t full, int64_t halves, int64_t cus) {
+  const int64_t late = full % cus, early = cus - late;          // CUs that run one full tile more, and the others
+  const int64_t t_early = full / cus * kFullClocks, t_late = t_early + kFullClocks;
   const int64_t end = late > 0 ? t_late : t_early;
   if (halves == 0) return end;
   // halves done once the early CUs have run k: early * k + late * (k - 2) at
   // their k-th end, early * k + late * (k - 1) at the late CUs' next one
   static_assert(kFullClocks > kHalfClocks && kFullClocks < 2 * kHalfClocks, "the order of the two groups' ends");
-  for (int64_t k = std::max<int64_t>(1, halves / kCus - 1);; ++k) {
+  for (int64_t k = std::max<int64_t>(1, halves / cus - 1);; ++k) {
     if (early * k + late * std::max<int64_t>(0, k - 2) >= halves) return std::max(end, t_early + k * kHalfClocks);
     if (early * k + late * (k - 1) >= halves) return std::max(end, t_late + (k - 1) * kHalfClocks);
   }
@@ -793,15 +793,15 @@ struct GemmPick {
 // with 16 full tile rows (304 tiles on 256 CUs, 48 in a second round) and one
 // half row, 392 us with 13 and 7; 4096 x 4480 x 12800 457 -> 381 us, 3333 x
 // 6150 x 4096 200 -> 172.
-inline GemmPick pick_gemm(int64_t M, int64_t N, int64_t K) {
+inline GemmPick pick_gemm(int64_t M, int64_t N, int64_t K, int64_t cus) {
   auto tiles = [&](int64_t tm, int64_t tn) { return ((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
-  auto rounds = [&](int64_t n) { return (n + kCus - 1) / kCus; };
+  auto rounds = [&](int64_t n) { return (n + cus - 1) / cus; };
   const int64_t tiles_m = (M + kGBM - 1) / kGBM, tiles_n = (N + kGBN - 1) / kGBN;
   GemmPick best{nullptr, static_cast<int>(tiles_m)};
   int64_t cost = INT64_MAX;
   // a tile row fewer at a time (16 of them level out any last round)
   for (int64_t f = tiles_m; f >= std::max<int64_t>(0, tiles_m - 16); --f) {
-    const int64_t c = gemm_mixed_clocks(f * tiles_n, addr::gemm_half_rows(M, static_cast<int>(f)) * tiles_n);
+    const int64_t c = gemm_mixed_clocks(f * tiles_n, addr::gemm_half_rows(M, static_cast<int>(f)) * tiles_n, cus);
     if (c < cost) {
       cost = c;
       best.full_rows = static_cast<int>(f);
@@ -1186,7 +1186,7 @@ int gs_gemm_bf16_tn(const void* a, int64_t lda, const void* b, int64_t ldb, void
   const unsigned grid = static_cast<unsigned>(8 * ((total + 7) / 8));
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (pingpong_form(K, lda, ldb)) {
-    const GemmPick pick = pick_gemm(M, N, K);
+    const GemmPick pick = pick_gemm(M, N, K, device_cus());
     if (pick.stream != nullptr) {
       p.tiles_m = static_cast<int>((M + 16 * pick.stream->MB - 1) / (16 * pick.stream->MB));
       p.tiles_n = static_cast<int>((N + 16 * pick.stream->NB - 1) / (16 * pick.stream->NB));
@@ -1205,6 +1205,21 @@ int gs_gemm_bf16_tn(const void* a, int64_t lda, const void* b, int64_t ldb, void
   return GS_OK;
 }
 
+int gs_gemm_form(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int32_t cus, int32_t* form) {
+  const char* who = "gs_gemm_form";
+  GS_CHECK_ARG(M > 0 && N > 0 && K > 0 && cus >= 0 && form != nullptr, "%s: sizes", who);
+  if (!pingpong_form(K, lda, ldb)) {
+    form[0] = GS_GEMM_REGISTER;
+    form[1] = form[2] = kGBM;
+    return GS_OK;
+  }
+  const GemmPick pick = pick_gemm(M, N, K, cus > 0 ? cus : device_cus());
+  form[0] = pick.stream != nullptr ? GS_GEMM_STREAM : GS_GEMM_PINGPONG;
+  form[1] = pick.stream != nullptr ? 16 * pick.stream->MB : pick.full_rows;
+  form[2] = pick.stream != nullptr ? 16 * pick.stream->NB : addr::gemm_half_rows(M, pick.full_rows);
+  return GS_OK;
+}
+
 int64_t gs_check_gemm_addresses(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, char* msg,
                                 int64_t msg_len, int64_t* checked) {
   const char* who = "gs_check_gemm_addresses";
@@ -1219,7 +1234,7 @@ int64_t gs_check_gemm_addresses(int64_t M, int64_t N, int64_t K, int64_t lda, in
   m.tiles_m = static_cast<int>((M + kGBM - 1) / kGBM);
   m.tiles_n = static_cast<int>((N + kGBN - 1) / kGBN);
   if (pingpong_form(K, lda, ldb)) {
-    std::set<int> forms = {m.tiles_m, m.tiles_m - 1, m.tiles_m / 2, 0, pick_gemm(M, N, K).full_rows};
+    std::set<int> forms = {m.tiles_m, m.tiles_m - 1, m.tiles_m / 2, 0, pick_gemm(M, N, K, 256).full_rows};
     for (int full : forms) m.pingpong(full);
     for (const StreamForm& f : kStreamForms)
       if (K / kPBK / f.W >= (f.RS + f.MB + f.NB - 1) / (f.MB + f.NB)) m.stream(f);

@@ -485,6 +485,15 @@ int gs_switch_lora_shrink_expand(void* out, int32_t out_dtype, int64_t stride_om
  * ---------------------------------------------------------------------- */
 int gs_gemm_bf16_tn(const void* a, int64_t lda, const void* b, int64_t ldb, void* c, int64_t ldc, int64_t M,
                     int64_t N, int64_t K, void* stream);
+/* The kernel that such a call takes on `cus` compute units (0: the current
+ * device's): form[0] GS_GEMM_REGISTER (form[1], form[2] its tile), GS_GEMM_STREAM
+ * (its tile) or GS_GEMM_PINGPONG (tile rows of 256, then of 128 rows).  The
+ * streaming form sums K in four interleaved parts, the others in order, so a
+ * row's bits may depend on how many rows the call has. */
+#define GS_GEMM_REGISTER 0
+#define GS_GEMM_PINGPONG 1
+#define GS_GEMM_STREAM 2
+int gs_gemm_form(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int32_t cus, int32_t* form);
 
 /* Test support (no counterpart in the reference; makes no HIP call).  Replays
  * on the host every global and LDS access of gs_gemm_bf16_tn's kernels for

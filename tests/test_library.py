@@ -323,6 +323,21 @@ def test_bitmask_kernel_choice(M, na, modules, block_m, table):
     assert switched._lib.load().gs_bitmask_table_form(M, na + 1, modules, block_m) == int(table)
 
 
+def _gemm_form(M, N, K, cus, ld=None):
+    out = (ctypes.c_int32 * 3)()
+    assert switched._lib.load().gs_gemm_form(M, N, K, ld or K, ld or K, cus, out) == 0
+    return tuple(out)
+
+
+def test_gemm_form_follows_the_compute_units():
+    """The rounds of tiles that the choice counts are the device's, not those of one chip."""
+    assert _gemm_form(4144, 4864, 12800, 256) == (1, 13, 7)
+    assert _gemm_form(2048, 4864, 12800, 256) == (1, 8, 0) and _gemm_form(2048, 4864, 12800, 128) == (1, 6, 4)
+    assert _gemm_form(200, 9000, 640, 256) == (2, 64, 64) and _gemm_form(200, 9000, 640, 128) == (1, 0, 2)
+    assert _gemm_form(256, 7296, 4096, 0) == _gemm_form(256, 7296, 4096, 256)      # no device here: 256 of them
+    assert _gemm_form(300, 7296, 1000, 256) == (0, 256, 256) and _gemm_form(300, 7296, 4096, 256, 1 << 23) == (0, 256, 256)
+
+
 def test_host_tables_follow_the_pack():
     """The tables kept with a pack are made again after any field they follow
     from changes, in place or by assignment; the class views after a device
