@@ -8,6 +8,8 @@ one bf16 step away from the reference's rounding: tolerance 2^-7 relative plus
 
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 
@@ -25,6 +27,16 @@ def _check(got, x, w):
     err = (got.float() - ref).abs()
     bad = err > 2.0 ** -7 * ref.abs() + 1e-5
     assert not bool(bad.any()), f"{int(bad.sum())} elements off, max abs err {float(err.max()):.3e}"
+
+
+REGISTER, PINGPONG, STREAM = 0, 1, 2
+
+
+def _form(M, N, K, cus=256, ld=None):
+    """(kernel, its tile -- or the ping-pong form's tile rows of 256 and of 128) of a call on ``cus`` compute units."""
+    out = (ctypes.c_int32 * 3)()
+    assert switched._lib.load().gs_gemm_form(M, N, K, ld or K, ld or K, cus, out) == 0
+    return tuple(out)
 
 
 @pytest.mark.parametrize("M,N,K,seed", [
@@ -45,55 +57,44 @@ def test_gemm_matches_fp32_reference(dev, M, N, K, seed):
     _check(got, x, w)
 
 
-@pytest.mark.parametrize("M,N,K", [
-    (256, 256, 128),            # the two k-tiles that the direct-to-LDS form's stages hold, nothing left to issue
-    (128, 264, 192),            # a thin last tile row alone; an odd number of k-tiles
-    (385, 520, 256),            # a thin tile row of one row more than half a tile is not thin: 256 + 129
-    (384, 1032, 320),           # full tiles, then thin ones, over two tile columns and a partial one
-    (2049, 775, 128),           # one row in the thin row; columns that end inside an 8-column store
-    (300, 301, 256),            # rows of C that are not 16-byte aligned
-    (1, 33, 64), (300, 7296, 64), (1025, 257, 64), (128, 264, 64),   # one k-tile
+@pytest.mark.parametrize("M,N,K,halves", [
+    (256, 256, 128, 2),          # the two k-tiles that the direct-to-LDS form's stages hold
+    (128, 264, 192, 1),          # a full tile row; an odd number of k-tiles
+    (385, 520, 256, 4),          # the last tile row of one row
+    (384, 1032, 320, 3),         # full tile rows over four tile columns and a partial one
+    (2049, 775, 128, 17),        # columns that end inside an 8-column store
+    (300, 301, 256, 3),          # rows of C that are not 16-byte aligned
+    (1, 33, 64, 1), (300, 7296, 64, 3), (1025, 257, 64, 9), (128, 264, 64, 1),   # one k-tile
+    (777, 7296, 256, 7), (1100, 6001, 192, 9), (129, 300, 128, 2),
 ])
-def test_gemm_pingpong_tile_edges(dev, M, N, K):
+def test_gemm_pingpong_128_row_tiles(dev, M, N, K, halves):
+    assert _form(M, N, K) == (PINGPONG, 0, halves)
     test_gemm_matches_fp32_reference(dev, M, N, K, M + N)
 
 
-@pytest.mark.parametrize("M,N,K", [
-    # streaming forms, K from the fewest chunks a wave may have to uneven shares of them; ragged rows and columns
-    (1, 33, 1088), (7, 4480, 4096), (16, 45, 1024),                   # 16 x 32 tiles
-    (32, 7296, 1088), (27, 9001, 768),                                # 32 x 32
-    (64, 7296, 1024), (49, 8003, 576),                                # 64 x 32
-    (128, 7296, 576), (113, 16000, 512), (70, 14989, 1344),           # 64 x 64
-    (256, 7296, 512), (255, 7290, 1152), (300, 6149, 832),            # 128 x 64
-    # 128-row tiles of the ping-pong form (too few 256-row ones to fill the CUs)
-    (777, 7296, 256), (1100, 6001, 192), (129, 300, 128),
-    # 256-row tiles, then 128-row ones that level out the last round: a ragged last row, ragged columns
-    (4144, 4864, 128), (2500, 8450, 192), (3333, 6150, 128),
+@pytest.mark.parametrize("M,N,K,full,halves", [
+    # 256-row tiles alone, the last of 8 rows (its second half past M) and of 200
+    (4104, 256, 128, 17, 0), (4104, 250, 64, 17, 0), (4104, 250, 192, 17, 0), (4296, 256, 128, 17, 0),
+    (4296, 250, 320, 17, 0), (4360, 512, 64, 18, 0),
+    # then 128-row ones that level out the last round: a ragged last row, ragged columns
+    (4144, 4864, 128, 13, 7), (2500, 8450, 192, 7, 6), (3333, 6150, 128, 10, 7), (700, 30001, 64, 2, 2),
 ])
-def test_gemm_forms_for_few_tiles(dev, M, N, K):
+def test_gemm_pingpong_256_row_tiles(dev, M, N, K, full, halves):
+    assert _form(M, N, K) == (PINGPONG, full, halves)
     test_gemm_matches_fp32_reference(dev, M, N, K, M + N + K)
 
 
-@pytest.mark.parametrize("M,N,K,ldc,off", [
-    (497, 2543, 128, 2543, 0),        # odd rows of C, 128-row tiles
-    (300, 301, 256, 302, 0), (1, 255, 128, 255, 0), (129, 257, 192, 261, 0),
-    (4104, 250, 128, 251, 0),         # 256-row tiles, the last of 8 rows
-    (300, 512, 128, 520, 1),          # rows of whole 16 bytes that start off them
-    (7, 4481, 4096, 4481, 0), (27, 9001, 768, 9001, 0), (64, 7295, 1024, 7297, 0), (128, 7294, 576, 7294, 0),
-    (255, 7290, 1152, 7290, 0), (256, 7296, 512, 7304, 3),               # streaming forms
+@pytest.mark.parametrize("M,N,K,tile", [
+    # streaming forms, K from the fewest chunks a wave may have to uneven shares of them; ragged rows and columns
+    (1, 33, 1088, (16, 32)), (7, 4480, 4096, (16, 32)), (16, 45, 1024, (16, 32)),
+    (32, 7296, 1088, (32, 32)), (27, 9001, 768, (32, 32)),
+    (64, 7296, 1024, (64, 32)), (49, 8003, 576, (64, 32)),
+    (128, 7296, 576, (64, 64)), (300, 6149, 832, (64, 64)),
+    (113, 16000, 512, (128, 64)), (70, 14989, 1344, (128, 64)), (256, 7296, 512, (128, 64)), (255, 7290, 1152, (128, 64)),
 ])
-def test_gemm_rows_of_c_off_16_bytes(dev, M, N, K, ldc, off):
-    """Only C's own elements are written, whatever the alignment of its rows."""
-    g = torch.Generator(device=dev).manual_seed(M + N)
-    x = torch.randn(M, K, generator=g, device=dev).to(torch.bfloat16)
-    w = (torch.randn(N, K, generator=g, device=dev) / K ** 0.5).to(torch.bfloat16)
-    buf = torch.full((M * ldc + off + 8,), 7.0, dtype=torch.bfloat16, device=dev)
-    out = buf[off:].as_strided((M, N), (ldc, 1))
-    switched.linear_bf16(x, w, out)
-    _check(out, x, w)
-    written = torch.zeros_like(buf, dtype=torch.bool)
-    written[off:].as_strided((M, N), (ldc, 1)).fill_(True)
-    assert (buf[~written] == 7.0).all()
+def test_gemm_streaming_forms(dev, M, N, K, tile):
+    assert _form(M, N, K) == (STREAM, *tile)
+    test_gemm_matches_fp32_reference(dev, M, N, K, M + N + K)
 
 
 @pytest.mark.parametrize("M,N,K", [(333, 520, 1024), (200, 9000, 640), (900, 7000, 320)])
