@@ -68,38 +68,52 @@ GS_HD int64_t reg_a_elem(bool ok, int j, int64_t astep_elems, int64_t kp, int64_
 GS_HD int64_t reg_x_elem(bool ok, int64_t kp, int64_t k_lo) { return ok ? kp : k_lo; }
 
 // ---- expand (expand_kernel, expand_sparse_kernel) --------------------------
+// An expand launch cuts the (tile, sub-tile) pairs of `total` tiles in one of two
+// ways.  Whole parts (xcd_item): every XCD takes whole tiles, every tile is cut
+// into expand_groups equal parts (part g: expand_part), a workgroup has one.
+// Spans (expand_span): the pairs in tile order, an eighth of them to each XCD
+// and equal shares of that to its workgroups, which may cross into next tiles.
+
+// Parts per tile: as many as keep 8 * ceil(total / 8) * groups within wt
+// workgroups, 1 .. n_sub.
+GS_HD int expand_groups(int total, int n_sub, int wt) {
+  const int t8 = 8 * ((total + 7) / 8);
+  int g = t8 > 0 ? wt / t8 : n_sub;
+  if (g > n_sub) g = n_sub;
+  if (g < 1) g = 1;
+  return g;
+}
+GS_HD void expand_part(int g, int groups, int n_sub, int& sub, int& count) {
+  sub = (g * n_sub) / groups;
+  count = ((g + 1) * n_sub) / groups - sub;
+}
 // Part i of `parts` near-equal contiguous ranges of n items: [lo, lo + count).
 GS_HD void even_range(int n, int parts, int i, int& lo, int& count) {
   const int q = n / parts, r = n - q * parts;
   lo = i * q + imin(i, r);
   count = q + (i < r ? 1 : 0);
 }
-// The sub-tiles of workgroup b of an expand launch of `grid` (a multiple of 8)
-// workgroups: `count` from sub-tile `sub` of tile `tile` on, tile after tile, of
-// `total` tiles (count 0: none).  XCD b % 8 takes an eighth of them, its
-// workgroups near-equal shares of that.  With
-// whole groups, every XCD takes whole tiles and every tile is cut into as many
-// equal spans as fit, so that no span crosses into a second tile: always (the
-// grid then holds 8 * ceil(total / 8)), or from kExpandWholeTiles tiles on
-// while the grid holds them.
-enum ExpandCut { kCutSpans, kCutWholeFrom64, kCutWhole };
-constexpr int kExpandWholeTiles = 64;
-GS_HD void expand_span(int b, int grid, int total, int n_sub, ExpandCut cut, int& tile, int& sub, int& count) {
-  const int tpx = (total + 7) >> 3;
-  if (total > 0 && (cut == kCutWhole || (cut == kCutWholeFrom64 && total >= kExpandWholeTiles && 8 * tpx <= grid))) {
-    const int groups = imin(grid / (8 * tpx), n_sub);
-    const int j = b >> 3, g = j / tpx;
-    tile = (b & 7) * tpx + j - g * tpx;
-    sub = (g * n_sub) / groups;
-    count = g < groups && tile < total ? ((g + 1) * n_sub) / groups - sub : 0;
-    return;
-  }
+// The span of workgroup b of `grid` (a multiple of 8): `count` sub-tiles from
+// sub-tile `sub` of tile `tile` on (count 0: none).
+GS_HD void expand_span(int b, int grid, int total, int n_sub, int& tile, int& sub, int& count) {
   int xlo, xn;
   even_range(total * n_sub, 8, b & 7, xlo, xn);
   int lo;
   even_range(xn, grid >> 3, b >> 3, lo, count);
   tile = (xlo + lo) / n_sub;
   sub = xlo + lo - tile * n_sub;
+}
+// Whether spans pay: the mean share is shorter than the longest part by at least
+// 3/2 sub-tiles, what the start of a second tile costs.
+GS_HD bool expand_spans_pay(int grid, int total, int n_sub) {
+  const int groups = expand_groups(total, n_sub, grid);
+  return (2 * ((n_sub + groups - 1) / groups) - 3) * grid >= 2 * total * n_sub;
+}
+// Whether a launch of `grid` workgroups that may walk takes spans: for the tile
+// counts that the host found (span_lo .. span_hi), or with more tiles than
+// workgroups.
+GS_HD bool expand_takes_spans(int grid, int total, int span_lo, int span_hi) {
+  return (total >= span_lo && total <= span_hi) || 8 * ((total + 7) >> 3) > grid;
 }
 // First output column of the lane's 16-byte y piece in sub-tile sub of NT
 // columns (the last piece of a partial sub-tile re-reads the row's last one).

@@ -496,21 +496,16 @@ __global__ __launch_bounds__(kThreads) void reduce_parts_kernel(const float* __r
 }
 
 // ----------------------------------------------------------------------------
-// Expand.  The batch's (tile, column sub-tile of NT columns) pairs, tile by
-// tile (a tile is up to 32 slots of one adapter), are cut into one contiguous
-// span per workgroup of a launch that fills the GPU once (addr::expand_span):
-// an eighth of them to each XCD, so an adapter's tiles mostly share an L2, and
-// equal shares to its workgroups.  A span mostly lies inside one tile, whose
-// start -- the tile lookup and the staging of its shrink values -- is then
-// paid once per workgroup; one that crosses into the next tile pays it again.
-// Whole column groups per tile in place of spans left workgroup slots without
-// work and XCDs with fewer tiles than others: 4096 rows x 4096 of 48 adapters
-// 17.5 -> 16.1 us, 256 x 6144 of 12 (13 tiles) 7.0 -> 6.3, and 22.2 -> 18.6
-// in the pair expand.  The 256-column form, whose start costs about three of
-// its sub-tiles, keeps whole groups (in the pair expand from 64 tiles on): 125
-// tiles x 4096 16.2 us against 17.0, x 25600 82.5 against 84.5 with spans.  From there it is bound by the y stream: 4500 rows x 25600
-// take 97 us, 4.76 TB/s read + written, the rate of a bare read-modify-write
-// of the same rows (4.7 TB/s).
+// Expand.  The batch's (tile, column sub-tile of NT columns) pairs (a tile is up
+// to 32 slots of one adapter) are cut for one round of workgroups: every tile
+// into as many equal parts as fit, one part to a workgroup, each XCD whole
+// tiles.  A part's start -- the tile lookup and the staging of its shrink values
+// -- is paid once, and an adapter's tiles share an L2.  Where that leaves many
+// workgroups without work (264 tiles on 1024 workgroups: 3 parts each), spans of
+// equal length that cross into next tiles, and pay their start again, are the
+// shorter ones (expand_span_range).  From there it is bound by the y stream:
+// 4500 rows x 25600 take 97 us, 4.76 TB/s read + written, the rate of a bare
+// read-modify-write of the same rows (4.7 TB/s).
 // The tile's shrink values for every slice (z rows, or the sum of
 // the split-K partials rounded to the element type exactly like a
 // materialised z) are staged in LDS once.  Per sub-tile each wave computes NBW
@@ -538,6 +533,8 @@ struct ExpandParams {
   const int32_t* ranks;
   int NA;
   int max_rank;
+  int wt;                 // workgroups that fill the GPU once; those of the launch where it walks
+  int span_lo, span_hi;   // tile counts for which a launch that may walk takes spans
   const int32_t* seg;
   const int32_t* perm;
   RankWindow rw;          // adapters of this launch's rank class
@@ -630,7 +627,7 @@ struct NoHook {
 template <bool BF16, int NBW, int PRE, bool PIPE, typename Hook = NoHook>
 __device__ __forceinline__ void expand_item(const ExpandParams& p, const TileRef& tr, int sub0, int nsub,
                                             int nparts, float (&dtile)[kTM][4 * NBW * 32 + kOutPad], char* zs,
-                                            Hook before_last = Hook{}) {
+                                            int tid, Hook before_last = Hook{}) {
   constexpr int NT = 4 * NBW * 32;           // columns per sub-tile
   // read-modify-write mapping: each lane owns one 16-byte piece per row it
   // touches, consecutive lanes consecutive pieces, so every wave access
@@ -648,7 +645,6 @@ __device__ __forceinline__ void expand_item(const ExpandParams& p, const TileRef
   constexpr bool YNT = NBW == 2;
 
   const int r = tr.rank;
-  const int tid = threadIdx.x;
   const int wave = tid >> 6;
   const int l = tid & 63;
   const int i = l & 31;
@@ -827,38 +823,44 @@ __device__ __forceinline__ void expand_item(const ExpandParams& p, const TileRef
   compute(sub0 + nsub - 1, bc, yc);
 }
 
-// The cut of an expand launch: whole groups for the 256-column form (one item
-// per workgroup, compiled without the walk), which in the pair expand takes
-// spans below 64 tiles.
-constexpr addr::ExpandCut expand_cut(int NBW, bool pair) {
-  return NBW == 1 ? addr::kCutSpans : (pair ? addr::kCutWholeFrom64 : addr::kCutWhole);
-}
+// The expand kernels of whole parts are compiled without the walk (kOneItem),
+// whose second item costs registers; the pair expand always has it.
+enum ExpandWalk { kOneItem, kWalk };
 
-// A workgroup's span of the launch (addr::expand_span).  before_last() runs
-// before the span's last sub-tile's products.
-template <bool BF16, int NBW, int PRE, bool PAIR, typename Hook = NoHook>
+// A workgroup's part or span of a launch that may walk.  before_last() runs
+// before its last sub-tile's products.
+template <bool BF16, int NBW, int PRE, typename Hook = NoHook>
 __device__ __forceinline__ void expand_walk(const ExpandParams& p, float (&dtile)[kTM][4 * NBW * 32 + kOutPad],
                                             char* zs, Hook before_last = Hook{}) {
   constexpr int NT = 4 * NBW * 32;
   const int n_sub = (p.out_total + NT - 1) / NT;
-  int tile = 0, left = 0, sub = 0, total = 0;
-  TileRef tr = locate_item<kTM, kExpandBalanced>(p.seg, p.ranks, p.b_off, p.NA, p.rw,
-                                                 [&](int tot) {
-                                                   int first;
-                                                   addr::expand_span(static_cast<int>(blockIdx.x),
-                                                                     static_cast<int>(gridDim.x), tot, n_sub,
-                                                                     expand_cut(NBW, PAIR), tile, first, left);
-                                                   return XcdItem{left > 0 ? tile : -1, first};
-                                                 }, sub, total);
-  if (left <= 0) return;
-  if constexpr (expand_cut(NBW, PAIR) == addr::kCutWhole) {
-    expand_item<BF16, NBW, PRE, false>(p, tr, sub, left, p.nparts, dtile, zs, before_last);
-    return;
-  }
+  int tile = 0, left = 0, sub = 0, total = 0, groups = 0;
+  TileRef tr = locate_item<kTM, kExpandBalanced>(
+      p.seg, p.ranks, p.b_off, p.NA, p.rw,
+      [&](int tot) {
+        const int b = static_cast<int>(blockIdx.x);
+        if (addr::expand_takes_spans(p.wt, tot, p.span_lo, p.span_hi)) {
+          int first;
+          addr::expand_span(b, p.wt, tot, n_sub, tile, first, left);
+          return XcdItem{left > 0 ? tile : -1, first};
+        }
+        groups = addr::expand_groups(tot, n_sub, p.wt);
+        return xcd_item(b, tot, groups);
+      },
+      sub, total);
+  if (tr.g == 0) return;
+  if (groups > 0) addr::expand_part(sub, groups, n_sub, sub, left);
+  // (the same in every lane: in scalar registers across the items)
+  left = __builtin_amdgcn_readfirstlane(left);
+  tile = __builtin_amdgcn_readfirstlane(tile);
   for (;;) {
     const int n = min(left, n_sub - sub);
     left -= n;
-    expand_item<BF16, NBW, PRE, false>(p, tr, sub, n, p.nparts, dtile, zs, [&]() {
+    // (what the lanes derive from their number is worked out again for each
+    // item: kept across them it took the registers of the rank-64 form)
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    expand_item<BF16, NBW, PRE, false>(p, tr, sub, n, p.nparts, dtile, zs, tid, [&]() {
       if (left == 0) before_last();
     });
     if (left == 0) return;
@@ -868,21 +870,36 @@ __device__ __forceinline__ void expand_walk(const ExpandParams& p, float (&dtile
   }
 }
 
-// LOOP = false: the workgroups' spans.  LOOP = true (a rank class expected to
-// hold few tiles, laid out flat with one sub-tile per item, grid capped at one
-// round): a workgroup takes items blockIdx.x, + gridDim.x, ... while they lie
-// in the batch's item range.
+// LOOP = false: the workgroups' parts or spans (WALK).  LOOP = true (a rank
+// class expected to hold few tiles, laid out flat with one sub-tile per item,
+// grid capped at one round): a workgroup takes items blockIdx.x, + gridDim.x, ...
+// while they lie in the batch's item range.
 // The narrow bf16 forms up to rank 64 hold 4 workgroups per CU (<= 128
 // registers per lane; the rank-64 multiswitch projection measured faster at
 // 4 than at 3).
-template <bool BF16, int NBW, int PRE, bool LOOP>
+template <bool BF16, int NBW, int PRE, bool LOOP, ExpandWalk WALK = kOneItem>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BF16 && NBW == 1 && PRE <= 4 && !LOOP ? 4 : 1)))
 void expand_kernel(ExpandParams p) {
   constexpr int NT = 4 * NBW * 32;
   __shared__ float dtile[kTM][NT + kOutPad];
   extern __shared__ __align__(16) char zs[];   // [32][S*max_rank + 8] element type
   if constexpr (!LOOP) {
-    expand_walk<BF16, NBW, PRE, false>(p, dtile, zs);
+    if constexpr (WALK == kWalk) {
+      expand_walk<BF16, NBW, PRE>(p, dtile, zs);
+    } else {
+      const int n_sub = (p.out_total + NT - 1) / NT;
+      int sub = 0, groups = 1, total = 0;
+      const TileRef tr = locate_tile_by<kTM, kExpandBalanced>(p.seg, p.ranks, p.b_off, p.NA, p.rw,
+                                                              static_cast<int>(blockIdx.x), false,
+                                                              [&](int tot) {
+                                                                groups = addr::expand_groups(tot, n_sub, p.wt);
+                                                                return groups;
+                                                              }, sub, total);
+      if (tr.g == 0) return;
+      int sub0, count;
+      addr::expand_part(sub, groups, n_sub, sub0, count);
+      if (count > 0) expand_item<BF16, NBW, PRE, false>(p, tr, sub0, count, p.nparts, dtile, zs, threadIdx.x);
+    }
     return;
   }
   const int n_sub = (p.out_total + NT - 1) / NT;
@@ -899,7 +916,7 @@ void expand_kernel(ExpandParams p) {
   }
   const int items = work_items(total, n_sub, true);
   for (;;) {
-    if (tr.g != 0) expand_item<BF16, NBW, PRE, true>(p, tr, sub, 1, nparts, dtile, zs);
+    if (tr.g != 0) expand_item<BF16, NBW, PRE, true>(p, tr, sub, 1, nparts, dtile, zs, threadIdx.x);
     lin += static_cast<int>(gridDim.x);
     if (lin >= items) break;
     lds_barrier();                         // every wave is done with zs and dtile before the next item
@@ -1286,7 +1303,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   // the first claim goes out before the small class's last sub-tile, so its
   // round trip passes while that sub-tile is computed; its result is written
   // to LDS only afterwards (no wait for it before)
-  expand_walk<true, NBW, PRE, true>(p0, dtile, zs, [&]() {
+  expand_walk<true, NBW, PRE>(p0, dtile, zs, [&]() {
     if (threadIdx.x == 0) ticket = claim_next(claim);
     early = true;
   });
@@ -1608,13 +1625,45 @@ int prepare_expand(ExpandParams& p, const char* who, int32_t dtype, void* y, int
   return GS_OK;
 }
 
-// Workgroups of a column-split expand launch: one round (wt), at most one per
-// (tile slot, sub-tile), a multiple of 8 (addr::expand_span); cut into whole
-// groups, one per tile slot when those alone exceed a round.
-int64_t expand_grid(int64_t wt, int max_tiles, int64_t n_sub, addr::ExpandCut cut) {
+// Workgroups of a column-split expand launch, a multiple of 8: one round (wt),
+// at most one per (tile slot, sub-tile); without a walk one per tile slot when
+// those alone exceed a round.
+int64_t expand_grid(int64_t wt, int max_tiles, int64_t n_sub, bool walks) {
   const int64_t t8 = (static_cast<int64_t>(max_tiles) + 7) / 8 * 8;
-  if (cut == addr::kCutWhole) return (std::min<int64_t>(std::max(wt, t8), t8 * n_sub) + 7) / 8 * 8;
+  return (std::min<int64_t>(walks ? wt : std::max(wt, t8), t8 * n_sub) + 7) / 8 * 8;
+}
+// ... of the flat form, a round of workgroups that loop over the items.
+int64_t expand_flat_grid(int64_t wt, int max_tiles, int64_t n_sub) {
   return (std::min<int64_t>(wt, static_cast<int64_t>(max_tiles) * n_sub) + 7) / 8 * 8;
+}
+// The tile counts for which a launch of 128-column sub-tiles takes spans: those
+// next to the count that T tokens of so many adapters are expected to fill for
+// which spans pay too (the kernel compares: the rule itself, in every
+// workgroup's first chain, took 0.8 us); none (hi 0) if they don't pay there.
+struct SpanRange {
+  int lo = 1, hi = 0;
+};
+SpanRange expand_span_range(int64_t grid, int64_t T, int adapters, int max_tiles, int64_t n_sub) {
+  SpanRange s;
+  const int64_t est = std::min<int64_t>(max_tiles, std::max<int64_t>(std::min<int64_t>(T, adapters),
+                                                                     (T + kTM - 1) / kTM + adapters / 2));
+  auto pays = [&](int64_t tiles) {
+    return 8 * ((tiles + 7) / 8) <= grid &&
+           addr::expand_spans_pay(static_cast<int>(grid), static_cast<int>(tiles), static_cast<int>(n_sub));
+  };
+  if (est < 1 || !pays(est)) return s;
+  s.lo = s.hi = static_cast<int>(est);
+  while (s.lo > 1 && s.lo > est / 2 && pays(s.lo - 1)) --s.lo;
+  while (s.hi < max_tiles && s.hi < 2 * est && pays(s.hi + 1)) ++s.hi;
+  return s;
+}
+// The kernel that walks (compiled for bf16 ranks up to 64): where spans pay for
+// the expected tiles, or there may be more tiles than workgroups.  Rank 64, 24
+// adapters: 8192 x 16384 209 -> 176 us, x 6144 122 -> 111, x 4096 55.4 -> 51.2.
+// Spans where they don't pay: 1500 x 16384 49.2 -> 53.7, 2767 x 4096 30.7 -> 33.2,
+// 1 x 4096 9.9 -> 10.6.
+bool expand_walks(bool bf16, int NBW, int PRE, int64_t wt, int max_tiles, const SpanRange& s) {
+  return bf16 && NBW == 1 && PRE <= 4 && (s.hi > 0 || max_tiles > wt);
 }
 
 // Workgroups of a rank-split (sparse) expand launch: one round, at most one
@@ -1623,36 +1672,51 @@ int64_t sparse_grid(int64_t wt, int max_tiles, int64_t n_sub) {
   return std::max<int64_t>(1, std::min<int64_t>(wt, static_cast<int64_t>(max_tiles) * n_sub));
 }
 
-template <bool BF16, int NBW, int PRE>
-void launch_expand_t(int max_tiles, size_t lds, ExpandParams p, hipStream_t st) {
-  auto kern = p.flat ? expand_kernel<BF16, NBW, PRE, true> : expand_kernel<BF16, NBW, PRE, false>;
-  if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-  // workgroups resident per CU for this LDS size, queried once per size and
-  // kernel form and kept as one word (lds << 16 | count) so concurrent
-  // callers read a consistent pair
-  static std::atomic<uint64_t> occ_of[2];
-  std::atomic<uint64_t>& occ = occ_of[p.flat ? 1 : 0];
+// Workgroups of `kern` resident per CU at this LDS size, queried once per size
+// and kept as one word (lds << 16 | count) so concurrent callers read a
+// consistent pair.
+int64_t expand_occupancy(const void* kern, size_t lds, std::atomic<uint64_t>& occ) {
+  if (lds > 64 * 1024) (void)hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
   uint64_t o = occ.load(std::memory_order_relaxed);
   if (o == 0 || (o >> 16) != lds) {
     int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void*>(kern), kThreads, lds) != hipSuccess || n < 1) n = 1;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kern, kThreads, lds) != hipSuccess || n < 1) n = 1;
     o = (static_cast<uint64_t>(lds) << 16) | static_cast<uint64_t>(std::min(n, 0xffff));
     occ.store(o, std::memory_order_relaxed);
   }
+  return static_cast<int64_t>(o & 0xffff);
+}
+
+template <bool BF16, int NBW, int PRE>
+void launch_expand_t(int64_t T, int adapters, size_t lds, ExpandParams p, hipStream_t st) {
   constexpr int NT = 4 * NBW * 32;
-  const int grid = static_cast<int>(expand_grid(static_cast<int64_t>(o & 0xffff) * device_cus(), max_tiles,
-                                                (p.out_total + NT - 1) / NT,
-                                                p.flat ? addr::kCutSpans : expand_cut(NBW, false)));
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(kThreads), lds, st, p);
+  const int64_t n_sub = (p.out_total + NT - 1) / NT;
+  const int max_tiles = max_tiles_for(T, adapters);
+  static std::atomic<uint64_t> occ[3];
+  auto kern = p.flat ? expand_kernel<BF16, NBW, PRE, true> : expand_kernel<BF16, NBW, PRE, false>;
+  int64_t wt = expand_occupancy(reinterpret_cast<const void*>(kern), lds, occ[p.flat ? 1 : 0]) * device_cus();
+  int64_t grid = p.flat ? expand_flat_grid(wt, max_tiles, n_sub) : expand_grid(wt, max_tiles, n_sub, false);
+  if constexpr (BF16 && NBW == 1 && PRE <= 4) {
+    const SpanRange sr = expand_span_range(grid, T, adapters, max_tiles, n_sub);
+    if (!p.flat && expand_walks(BF16, NBW, PRE, wt, max_tiles, sr)) {
+      kern = expand_kernel<BF16, NBW, PRE, false, kWalk>;
+      wt = expand_occupancy(reinterpret_cast<const void*>(kern), lds, occ[2]) * device_cus();
+      wt = grid = expand_grid(wt, max_tiles, n_sub, true);
+      p.span_lo = sr.lo;
+      p.span_hi = sr.hi;
+    }
+  }
+  p.wt = static_cast<int>(wt);
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(grid)), dim3(kThreads), lds, st, p);
 }
 
 // NBW = 2 is chosen for at most 2 k-groups of lora_B only (expand_form).
 template <bool BF16>
-void launch_expand_form(int NBW, int PRE, int max_tiles, size_t lds, const ExpandParams& p, hipStream_t st) {
-  if (NBW == 2) launch_expand_t<BF16, 2, 2>(max_tiles, lds, p, st);
-  else if (PRE == 2) launch_expand_t<BF16, 1, 2>(max_tiles, lds, p, st);
-  else if (PRE == 4) launch_expand_t<BF16, 1, 4>(max_tiles, lds, p, st);
-  else launch_expand_t<BF16, 1, 8>(max_tiles, lds, p, st);
+void launch_expand_form(int NBW, int PRE, int64_t T, int adapters, size_t lds, const ExpandParams& p, hipStream_t st) {
+  if (NBW == 2) launch_expand_t<BF16, 2, 2>(T, adapters, lds, p, st);
+  else if (PRE == 2) launch_expand_t<BF16, 1, 2>(T, adapters, lds, p, st);
+  else if (PRE == 4) launch_expand_t<BF16, 1, 4>(T, adapters, lds, p, st);
+  else launch_expand_t<BF16, 1, 8>(T, adapters, lds, p, st);
 }
 
 // The rank-split expand takes a sparse bf16 class whose sub-tiles of 128
@@ -1724,10 +1788,9 @@ void launch_expand(bool bf16, int64_t T, int adapters, ExpandParams p, hipStream
     launch_expand_sparse(T, adapters, p, st);
     return;
   }
-  const int max_tiles = max_tiles_for(T, adapters);
   const size_t lds = expand_lds_bytes(bf16, p.si.S, p.max_rank);
-  if (bf16) launch_expand_form<true>(f.NBW, f.PRE, max_tiles, lds, p, st);
-  else launch_expand_form<false>(f.NBW, f.PRE, max_tiles, lds, p, st);
+  if (bf16) launch_expand_form<true>(f.NBW, f.PRE, T, adapters, lds, p, st);
+  else launch_expand_form<false>(f.NBW, f.PRE, T, adapters, lds, p, st);
 }
 
 
@@ -1811,7 +1874,17 @@ int pair_expand_occupancy(const void* kern, size_t lds) {
 int64_t pair_expand_grid(const PairForm& f, int64_t T, int adapters0, size_t lds, const ExpandParams& e0) {
   const int64_t wt = static_cast<int64_t>(pair_expand_occupancy(expand_pair_fn_of(f), lds)) * device_cus();
   const int NT = 4 * f.f0.NBW * 32;
-  return expand_grid(wt, max_tiles_for(T, adapters0), (e0.out_total + NT - 1) / NT, expand_cut(f.f0.NBW, true));
+  return expand_grid(wt, max_tiles_for(T, adapters0), (e0.out_total + NT - 1) / NT, true);
+}
+
+// The pair expand always may walk.  The 256-column form, whose start costs
+// about three of its sub-tiles, takes spans below 64 tiles.
+void set_pair_spans(ExpandParams& e0, const PairForm& f, int64_t T, int adapters0, int64_t grid) {
+  const int NT = 4 * f.f0.NBW * 32;
+  const SpanRange sr = expand_span_range(grid, T, adapters0, max_tiles_for(T, adapters0), (e0.out_total + NT - 1) / NT);
+  e0.wt = static_cast<int>(grid);
+  e0.span_lo = f.f0.NBW == 2 ? 1 : sr.lo;
+  e0.span_hi = f.f0.NBW == 2 ? 63 : sr.hi;
 }
 
 // Workgroups that sum the large class's partials (sum_partials): for the tiles
@@ -2248,20 +2321,37 @@ struct AddrModel {
       while (s_hi + 1 < si.S && c_last >= si.bounds[s_hi + 1]) ++s_hi;
       stage(tr, s_lo, s_hi, s_lo * r, zs_ld, lds, nparts);
     };
-    const addr::ExpandCut cut = flat ? addr::kCutSpans : expand_cut(f.NBW, pair);
-    const int64_t grid = expand_grid(wt, max_tiles, n_sub, cut);
     if (flat) {
-      for_items("expand_kernel", grid, true, work_items(total, n_sub, true), [&](int lin) {
+      for_items("expand_kernel", expand_flat_grid(wt, max_tiles, n_sub), true, work_items(total, n_sub, true), [&](int lin) {
         const XcdItem it = work_item(lin, total, n_sub, true);
         item(tl[it.tile], it.sub, 1);
       });
       return;
     }
-    // the workgroups' spans: each (tile, sub-tile) exactly once, in order per XCD
+    SpanRange sr = expand_span_range(expand_grid(wt, max_tiles, n_sub, false), T, adapters, max_tiles, n_sub);
+    const bool walks = pair || expand_walks(bf16, f.NBW, f.PRE, wt, max_tiles, sr);
+    const int grid = static_cast<int>(expand_grid(wt, max_tiles, n_sub, walks));
+    if (pair) {
+      ExpandParams e0 = e;
+      PairForm pf;
+      pf.f0 = f;
+      set_pair_spans(e0, pf, T, adapters, grid);
+      sr = {e0.span_lo, e0.span_hi};
+    }
+    const bool spans = walks && addr::expand_takes_spans(grid, total, sr.lo, sr.hi);
+    const int groups = addr::expand_groups(total, n_sub, walks ? grid : static_cast<int>(wt));
+    // the workgroups' parts or spans: each (tile, sub-tile) exactly once, in order per XCD
     std::vector<char> seen(static_cast<size_t>(total) * n_sub, 0);
-    for (int64_t b = 0; b < grid; ++b) {
+    for (int b = 0; b < grid; ++b) {
       int tile = 0, sub = 0, left = 0;
-      addr::expand_span(static_cast<int>(b), static_cast<int>(grid), total, n_sub, cut, tile, sub, left);
+      if (spans) {
+        addr::expand_span(b, grid, total, n_sub, tile, sub, left);
+      } else {
+        const XcdItem it = xcd_item(b, total, groups);
+        if (it.tile < 0) continue;
+        tile = it.tile;
+        addr::expand_part(it.sub, groups, n_sub, sub, left);
+      }
       while (left > 0) {
         const int n = std::min(left, n_sub - sub);
         const int64_t lo = static_cast<int64_t>(tile) * n_sub + sub;
@@ -2480,13 +2570,14 @@ int switched_lora_impl(const char* who, int32_t dtype, const void* x, int64_t ld
     const ShrinkPlan pl1 = plan_class(num_tokens, hidden, num_slices, cls[1], bf16, max_part_bytes);
     const ShrinkParams sp0 = shrink_params(cls[0], pl0, L.off[0], ldz);
     const ShrinkParams sp1 = shrink_params(cls[1], pl1, L.off[1], ldz);
-    const ExpandParams e0 = expand_params(cls[0], pl0, sp0, ldz);
+    ExpandParams e0 = expand_params(cls[0], pl0, sp0, ldz);
     ExpandParams e1 = expand_params(cls[1], pl1, sp1, ldz);
     const PairForm f = pair_form(bf16, num_tokens, pl0, pl1, e0, e1);
     if (f.ok) {
       int* claim = reinterpret_cast<int*>(static_cast<char*>(workspace) + L.claim);
       const size_t lds = pair_lds_bytes(num_slices, cls[0].max_rank, cls[1].max_rank);
       const int64_t egrid = pair_expand_grid(f, num_tokens, cls[0].adapters, lds, e0);
+      set_pair_spans(e0, f, num_tokens, cls[0].adapters, egrid);
       e1.sum_wgs = pair_sum_wgs(e1, cls[1], egrid);
       launch_shrink_pair(f, pl0.grid, sp0, sp1, claim, st);
       GS_CHECK_LAUNCH(who);
@@ -2713,6 +2804,19 @@ int gs_switched_lora_noalloc(int32_t dtype, const void* x, int64_t ldx, void* y,
   return switched_lora_impl(who, dtype, x, ldx, y, ldy, num_tokens, hidden, out_total, slice_bounds, num_slices,
                             a_pack, a_off, b_pack, b_off, ranks, num_adapters, max_rank, ranks_host, seg_offsets, perm,
                             base + part, base, part, stream, part_budget);
+}
+
+int gs_expand_span_tiles(int64_t num_tokens, int32_t num_adapters, int32_t out_total, int32_t workgroups,
+                         int32_t* range) {
+  const char* who = "gs_expand_span_tiles";
+  GS_CHECK_ARG(num_tokens > 0 && num_adapters > 0 && out_total > 0 && workgroups > 0 && range != nullptr, "%s: sizes", who);
+  const int max_tiles = max_tiles_for(num_tokens, num_adapters);
+  const int64_t n_sub = (out_total + 127) / 128;
+  const SpanRange s = expand_span_range(expand_grid(workgroups, max_tiles, n_sub, false), num_tokens, num_adapters,
+                                        max_tiles, n_sub);
+  range[0] = s.lo;
+  range[1] = s.hi;
+  return GS_OK;
 }
 
 int64_t gs_check_segment_addresses(int32_t dtype, int64_t num_tokens, int32_t hidden, int64_t ldx, int32_t out_total,

@@ -270,6 +270,13 @@ int gs_switched_lora(int32_t dtype, const void* x, int64_t ldx, void* y, int64_t
                      const int32_t* seg_offsets, const int32_t* perm, void* z, void* workspace,
                      int64_t workspace_bytes, void* stream);
 
+/* Test support (makes no HIP call).  The tile counts range[0] .. range[1]
+ * (none: range[1] = 0) for which an expand of 128-column sub-tiles on
+ * `workgroups` workgroups cuts a batch into spans that cross tiles; other
+ * batches have one part of a tile to a workgroup. */
+int gs_expand_span_tiles(int64_t num_tokens, int32_t num_adapters, int32_t out_total, int32_t workgroups,
+                         int32_t* range);
+
 /* Test support (no counterpart in the reference; makes no HIP call).  Replays
  * on the host every global and LDS access the segment kernels would make for
  * this call -- the launches of gs_switched_lora with a caller workspace and

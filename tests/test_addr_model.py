@@ -129,6 +129,9 @@ EDGE = [
     (4096, 12800, (4096,), [(8, 16, 32, 64)[a % 4] for a in range(48)], 9, 0.15),
     (200, 1024, (1024,), [128, 512], 10, 0.3),                    # large class only
     (400, 4096, (4096, 1024, 1024), [32] * 6 + [512], 11, 0.1),
+    (8192, 64, (4096,), [64] * 24, 12, 0.1),                      # expand spans that cross tiles ...
+    (7500, 64, (2048, 2048), [64] * 100, 13, 0.0),                # ... of more than 64 adapters and two slices
+    (40000, 64, (128,), [64, 40, 64], 14, 0.0),                   # ... more tiles than workgroups
 ]
 
 
@@ -139,7 +142,7 @@ def test_edge_shapes(T, H, slices, ranks, seed, base):
     eff = rng.integers(1, NA + 1, size=T)
     eff[rng.random(T) < base] = 0
     for dt in (_lib.GS_DTYPE_BF16, _lib.GS_DTYPE_FP32):
-        if dt == _lib.GS_DTYPE_FP32 and len(slices) * max(ranks) > 512:
+        if dt == _lib.GS_DTYPE_FP32 and (len(slices) * max(ranks) > 512 or T > 5000):
             continue                                          # refused by the fp32 expand's LDS limit
         _check(T, H, slices, ranks, eff, dt)
     # a row stride wider than the row, and an all-base batch

@@ -289,10 +289,24 @@ def test_one_adapter_past_2e18_slots(dev):
 
 
 @pytest.mark.parametrize("T,NA,rank,slices", [
-    (40000, 3, 8, (128,)),              # more tiles than workgroups, one sub-tile each: a span is several tiles
-    (12000, 40, 32, (256, 128, 128)),   # spans that cross tiles, adapters and slices
+    (40000, 3, 64, (128,)),             # more tiles than workgroups, one sub-tile each: a span is several tiles
+    (8192, 24, 64, (4096,)),            # spans that cross tiles and adapters
+    (7500, 100, 64, (2048, 2048)),      # ... and slices, of more than 64 adapters (the two-pass tile lookup)
+    (8192, 48, 40, (2560, 512, 1024)),  # ... with a part-filled last k-group
+])
+def test_expand_spans_across_tiles(dev, T, NA, rank, slices):
+    import ctypes
+    tiles = (ctypes.c_int32 * 2)()
+    assert switched._lib.load().gs_expand_span_tiles(T, NA, sum(slices), 1024, tiles) == 0
+    assert tiles[1] > 0 or T // 32 > 1024
+    test_expand_spans(dev, T, NA, rank, slices)
+
+
+@pytest.mark.parametrize("T,NA,rank,slices", [
+    (40000, 3, 8, (128,)),              # more tiles than workgroups, one sub-tile each
+    (12000, 40, 32, (256, 128, 128)),   # parts of tiles over slices (the 256-column form)
     (9000, 100, 64, (384,)),            # more than 64 adapters (the two-pass tile lookup), the 128-column form
-    (33, 2, 16, (4096,)),               # fewer sub-tiles than workgroups: some have no span
+    (33, 2, 16, (4096,)),               # fewer sub-tiles than workgroups: some have no part
 ])
 def test_expand_spans(dev, T, NA, rank, slices):
     H, rng = 64, np.random.default_rng(T)

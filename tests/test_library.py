@@ -338,6 +338,19 @@ def test_gemm_form_follows_the_compute_units():
     assert _gemm_form(300, 7296, 1000, 256) == (0, 256, 256) and _gemm_form(300, 7296, 4096, 256, 1 << 23) == (0, 256, 256)
 
 
+@pytest.mark.parametrize("T,adapters,out,tiles,spans", [
+    (1, 24, 4096, 1, False), (16, 48, 4096, 15, False), (256, 24, 16384, 24, False), (600, 5, 2560, 19, False),
+    (1127, 5, 16384, 30, False), (1500, 24, 16384, 56, False), (2767, 24, 4096, 98, False), (2767, 13, 4096, 89, False),
+    (3087, 5, 2560, 81, False), (4144, 5, 4096, 103, False), (4144, 24, 2560, 138, False),
+    (8192, 24, 16384, 264, True), (8192, 24, 6144, 264, True), (8192, 48, 4096, 278, True), (4144, 48, 16384, 150, True)])
+def test_expand_spans_only_where_they_pay(T, adapters, out, tiles, spans):
+    """Spans that cross tiles pay their start twice; measured slower than one part of a tile to a workgroup at the
+    first eleven (1024 workgroups, ranks up to 64), faster at the others."""
+    r = (ctypes.c_int32 * 2)()
+    assert switched._lib.load().gs_expand_span_tiles(T, adapters, out, 1024, r) == 0
+    assert (r[0] <= tiles <= r[1]) == spans, tuple(r)
+
+
 def test_host_tables_follow_the_pack():
     """The tables kept with a pack are made again after any field they follow
     from changes, in place or by assignment; the class views after a device
