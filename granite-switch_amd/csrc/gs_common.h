@@ -395,6 +395,57 @@ __device__ __forceinline__ TileRef find_tile(const int32_t* __restrict__ seg, co
   return ref;
 }
 
+// The adapter table in one wave (<= 64 adapters): lane l holds adapter l + 1.
+struct AdapterLane {
+  int lo, hi, rk;
+  int64_t of;
+};
+__device__ __forceinline__ AdapterLane load_adapters(const int32_t* __restrict__ seg, const int32_t* __restrict__ ranks,
+                                                     const int64_t* __restrict__ offs, int num_adapters) {
+  AdapterLane a{0, 0, -1, 0};
+  const int g = 1 + __lane_id();
+  if (g <= num_adapters) {
+    a.lo = seg[g - 1];
+    a.hi = seg[g];
+    a.rk = ranks[g];
+    a.of = offs[g];
+  }
+  return a;
+}
+// Tiles of TM slots of the lane's adapter, when its rank is in the window.
+template <int TM>
+__device__ __forceinline__ int lane_tiles(const AdapterLane& a, RankWindow rw) {
+  return in_window(rw, a.rk) ? (a.hi - a.lo + TM - 1) / TM : 0;
+}
+// Inclusive scan over the wave's lanes; its total in every lane.
+__device__ __forceinline__ int scan_lanes(int v, int& total) {
+  const int l = __lane_id();
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    int u = __shfl_up(v, d, 64);
+    if (l >= d) v += u;
+  }
+  total = __shfl(v, 63, 64);
+  return v;
+}
+// Tile `tile` of the lanes' tiles (ntiles each, incl their scan); g = 0: none.
+template <int TM, bool BAL>
+__device__ __forceinline__ TileRef tile_of_lanes(const AdapterLane& a, int ntiles, int incl, int tile) {
+  TileRef ref{0, 0, 0, 0, 0};
+  const int excl = incl - ntiles;
+  const uint64_t bal = __ballot(ntiles > 0 && tile >= excl && tile < incl);
+  if (bal == 0) return ref;
+  const int src = __ffsll(static_cast<long long>(bal)) - 1;
+  const int jj = tile - __shfl(excl, src, 64);
+  const int slo = __shfl(a.lo, src, 64);
+  const int shi = __shfl(a.hi, src, 64);
+  ref.g = 1 + src;
+  tile_span<TM, BAL>(slo, shi, jj, ref.slot0, ref.nrows);
+  ref.rank = __shfl(a.rk, src, 64);
+  ref.off = __shfl(a.of, src, 64);
+  return ref;
+}
+
 // The tile of a workgroup's (first) item, in one pass over the adapter table
 // when it fits one wave (<= 64 adapters): the tile count and the tile's lookup
 // share the same loads.  item_of(total tiles) names the item (every wave
@@ -412,40 +463,12 @@ __device__ __forceinline__ TileRef locate_item(const int32_t* __restrict__ seg, 
     sub = it.sub;
     return it.tile < 0 ? ref : find_tile<TM, BAL>(seg, ranks, offs, num_adapters, rw, it.tile);
   }
-  const int l = __lane_id();
-  const int g = 1 + l;
-  int ntiles = 0, lo = 0, hi = 0, rk = 0;
-  int64_t of = 0;
-  if (g <= num_adapters) {
-    lo = seg[g - 1];
-    hi = seg[g];
-    rk = ranks[g];
-    of = offs[g];
-    ntiles = in_window(rw, rk) ? (hi - lo + TM - 1) / TM : 0;
-  }
-  int incl = ntiles;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    int v = __shfl_up(incl, d, 64);
-    if (l >= d) incl += v;
-  }
-  const int total = __shfl(incl, 63, 64);
-  total_out = total;
-  const XcdItem it = item_of(total);
+  const AdapterLane a = load_adapters(seg, ranks, offs, num_adapters);
+  const int ntiles = lane_tiles<TM>(a, rw);
+  const int incl = scan_lanes(ntiles, total_out);
+  const XcdItem it = item_of(total_out);
   sub = it.sub;
-  if (it.tile < 0) return ref;
-  const int excl = incl - ntiles;
-  const uint64_t bal = __ballot(ntiles > 0 && it.tile >= excl && it.tile < incl);
-  if (bal == 0) return ref;
-  const int src = __ffsll(static_cast<long long>(bal)) - 1;
-  const int jj = it.tile - __shfl(excl, src, 64);
-  const int slo = __shfl(lo, src, 64);
-  const int shi = __shfl(hi, src, 64);
-  ref.g = 1 + src;
-  tile_span<TM, BAL>(slo, shi, jj, ref.slot0, ref.nrows);
-  ref.rank = __shfl(rk, src, 64);
-  ref.off = __shfl(of, src, 64);
-  return ref;
+  return it.tile < 0 ? ref : tile_of_lanes<TM, BAL>(a, ntiles, incl, it.tile);
 }
 
 // The tile of work item `lin` of a 1-D launch over (tile, sub) pairs (see

@@ -827,29 +827,31 @@ __device__ __forceinline__ void expand_item(const ExpandParams& p, const TileRef
 // whose second item costs registers; the pair expand always has it.
 enum ExpandWalk { kOneItem, kWalk };
 
-// A workgroup's part or span of a launch that may walk.  before_last() runs
-// before its last sub-tile's products.
+// A workgroup's part or span of a launch that may walk: where it starts in a
+// batch of `total` tiles (a span: groups 0, `left` sub-tiles), then its items.
+// before_last() runs before the last sub-tile's products.
+struct WalkStart {
+  int tile = 0, left = 0, groups = 0;
+  __device__ __forceinline__ XcdItem first(const ExpandParams& p, int total, int n_sub) {
+    const int b = static_cast<int>(blockIdx.x);
+    if (addr::expand_takes_spans(p.wt, total, p.span_lo, p.span_hi)) {
+      int sub;
+      addr::expand_span(b, p.wt, total, n_sub, tile, sub, left);
+      return XcdItem{left > 0 ? tile : -1, sub};
+    }
+    groups = addr::expand_groups(total, n_sub, p.wt);
+    return xcd_item(b, total, groups);
+  }
+};
 template <bool BF16, int NBW, int PRE, typename Hook = NoHook>
-__device__ __forceinline__ void expand_walk(const ExpandParams& p, float (&dtile)[kTM][4 * NBW * 32 + kOutPad],
-                                            char* zs, Hook before_last = Hook{}) {
+__device__ __forceinline__ void expand_walk(const ExpandParams& p, const WalkStart& start, TileRef tr, int sub,
+                                            float (&dtile)[kTM][4 * NBW * 32 + kOutPad], char* zs,
+                                            Hook before_last = Hook{}) {
   constexpr int NT = 4 * NBW * 32;
   const int n_sub = (p.out_total + NT - 1) / NT;
-  int tile = 0, left = 0, sub = 0, total = 0, groups = 0;
-  TileRef tr = locate_item<kTM, kExpandBalanced>(
-      p.seg, p.ranks, p.b_off, p.NA, p.rw,
-      [&](int tot) {
-        const int b = static_cast<int>(blockIdx.x);
-        if (addr::expand_takes_spans(p.wt, tot, p.span_lo, p.span_hi)) {
-          int first;
-          addr::expand_span(b, p.wt, tot, n_sub, tile, first, left);
-          return XcdItem{left > 0 ? tile : -1, first};
-        }
-        groups = addr::expand_groups(tot, n_sub, p.wt);
-        return xcd_item(b, tot, groups);
-      },
-      sub, total);
   if (tr.g == 0) return;
-  if (groups > 0) addr::expand_part(sub, groups, n_sub, sub, left);
+  int tile = start.tile, left = start.left;
+  if (start.groups > 0) addr::expand_part(sub, start.groups, n_sub, sub, left);
   // (the same in every lane: in scalar registers across the items)
   left = __builtin_amdgcn_readfirstlane(left);
   tile = __builtin_amdgcn_readfirstlane(tile);
@@ -885,7 +887,12 @@ void expand_kernel(ExpandParams p) {
   extern __shared__ __align__(16) char zs[];   // [32][S*max_rank + 8] element type
   if constexpr (!LOOP) {
     if constexpr (WALK == kWalk) {
-      expand_walk<BF16, NBW, PRE>(p, dtile, zs);
+      const int n_sub = (p.out_total + NT - 1) / NT;
+      WalkStart start;
+      int sub = 0, total = 0;
+      const TileRef tr = locate_item<kTM, kExpandBalanced>(p.seg, p.ranks, p.b_off, p.NA, p.rw,
+                                                           [&](int tot) { return start.first(p, tot, n_sub); }, sub, total);
+      expand_walk<BF16, NBW, PRE>(p, start, tr, sub, dtile, zs);
     } else {
       const int n_sub = (p.out_total + NT - 1) / NT;
       int sub = 0, groups = 1, total = 0;
@@ -938,12 +945,14 @@ void expand_kernel(ExpandParams p) {
 // shrink values are staged.
 // ----------------------------------------------------------------------------
 constexpr int kSpNT = 128;                   // columns per item of expand_sparse_kernel
+constexpr int kSumRows = 4;                  // rows of a tile whose partials every item sums for itself
 
 // One item of the rank-split expand: tile tr, sub-tile `sub` of 32 * QB
 // columns (inside one slice).  red: the waves' partial deltas.  Each output
 // element is the same sum in the same order whatever QB: wave w's k-groups
 // [w*KG, (w+1)*KG) in order, then (w0 + w2) + (w1 + w3).
-// SUMMED: split-K partials may be summed in z already (sum_partials).
+// SUMMED: the split-K partials of tiles of more than kSumRows rows may be summed
+// in z already (sum_partials).
 template <int KG, int QB, bool SUMMED = false>
 __device__ __forceinline__ void expand_sparse_item(const ExpandParams& p, const TileRef& tr, int sub, int nparts,
                                                    float (&red)[2][kTM][32 * QB + kOutPad], char* zs) {
@@ -995,7 +1004,7 @@ __device__ __forceinline__ void expand_sparse_item(const ExpandParams& p, const 
     // (pieces past the rank read the row's first piece and are masked) and
     // the y pieces
     uint2 w[ZIT];
-    if (!SUMMED && nparts == 0) {   // uniform
+    if (nparts == 0) {   // uniform
       const uint16_t* zp = static_cast<const uint16_t*>(p.z) + zo + s * r;
 #pragma unroll
       for (int j = 0; j < ZIT; ++j) {
@@ -1020,10 +1029,10 @@ __device__ __forceinline__ void expand_sparse_item(const ExpandParams& p, const 
     for (int ps = 0; ps < PASSES; ++ps) yv[ps] = ld16(static_cast<const char*>(p.y) + (yrow[ps] + n_tile0 + cx) * 2);
     uint32_t unsummed = ~0u;               // pieces j of this thread whose partials it sums itself
     if constexpr (SUMMED) {
-      // the summed pieces (or z, when the shrink was not split), the youngest
-      // loads: the sums have had the longest time.  Agent scope: another XCD
-      // may have stored them in this launch.  zo is 0: the pair's z is by slot
-      if (nparts == 0 || p.sum_wgs > 0) {   // uniform
+      // the summed pieces, the youngest loads: the sums have had the longest
+      // time.  Agent scope: another XCD may have stored them in this launch.
+      // zo is 0: the pair's z is by slot
+      if (nparts >= 2 && p.sum_wgs > 0 && tr.nrows > kSumRows) {   // uniform
         const uint16_t* zp = static_cast<const uint16_t*>(p.z) + s * r;
         uint64_t zv[ZIT];
 #pragma unroll
@@ -1048,7 +1057,7 @@ __device__ __forceinline__ void expand_sparse_item(const ExpandParams& p, const 
     // the slice's shrink values of the tile's rows in LDS: the z pieces
     // loaded above, or split-K partials summed in ks order (kPartGroup at a
     // time) and rounded to bf16 as a stored z would be
-    if (!SUMMED && nparts == 0) {
+    if (nparts == 0) {
 #pragma unroll
       for (int j = 0; j < ZIT; ++j) {
         const int it = tid + j * kThreads;
@@ -1165,20 +1174,18 @@ __device__ __forceinline__ int sparse_nparts(const ExpandParams& p) {
 // waits: a reader takes the pieces that are there and sums the ones still
 // marked kUnsummed as before, in the same order, so the bits are the same
 // either way.  Pieces are 8 bytes, stored and loaded whole at agent scope.
-// Pair expand of 256 tokens, 12 rank-32 adapters and one of rank 512: 4096 ->
-// 4096 20.5 -> 13.2 us, 4096 -> 6144 18.6 -> 13.7, 4096 -> 25600 30.0 -> 24.6.
+// A tile of at most kSumRows rows, or a class whose shrink was not split, is
+// read as without the sums: they would only put a workgroup's own items later
+// and z beyond the L2 (a step whose rank-512 adapter has 2 rows 8.10 ms of 8.02).
+// Both launches, 12 rank-32 adapters and one of rank 512, items summing for
+// themselves / with the sums: 256 x 4096 -> 4096 31.7 / 20.9 us, -> 6144 32.0 /
+// 26.2, -> 25600 40.0 / 34.7; 4144 x 4096 -> 25600 220 / 171.
 // A deeper k-split, which the cheaper sums would allow, lost in the shrink
-// what it gained (4096 -> 6144: 13.6 -> 17.6 us).
-__device__ __forceinline__ void sum_partials(const ExpandParams& p) {
-  const int u = static_cast<int>(blockIdx.x);
-  if (u >= p.sum_wgs) return;
-  const int nparts = sparse_nparts(p);
-  if (nparts == 0) return;
-  const int wpt = addr::sum_wgs_per_tile(kTM, p.si.S * p.max_rank, kThreads);
-  const TileRef tr = find_tile<kTM, kExpandBalanced>(p.seg, p.ranks, p.b_off, p.NA, p.rw, u / wpt);
-  if (tr.g == 0) return;
+// what it gained (256 x 4096 -> 6144: 13.6 -> 17.6 us).
+// part: the workgroup's among the wpt of its tile tr.
+__device__ __forceinline__ void sum_partials(const ExpandParams& p, const TileRef& tr, int nparts, int part) {
   const int per_row = (p.si.S * tr.rank) >> 2;
-  const int it = (u % wpt) * kThreads + static_cast<int>(threadIdx.x);
+  const int it = part * kThreads + static_cast<int>(threadIdx.x);
   const int row = addr::stage_row(it, per_row);
   if (row >= tr.nrows) return;
   const int c4 = addr::stage_col(it, row, per_row, 0);
@@ -1288,7 +1295,8 @@ __global__ __launch_bounds__(kThreads) void shrink_dma_pair_kernel(ShrinkParams 
 }
 
 template <int NBW, int PRE, int KG>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void expand_pair_kernel(ExpandParams p0, ExpandParams p1, int* claim) {
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(KG == 8 ? 2 : 3)))
+void expand_pair_kernel(ExpandParams p0, ExpandParams p1, int* claim) {
   constexpr int NT = 4 * NBW * 32;
   constexpr int kD = static_cast<int>(sizeof(float)) * kTM * (NT + kOutPad);
   constexpr int kR = static_cast<int>(sizeof(float)) * 2 * kTM * (32 * kPairQB + kOutPad);
@@ -1297,20 +1305,52 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   extern __shared__ __align__(16) char zs[];   // either class's shrink values
   auto& dtile = *reinterpret_cast<float(*)[kTM][NT + kOutPad]>(buf);
   auto& red = *reinterpret_cast<float(*)[2][kTM][32 * kPairQB + kOutPad]>(buf);
-  sum_partials(p1);
+  // both classes' tile counts, the workgroup's first small-class tile and the
+  // large-class tile that it sums for, in one pass over the adapter table
+  const int n_sub = (p0.out_total + NT - 1) / NT;
+  const int u = static_cast<int>(blockIdx.x);
+  const int wpt = addr::sum_wgs_per_tile(kTM, p1.si.S * p1.max_rank, kThreads);
+  int total1, nparts1 = p1.nparts, sub0;
+  WalkStart start;
+  TileRef tr0{0, 0, 0, 0, 0}, trs{0, 0, 0, 0, 0};
+  if (p0.NA <= 64) {
+    const AdapterLane a = load_adapters(p0.seg, p0.ranks, p0.b_off, p0.NA);
+    const int n0 = lane_tiles<kTM>(a, p0.rw), n1 = lane_tiles<kTM>(a, p1.rw);
+    int total0;
+    const int incl0 = scan_lanes(n0, total0), incl1 = scan_lanes(n1, total1);
+    if (p1.ks_target > 0) {
+      int tiles64;
+      scan_lanes(lane_tiles<kTMS>(a, p1.rw), tiles64);
+      nparts1 = dyn_ksplit(tiles64, p1.ks_chunks, p1.ks_target, p1.nparts);
+      if (nparts1 <= 1) nparts1 = 0;
+    }
+    if (u < p1.sum_wgs) trs = tile_of_lanes<kTM, kExpandBalanced>(a, n1, incl1, u / wpt);
+    const XcdItem it0 = start.first(p0, total0, n_sub);
+    sub0 = it0.sub;
+    if (it0.tile >= 0) tr0 = tile_of_lanes<kTM, kExpandBalanced>(a, n0, incl0, it0.tile);
+  } else {
+    total1 = count_tiles<kTM>(p1.seg, p1.ranks, p1.NA, p1.rw);
+    nparts1 = sparse_nparts(p1);
+    if (u < p1.sum_wgs) trs = find_tile<kTM, kExpandBalanced>(p1.seg, p1.ranks, p1.b_off, p1.NA, p1.rw, u / wpt);
+    int total0;
+    tr0 = locate_item<kTM, kExpandBalanced>(p0.seg, p0.ranks, p0.b_off, p0.NA, p0.rw,
+                                            [&](int tot) { return start.first(p0, tot, n_sub); }, sub0, total0);
+  }
+  // the same in every lane: in scalar registers past the small items
+  total1 = __builtin_amdgcn_readfirstlane(total1);
+  nparts1 = __builtin_amdgcn_readfirstlane(nparts1);
+  if (nparts1 >= 2 && trs.nrows > kSumRows) sum_partials(p1, trs, nparts1, u % wpt);
   int ticket = 0;
   bool early = false;                      // uniform: the small items ran and claimed
   // the first claim goes out before the small class's last sub-tile, so its
   // round trip passes while that sub-tile is computed; its result is written
   // to LDS only afterwards (no wait for it before)
-  expand_walk<true, NBW, PRE>(p0, dtile, zs, [&]() {
+  expand_walk<true, NBW, PRE>(p0, start, tr0, sub0, dtile, zs, [&]() {
     if (threadIdx.x == 0) ticket = claim_next(claim);
     early = true;
   });
   const int n_sub1 = p1.out_total / (32 * kPairQB);
-  const int total1 = count_tiles<kTM>(p1.seg, p1.ranks, p1.NA, p1.rw);
   const int items1 = work_items(total1, n_sub1, true);
-  const int nparts1 = sparse_nparts(p1);
   if (threadIdx.x == 0)
     claimed = early ? ticket : claim_next(claim);
   lds_barrier();                           // every wave is past the small item; `claimed` is written
@@ -1870,21 +1910,29 @@ int pair_expand_occupancy(const void* kern, size_t lds) {
   return n;
 }
 
-// The pair expand's grid: the small class's, at the pair kernel's occupancy.
+// The pair expand's grid: the small class's, on 2 workgroups per CU, 3 with the
+// narrowest large class.  Where the kernel's registers would allow one more, its
+// workgroups' starts cost more than they hide (48 adapters of rank 8 to 64 and
+// one of 256: 600 x 4096 27.1 us on 2, 31.0 on 3; 256 x 4096 26.5, 29.5).
 int64_t pair_expand_grid(const PairForm& f, int64_t T, int adapters0, size_t lds, const ExpandParams& e0) {
-  const int64_t wt = static_cast<int64_t>(pair_expand_occupancy(expand_pair_fn_of(f), lds)) * device_cus();
+  const int occ = std::min(pair_expand_occupancy(expand_pair_fn_of(f), lds), f.KG1 == 2 ? 3 : 2);
+  const int64_t wt = static_cast<int64_t>(occ) * device_cus();
   const int NT = 4 * f.f0.NBW * 32;
   return expand_grid(wt, max_tiles_for(T, adapters0), (e0.out_total + NT - 1) / NT, true);
 }
 
 // The pair expand always may walk.  The 256-column form, whose start costs
-// about three of its sub-tiles, takes spans below 64 tiles.
+// about three of its sub-tiles, takes spans for few tiles, whose sub-tiles leave
+// a quarter of the workgroups to the large class: parts leave XCDs without work
+// then (256 x 6144 of 12 + 1 adapters 27.0 -> 26.2 us; of 24 + 1, 64 x 6144, spans
+// of one or two sub-tiles 31.2 us, parts 29.6).
 void set_pair_spans(ExpandParams& e0, const PairForm& f, int64_t T, int adapters0, int64_t grid) {
   const int NT = 4 * f.f0.NBW * 32;
-  const SpanRange sr = expand_span_range(grid, T, adapters0, max_tiles_for(T, adapters0), (e0.out_total + NT - 1) / NT);
+  const int64_t n_sub = (e0.out_total + NT - 1) / NT;
+  const SpanRange sr = expand_span_range(grid, T, adapters0, max_tiles_for(T, adapters0), n_sub);
   e0.wt = static_cast<int>(grid);
   e0.span_lo = f.f0.NBW == 2 ? 1 : sr.lo;
-  e0.span_hi = f.f0.NBW == 2 ? 63 : sr.hi;
+  e0.span_hi = f.f0.NBW == 2 ? static_cast<int>(std::min<int64_t>(63, 3 * grid / (4 * n_sub))) : sr.hi;
 }
 
 // Workgroups that sum the large class's partials (sum_partials): for the tiles

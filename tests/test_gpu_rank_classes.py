@@ -399,14 +399,18 @@ def test_step_population_with_a_rank512_adapter(dev, proj):
     _say(f"  max abs err {err:.3e}")
 
 
-@pytest.mark.parametrize("slices,on_large", [((2048, 1024, 1024), 300), ((4096,), 33), ((256, 256), 1)])
-def test_pair_sums_beyond_the_expected_tiles_and_nan(dev, slices, on_large):
+@pytest.mark.parametrize("slices,on_large,small", [
+    ((2048, 1024, 1024), 300, 24), ((4096,), 33, 24), ((256, 256), 1, 24),
+    ((1024, 512), 4, 24), ((1024, 512), 5, 24),                  # the rows from which a tile's partials are summed
+    ((2048, 1024), 40, 70), ((2048, 1024), 3, 70),               # more than 64 adapters: the lookups in turn
+])
+def test_pair_sums_beyond_the_expected_tiles_and_nan(dev, slices, on_large, small):
     """The pair expand sums the large class's partials once for the tiles it is
     expected to hold; the items of further tiles (300 tokens where ~24 are
     expected), and pieces whose sum has the bits of the not-yet-summed mark
     (NaN), sum for themselves: the same bits as the classes in turn, also on
     replays of a graph over the same scratch."""
-    ranks = [32] * 24 + [512]
+    ranks = [32] * small + [512]
     NA, T = len(ranks), 600
     spec = workloads.ModuleSpec("m", 4096, slices, ranks, 512)
     md = workloads.make_module(spec, T, NA, torch.bfloat16, dev, seed=on_large)
