@@ -951,8 +951,10 @@ constexpr int kSumRows = 4;                  // rows of a tile whose partials ev
 // columns (inside one slice).  red: the waves' partial deltas.  Each output
 // element is the same sum in the same order whatever QB: wave w's k-groups
 // [w*KG, (w+1)*KG) in order, then (w0 + w2) + (w1 + w3).
-// SUMMED: the split-K partials of tiles of more than kSumRows rows may be summed
-// in z already (sum_partials).
+// SUMMED: nparts > 0 split-K partials, which may be summed in z already for tiles
+// of more than kSumRows rows (sum_partials).  (One form for both cost the
+// unsplit class 1 us of 40: 4144 x 4096 -> 6144, 12 adapters of rank 32 and one of
+// 512.)
 template <int KG, int QB, bool SUMMED = false>
 __device__ __forceinline__ void expand_sparse_item(const ExpandParams& p, const TileRef& tr, int sub, int nparts,
                                                    float (&red)[2][kTM][32 * QB + kOutPad], char* zs) {
@@ -1004,7 +1006,7 @@ __device__ __forceinline__ void expand_sparse_item(const ExpandParams& p, const 
     // (pieces past the rank read the row's first piece and are masked) and
     // the y pieces
     uint2 w[ZIT];
-    if (nparts == 0) {   // uniform
+    if (!SUMMED && nparts == 0) {   // uniform
       const uint16_t* zp = static_cast<const uint16_t*>(p.z) + zo + s * r;
 #pragma unroll
       for (int j = 0; j < ZIT; ++j) {
@@ -1032,7 +1034,7 @@ __device__ __forceinline__ void expand_sparse_item(const ExpandParams& p, const 
       // the summed pieces, the youngest loads: the sums have had the longest
       // time.  Agent scope: another XCD may have stored them in this launch.
       // zo is 0: the pair's z is by slot
-      if (nparts >= 2 && p.sum_wgs > 0 && tr.nrows > kSumRows) {   // uniform
+      if (p.sum_wgs > 0 && tr.nrows > kSumRows) {   // uniform
         const uint16_t* zp = static_cast<const uint16_t*>(p.z) + s * r;
         uint64_t zv[ZIT];
 #pragma unroll
@@ -1057,7 +1059,7 @@ __device__ __forceinline__ void expand_sparse_item(const ExpandParams& p, const 
     // the slice's shrink values of the tile's rows in LDS: the z pieces
     // loaded above, or split-K partials summed in ks order (kPartGroup at a
     // time) and rounded to bf16 as a stored z would be
-    if (nparts == 0) {
+    if (!SUMMED && nparts == 0) {
 #pragma unroll
       for (int j = 0; j < ZIT; ++j) {
         const int it = tid + j * kThreads;
@@ -1339,7 +1341,7 @@ void expand_pair_kernel(ExpandParams p0, ExpandParams p1, int* claim) {
   // the same in every lane: in scalar registers past the small items
   total1 = __builtin_amdgcn_readfirstlane(total1);
   nparts1 = __builtin_amdgcn_readfirstlane(nparts1);
-  if (nparts1 >= 2 && trs.nrows > kSumRows) sum_partials(p1, trs, nparts1, u % wpt);
+  if (nparts1 > 0 && trs.nrows > kSumRows) sum_partials(p1, trs, nparts1, u % wpt);
   int ticket = 0;
   bool early = false;                      // uniform: the small items ran and claimed
   // the first claim goes out before the small class's last sub-tile, so its
@@ -1358,7 +1360,10 @@ void expand_pair_kernel(ExpandParams p0, ExpandParams p1, int* claim) {
   while (it < items1) {
     int sub = 0;
     const TileRef tr = tile_at<kTM, kExpandBalanced>(p1.seg, p1.ranks, p1.b_off, p1.NA, p1.rw, it, true, total1, n_sub1, sub);
-    if (tr.g != 0) expand_sparse_item<KG, kPairQB, true>(p1, tr, sub, nparts1, red, zs);
+    if (tr.g != 0) {
+      if (nparts1 == 0) expand_sparse_item<KG, kPairQB>(p1, tr, sub, 0, red, zs);
+      else expand_sparse_item<KG, kPairQB, true>(p1, tr, sub, nparts1, red, zs);
+    }
     lds_barrier();                         // zs, buf and `claimed` are free
     if (threadIdx.x == 0) claimed = claim_next(claim);
     lds_barrier();
