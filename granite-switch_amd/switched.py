@@ -342,6 +342,11 @@ class PackedAdapters:
         )
 
 
+def _int_list(v):
+    """The values of a host table given as any sequence (array, tensor, tuple)."""
+    return v if v is None or isinstance(v, list) else [int(u) for u in v]
+
+
 class _HostTables:
     """What every call on a pack needs of its host-side fields, in the form the C
     calls take: built at the first call and kept with the pack, since building
@@ -354,9 +359,8 @@ class _HostTables:
 
     def __init__(self, p: PackedAdapters):
         self.fields = self._fields(p)
-        self.ranks_list = None if p.ranks_host is None else list(p.ranks_host)
-        self.a_list = None if p.a_off_host is None else list(p.a_off_host)
-        self.b_list = None if p.b_off_host is None else list(p.b_off_host)
+        self.ranks_list, self.a_list, self.b_list = (
+            None if v is None else list(_int_list(v)) for v in (p.ranks_host, p.a_off_host, p.b_off_host))
         self.bounds_list = p.slice_bounds
         self.bounds = _i32_array(self.bounds_list)
         self.ranks = _i32_array(self.ranks_list) if self.ranks_list else None    # None: one class up to max_rank
@@ -376,14 +380,14 @@ class _HostTables:
         return (p.a_pack.dtype, p.hidden, p.num_adapters, p.max_rank, tuple(p.output_slices), p.a_pack.device)
 
     def matches(self, p: PackedAdapters) -> bool:
-        return (self.ranks_list == p.ranks_host and self.a_list == p.a_off_host and self.b_list == p.b_off_host
-                and self.fields == self._fields(p))
+        return (self.ranks_list == _int_list(p.ranks_host) and self.a_list == _int_list(p.a_off_host)
+                and self.b_list == _int_list(p.b_off_host) and self.fields == self._fields(p))
 
     def rank_split(self, p: PackedAdapters) -> tuple:
         """``PackedAdapters.rank_split``; the views share p's device tensors, and
         are made again when those are replaced."""
         cut = _lib.GS_RANK_CLASS_SPLIT
-        if self.one_class is not None:
+        if self.one_class is not None and isinstance(p.ranks_host, list):      # (the views' ranks are a list)
             return (p, None) if self.one_class <= cut else (None, p)
         held = (p.a_pack, p.b_pack, p.a_off, p.b_off, p.ranks)
         if self._split is None or any(u is not v for u, v in zip(self._split[0], held)):

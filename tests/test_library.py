@@ -385,6 +385,21 @@ def test_host_tables_follow_the_pack():
     assert one._host_tables().ranks is None and one.rank_split() == (None, None)
 
 
+@pytest.mark.parametrize("kind", [np.asarray, tuple, torch.as_tensor])
+def test_host_tables_of_any_sequence(kind):
+    """A pack whose host tables are arrays, tuples or tensors: the first call and later ones."""
+    A, B = [torch.ones(3, 1, 128, 16)], [torch.ones(3, 1, 32, 128)]
+    for ranks in ([16, 8, 64], [16, 128, 64]):
+        pk = switched.PackedAdapters.from_slices(A, B, ranks)
+        exp = pk.ranks_host, pk.a_off_host, pk.b_off_host
+        pk.ranks_host, pk.a_off_host, pk.b_off_host = (kind(v) for v in exp)
+        h = pk._host_tables()
+        assert pk._host_tables() is h
+        assert (list(h.ranks), list(h.a_off), list(h.b_off)) == exp
+        small, large = pk.rank_split()
+        assert small.ranks_host == [r if r <= 64 else 0 for r in exp[0]] and (large is None) == (max(ranks) <= 64)
+
+
 def _packed_stub(H, slices, NA, max_rank, dtype=torch.bfloat16):
     """The attributes the small-path plan reads, without device memory."""
     from types import SimpleNamespace
