@@ -823,10 +823,6 @@ __device__ __forceinline__ void expand_item(const ExpandParams& p, const TileRef
   compute(sub0 + nsub - 1, bc, yc);
 }
 
-// The expand kernels of whole parts are compiled without the walk (kOneItem),
-// whose second item costs registers; the pair expand always has it.
-enum ExpandWalk { kOneItem, kWalk };
-
 // A workgroup's part or span of a launch that may walk: where it starts in a
 // batch of `total` tiles (a span: groups 0, `left` sub-tiles), then its items.
 // before_last() runs before the last sub-tile's products.
@@ -872,21 +868,21 @@ __device__ __forceinline__ void expand_walk(const ExpandParams& p, const WalkSta
   }
 }
 
-// LOOP = false: the workgroups' parts or spans (WALK).  LOOP = true (a rank
-// class expected to hold few tiles, laid out flat with one sub-tile per item,
+// LOOP = false: the workgroups' parts; WALK: or spans (kernels of their own, since
+// the walk's second item costs registers).  LOOP = true (a rank class expected to hold few tiles, laid out flat with one sub-tile per item,
 // grid capped at one round): a workgroup takes items blockIdx.x, + gridDim.x, ...
 // while they lie in the batch's item range.
 // The narrow bf16 forms up to rank 64 hold 4 workgroups per CU (<= 128
 // registers per lane; the rank-64 multiswitch projection measured faster at
 // 4 than at 3).
-template <bool BF16, int NBW, int PRE, bool LOOP, ExpandWalk WALK = kOneItem>
+template <bool BF16, int NBW, int PRE, bool LOOP, bool WALK = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BF16 && NBW == 1 && PRE <= 4 && !LOOP ? 4 : 1)))
 void expand_kernel(ExpandParams p) {
   constexpr int NT = 4 * NBW * 32;
   __shared__ float dtile[kTM][NT + kOutPad];
   extern __shared__ __align__(16) char zs[];   // [32][S*max_rank + 8] element type
   if constexpr (!LOOP) {
-    if constexpr (WALK == kWalk) {
+    if constexpr (WALK) {
       const int n_sub = (p.out_total + NT - 1) / NT;
       WalkStart start;
       int sub = 0, total = 0;
@@ -1744,7 +1740,7 @@ void launch_expand_t(int64_t T, int adapters, size_t lds, ExpandParams p, hipStr
   if constexpr (BF16 && NBW == 1 && PRE <= 4) {
     const SpanRange sr = expand_span_range(grid, T, adapters, max_tiles, n_sub);
     if (!p.flat && expand_walks(BF16, NBW, PRE, wt, max_tiles, sr)) {
-      kern = expand_kernel<BF16, NBW, PRE, false, kWalk>;
+      kern = expand_kernel<BF16, NBW, PRE, false, true>;
       wt = expand_occupancy(reinterpret_cast<const void*>(kern), lds, occ[2]) * device_cus();
       wt = grid = expand_grid(wt, max_tiles, n_sub, true);
       p.span_lo = sr.lo;
