@@ -395,7 +395,9 @@ __device__ __forceinline__ TileRef find_tile(const int32_t* __restrict__ seg, co
   return ref;
 }
 
-// The adapter table in one wave (<= 64 adapters): lane l holds adapter l + 1.
+// The adapter table in one wave (<= 64 adapters): lane l holds adapter l + 1.  For
+// several lookups in one pass (the pair expand); locate_item, which has one,
+// counts the tiles where it loads, 0.1 us shorter.
 struct AdapterLane {
   int lo, hi, rk;
   int64_t of;
@@ -463,12 +465,40 @@ __device__ __forceinline__ TileRef locate_item(const int32_t* __restrict__ seg, 
     sub = it.sub;
     return it.tile < 0 ? ref : find_tile<TM, BAL>(seg, ranks, offs, num_adapters, rw, it.tile);
   }
-  const AdapterLane a = load_adapters(seg, ranks, offs, num_adapters);
-  const int ntiles = lane_tiles<TM>(a, rw);
-  const int incl = scan_lanes(ntiles, total_out);
-  const XcdItem it = item_of(total_out);
+  const int l = __lane_id();
+  const int g = 1 + l;
+  int ntiles = 0, lo = 0, hi = 0, rk = 0;
+  int64_t of = 0;
+  if (g <= num_adapters) {
+    lo = seg[g - 1];
+    hi = seg[g];
+    rk = ranks[g];
+    of = offs[g];
+    ntiles = in_window(rw, rk) ? (hi - lo + TM - 1) / TM : 0;
+  }
+  int incl = ntiles;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    int v = __shfl_up(incl, d, 64);
+    if (l >= d) incl += v;
+  }
+  const int total = __shfl(incl, 63, 64);
+  total_out = total;
+  const XcdItem it = item_of(total);
   sub = it.sub;
-  return it.tile < 0 ? ref : tile_of_lanes<TM, BAL>(a, ntiles, incl, it.tile);
+  if (it.tile < 0) return ref;
+  const int excl = incl - ntiles;
+  const uint64_t bal = __ballot(ntiles > 0 && it.tile >= excl && it.tile < incl);
+  if (bal == 0) return ref;
+  const int src = __ffsll(static_cast<long long>(bal)) - 1;
+  const int jj = it.tile - __shfl(excl, src, 64);
+  const int slo = __shfl(lo, src, 64);
+  const int shi = __shfl(hi, src, 64);
+  ref.g = 1 + src;
+  tile_span<TM, BAL>(slo, shi, jj, ref.slot0, ref.nrows);
+  ref.rank = __shfl(rk, src, 64);
+  ref.off = __shfl(of, src, 64);
+  return ref;
 }
 
 // The tile of work item `lin` of a 1-D launch over (tile, sub) pairs (see
