@@ -18,6 +18,11 @@
 // split K over their waves (gemm_bf16_tn_stream_kernel); otherwise they are loaded into
 // registers, zero-filled past K, and written to padded LDS rows
 // (gemm_bf16_tn_kernel).
+//
+// Times in this file: graph replays over buffer sets that together exceed the
+// 256 MB MALL, so the operands come from HBM.  One set, its weights in the MALL
+// (as bench.py --layer-gemm times it), is faster for few rows: 256 x 7296 x 4096
+// 22.5 against 29.3 us, 16 x 7296 x 4096 11.5 against 13.7.
 #include <stdarg.h>
 
 #include <algorithm>
@@ -227,9 +232,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_tn_kernel(GemmParams p
 // banks.  B rows are staged in the order (addr::gemm_b_row) that gives a lane
 // 8 consecutive columns of its C row, stored as 16 bytes.
 //
-// Measured: 4144 x 27136 x 4096 894 -> 676 us (1363 TFLOP/s), 8192 x 26368 x
-// 4096 1443 TFLOP/s, against the form it replaces (one barrier per k-tile, all
-// waves reading, then all multiplying; 1 transfer stage in flight).
+// Measured: 4144 x 27136 x 4096 890 -> 658 us (1400 TFLOP/s), 8192 x 26368 x
+// 4096 1487 -> 1178 (1502), against the form it replaces (one barrier per
+// k-tile, all waves reading, then all multiplying; 1 transfer stage in flight).
+// Without a pause between calls the power limit takes 5 to 8 % of that.
 // ---------------------------------------------------------------------------
 constexpr int kPBK = 64;                        // k per tile
 constexpr int kPRow = kPBK * 2;                 // bytes of one operand row per tile (one cache line)
@@ -543,9 +549,9 @@ __global__ __launch_bounds__(512) void gemm_bf16_tn_pingpong_kernel(GemmParams p
 // HBM once.
 //
 // Bound by LDS (each byte written once and read once) and, for few rows, by
-// HBM: 256 x 7296 x 4096 76 -> 28.9 us and 256 x 4480 x 12800 245 -> 78 against
-// the 256 x 256 tiles; 16 x 7296 x 4096 47 -> 13.2 us (4.6 TB/s of weights),
-// 7 x 4480 x 4096 47 -> 8.9 us (4.1 TB/s).  Deeper rings and longer lookaheads
+// HBM: 256 x 7296 x 4096 76 -> 29.3 us and 256 x 4480 x 12800 245 -> 79 against
+// the 256 x 256 tiles; 16 x 7296 x 4096 47 -> 13.7 us (4.4 TB/s of weights),
+// 7 x 4480 x 4096 47 -> 11.2 us (3.3 TB/s).  Deeper rings and longer lookaheads
 // measured the same.
 // ---------------------------------------------------------------------------
 // s_waitcnt for "lgkmcnt <= n"
@@ -791,8 +797,7 @@ struct GemmPick {
 };
 // Ping-pong, 4144 x 4864 x 12800 (17 x 19 tiles, the last row of 48): 461 us
 // with 16 full tile rows (304 tiles on 256 CUs, 48 in a second round) and one
-// half row, 392 us with 13 and 7; 4096 x 4480 x 12800 457 -> 381 us, 3333 x
-// 6150 x 4096 200 -> 172.
+// half row, 389 us with 13 and 7; 4096 x 4480 x 12800 457 -> 384 us.
 inline GemmPick pick_gemm(int64_t M, int64_t N, int64_t K, int64_t cus) {
   auto tiles = [&](int64_t tm, int64_t tn) { return ((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
   auto rounds = [&](int64_t n) { return (n + cus - 1) / cus; };

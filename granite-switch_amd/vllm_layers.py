@@ -127,8 +127,9 @@ class SwitchedLoRALinear(nn.Module):
 
     _lora_ctx = None
     # x . w_ext^T through this library's MFMA GEMM gs_gemm_bf16_tn (True) or
-    # torch.mm, i.e. hipBLASLt (False, the default).  256 x 7296 x 4096:
-    # 23.5 against 38.4 us; 4144 x 27136 x 4096: 708 / 713; 4144 x 4864 x 12800: 405 / 404
+    # torch.mm, i.e. hipBLASLt (False, the default).  This library / torch, us
+    # (graph replays on one buffer set): 256 x 7296 x 4096 23.6 / 38.0; 4144 x
+    # 27136 x 4096 704 / 705; 4144 x 4864 x 4096 147 / 135, x 12800 404 / 397
     native_gemm = False
 
     def __init__(self, base_layer: nn.Module, num_adapters: int, max_lora_rank: int, num_slices: int = 1,
