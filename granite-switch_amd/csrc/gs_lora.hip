@@ -1174,7 +1174,7 @@ __device__ __forceinline__ int sparse_nparts(const ExpandParams& p) {
 // either way.  Pieces are 8 bytes, stored and loaded whole at agent scope.
 // A tile of at most kSumRows rows, or a class whose shrink was not split, is
 // read as without the sums: they would only put a workgroup's own items later
-// and z beyond the L2 (a step whose rank-512 adapter has 2 rows 8.10 ms of 8.02).
+// and z beyond the L2 (a step whose rank-512 adapter has 2 rows: 8.12 ms against 8.03).
 // Both launches, 12 rank-32 adapters and one of rank 512, items summing for
 // themselves / with the sums: 256 x 4096 -> 4096 31.7 / 20.9 us, -> 6144 32.0 /
 // 26.2, -> 25600 40.0 / 34.7; 4144 x 4096 -> 25600 220 / 171.
